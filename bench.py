@@ -68,20 +68,17 @@ PEAKS = {"mfma_f64": FP64_PEAK_TFLOPS, "mfma_f32": FP32_PEAK_TFLOPS, "valu_f64":
 
 
 def cr_solves_per_mode(n):
-    """r solves of BLKTRI's cyclic reduction of one mode with n = 2^k - 1 z
-    rows, in the partial-fraction form the GPU runs: each reduction level's
-    odd rows apply a product with 2h - 1 divisor roots, each even row two
-    chains of h - 1 solves; each back-substitution row its two chains and a
-    product of 2h - 1 roots (pot/blktri.f:72-170)."""
+    """r solves of the cyclic reduction of one mode with n = 2^k - 1 z rows as
+    the GPU runs it: leaves of 2^l - 1 rows (l = 4, or k - 1 where that is
+    less), each root solved once up and once down the tree, and every row at an
+    odd multiple of h >= 2^l with the 2h - 1 roots of its block, up (below the
+    top level) and down."""
     kx = int(round(np.log2(n + 1)))
-    tot = 0
-    for lv in range(kx - 1):
+    l0 = min(kx - 1, 4)
+    tot = 2 * ((n + 1) >> l0) * ((1 << l0) - 1)
+    for lv in range(l0, kx):
         h = 1 << lv
-        tot += len(range(h, n + 1, 2 * h)) * (2 * h - 1) + len(range(2 * h, n - h + 1, 2 * h)) * 2 * (h - 1)
-    for lv in range(kx - 1, -1, -1):
-        h, nrow = 1 << lv, (1 << (kx - lv)) - 1
-        for jj in range(1, nrow + 1, 2):
-            tot += (h - 1) * ((jj > 1) + (jj < nrow)) + 2 * h - 1
+        tot += (n + 1) // (2 * h) * (2 * h - 1) * (2 if lv < kx - 1 else 1)
     return tot
 
 
@@ -130,7 +127,7 @@ def stage_work(g, path, steps):
 # stage -> name prefixes of the kernels its timed launches run
 STAGE_KERNELS = {"fft_fwd": ("k_fft_forward<",), "fft_inv": ("k_fft_inverse<",),
                  "zfwd": ("k_zgemm_reg<true,",), "zinv": ("k_zgemm_reg<false,",),
-                 "rsolve": ("k_rsolve<",), "cr": ("k_cr_group<",), "resid": ("k_spec_residual",),
+                 "rsolve": ("k_rsolve<",), "cr": ("k_cr_leaf<", "k_cr_node<"), "resid": ("k_spec_residual",),
                  "planes": ("k_refine_plane<",),
                  "bdygen": ("k_bdy_",), "ghost": ("k_zaxphi<",)}
 

@@ -41,44 +41,37 @@ struct Term {
 };
 const Term *terms_table(int *count);  // the kMaxTerms terms, l-major, m ascending
 
-// Cyclic reduction of the per-mode systems (pot/blktri.f:60-260).  A program
-// is one PRDCT product, in one of two forms:
-//   chain (has_pre = 1, ops CR_SCALE): w = sgn x, y = pre w, then for each op
-//     solve (T_m - rt I) w = y along r and y = f w; the result is y;
-//   partial fractions (ops CR_PF): the result is sum over ops of
-//     f (T_m - rt I)^-1 (sgn x), the solves independent of each other.
-enum { CR_SCALE = 2, CR_PF = 3 };
-struct CrOp {
-    double rt, f;
-    int post, pad;
-};
-struct CrProg {
-    int off, nsolve, has_pre, pad;
-    double sgn, pre;
-};
-// One row a phase updates (1-based z row) and its programs (-1: none):
-//   CR_PHASE_ODD  (reduction, rows at odd multiples of h): P(row) = pm(Y(row))
-//   CR_PHASE_EVEN (reduction, rows at even multiples of h):
-//                 Y(row) = (pa(P(row-h)) + pc(P(row+h))) - Y(row)
-//   CR_PHASE_BACK (back substitution, odd multiples of h):
-//                 Y(row) = pm((Y(row) - pa(Y(row-h))) - pc(Y(row+h)))
-enum { CR_PHASE_ODD = 0, CR_PHASE_EVEN = 1, CR_PHASE_BACK = 2 };
-struct CrRow {
-    int row, pa, pc, pm;
-};
+// Cyclic reduction of the per-mode systems (pot/blktri.f:60-260) as a tree
+// over the z rows 1..n, n = 2^k - 1 (cr.hip).  Leaves: `rows` rows between
+// separators at multiples of rows + 1 (16, or half the column where that is
+// less).  Nodes: rows odd * h, h = rows + 1, 2 (rows + 1), .., (n+1)/2, each
+// with the roots of its block of 2h - 1 rows.  Phases in execution order: the leaves' messages, each level's
+// messages from the lowest up, each level's solutions from the top down, the
+// leaves' solutions.
+enum { CR_LEAF_UP = 0, CR_NODE_UP = 1, CR_NODE_DOWN = 2, CR_LEAF_DOWN = 3 };
 struct CrPhase {
-    int kind, h, row0, nrow;
+    int kind, h, nnode, rec0;  // nodes: their level's h, their number, the level's first root record
 };
+// a leaf's table, in doubles: U[16][20] (root p, row k; k = 16, 17: the
+// separators' part of the right-hand side), V[16][16] (row k, root p), the
+// roots, the weights of the messages to the right and left separator; zero
+// past the leaf's rows (roots: the last one repeated)
+constexpr int kLeafU = 0, kLeafV = 320, kLeafRoot = 576, kLeafRight = 592, kLeafLeft = 608, kLeafStride = 624;
+// a node's record per root (node_roots(h) of them, past the block's 2h - 1
+// the last root with zero weights): root,
+// weight of the message to the right and to the left, weights of the node's
+// right-hand side, the left and the right solved row
+constexpr int kNodeRec = 8;
+__host__ __device__ constexpr int node_roots(int h) { return h < 4 ? 8 : 2 * h; }
 struct CrPlan {
     int kx = 0;
+    int rows = 0, nleaf = 0;
     long nsolve = 0;               // r solves per mode
     std::vector<CrPhase> phases;   // in execution order
-    std::vector<CrRow> rows;
-    std::vector<CrProg> progs;
-    std::vector<CrOp> ops;
+    std::vector<double> leaf, node;
 };
-// Root tables and programs of the z operator tridiag(an, bn, cn) of order n
-// (an[0] = cn[n-1] = 0), n = 2^k - 1.
+// Tables of the z operator tridiag(an, bn, cn) of order n (an[0] = cn[n-1] =
+// 0), n = 2^k - 1.
 int build_cr_plan(CrPlan &plan, int n, const double *an, const double *bn, const double *cn);
 
 // Device-side grid tables and workspace.  All pointers are device memory.
@@ -106,10 +99,9 @@ struct DeviceGrid {
     double *rz_an = nullptr;     // [NZ]
     double *rz_cn = nullptr;     // [NZ]
     double *rz_bn = nullptr;     // [NZ] BN (BN(1) = -CN(1); the spectral residual)
-    // cyclic reduction programs (CrPlan, uploaded)
-    CrOp *cr_ops = nullptr;
-    CrProg *cr_progs = nullptr;
-    CrRow *cr_rows = nullptr;
+    // cyclic reduction tables (CrPlan, uploaded)
+    double *cr_leaf = nullptr;
+    double *cr_node = nullptr;
     // refinement buffers (allocated on first use): the binary32 right-hand
     // side / residual spectrum and eigen coordinates, the step statistics
     float *spec32 = nullptr;     // [L][KMAX][JMAX]

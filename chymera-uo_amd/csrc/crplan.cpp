@@ -1,18 +1,39 @@
 // Host-side plan of the per-mode cyclic reduction (pot/blktri.f): the root
 // tables BLKTRI's initialisation computes (COMPB, pot/blktri.f:264-344, with
-// the eigenvalues of TQLRAT, :348-423) and, for every row the reduction and
-// back-substitution touch, the r solves and combinations of PRDCT
-// (:177-260) as flat op lists: the products of scalar factors as BLKTRI
-// chains them, the products with multiplier roots in partial-fraction form
-// (independent solves, summed).
+// the eigenvalues of TQLRAT, :348-423) and the weights with which the
+// reduction's products (PRDCT, :177-260) become sums of independent r solves.
+//
+// The z rows form a tree.  Row i = odd * h has a block of the 2h - 1 rows
+// i-h+1 .. i+h-1; with P(a..b) = det(T + Z(a..b)) = prod (T - root) over the
+// block's roots (negated eigenvalues of the z sub-matrix), l and r the roots
+// of the block's halves (rows before and after i) and b_p those of the block,
+// the block's Green's function gives
+//   from (i, i):      P(l) P(r) / P                        = sum a_p  / (T - b_p)
+//   to the row i + h: (-1)^h prod AN(i+1 .. i+h) P(l) / P  = sum wR_p / (T - b_p)
+//   to the row i - h: (-1)^h prod CN(i-h .. i-1) P(r) / P  = sum wL_p / (T - b_p)
+//   from X(i - h):    (-1)^h prod AN(i-h+1 .. i) P(r) / P  = sum cL_p / (T - b_p)
+//   from X(i + h):    (-1)^h prod CN(i .. i+h-1) P(l) / P  = sum cR_p / (T - b_p)
+// which are BLKTRI's products with its root tables in each P: its chains
+// divide by the half blocks' roots that the product before them multiplied by.
+// Every weight is formed in long double, numerator and denominator factors in
+// pairs so that no partial product overflows.
 //
 // The roots are formed with the reference's own arithmetic and convergence
 // rule.  That matters for parity: the reference's FP64 result differs from the
 // exact solution of the discrete system by up to a few 1e-12 (256x128x256),
 // and that difference comes from these root values, not from the rounding of
 // the r solves (any elimination order with the same roots reproduces it to
-// ~1e-14).
+// ~1e-14).  It comes from the large blocks, whose smallest roots lie furthest
+// below the convergence rule's scale.  Blocks of up to 31 rows can be solved
+// at once, with their exact eigenvectors and BLKTRI's roots, and stay within
+// 7e-14 of the reference's result; at 63 rows the roots' errors no longer fit
+// those of the blocks inside and around them (4e-12; KMAX = 32..512).  The
+// leaves have 15 rows, and fewer than half of the column: solved as one leaf,
+// a whole column on a grid much finer in r than in z (512x16) lands 9e-13
+// away, with one node above the leaves 1.5e-13.
+#include <algorithm>
 #include <cmath>
+#include <numeric>
 #include <vector>
 
 #include "chypot_impl.h"
@@ -94,82 +115,77 @@ int rational_ql(int n, double *d, double *e2, double machep)
     return 0;
 }
 
-struct Builder {
-    int n = 0, kx = 0;
-    // lev[lv][b * (2^(lv+1)-1) + i]: roots of block b of level lv (rows
-    // 1 + b 2^lv .. b 2^lv + 2^(lv+1) - 1), negated eigenvalues of the z
-    // sub-tridiagonal, by increasing magnitude; level 0 = -BN(row)
-    std::vector<std::vector<double>> lev;
-    std::vector<CrOp> ops;
-    std::vector<CrProg> progs;
+typedef std::vector<long double> Factors;
 
-    const double *blk(int lv, int b) const { return lev[lv].data() + (size_t)b * ((2 << lv) - 1); }
-
-    // Program of a product with divisors and multiplier roots (na = 0), by
-    // partial fractions: prod_j (T - c_j) / prod_i (T - b_i) = sum_i alpha_i
-    // (T - b_i)^-1 with alpha_i = prod_j (b_i - c_j) / prod_{k != i} (b_i - b_k).
-    // The multipliers are the eigenvalues of the two halves of the divisor's
-    // block, which interlace with the divisor roots (Cauchy), so every alpha_i
-    // is >= 0 and the sum does not cancel: its rounding is that of one more
-    // elimination order (~1e-14 from BLKTRI's product order, which applies the
-    // same roots one after another).  The solves are independent.  Each alpha
-    // is formed in long double with every numerator factor paired with a
-    // denominator factor, so no partial product overflows.
-    int prog_mult(int nd, const double *div, int n1, const double *m1r, int n2, const double *m2r, int sgn)
-    {
-        CrProg p{};
-        p.off = (int)ops.size();
-        p.sgn = (nd > 0 && sgn <= 0) ? -1.0 : 1.0;
-        p.has_pre = 0;
-        std::vector<long double> c;
-        for (int j = 0; j < n1; ++j) c.push_back(m1r[j]);
-        for (int j = 0; j < n2; ++j) c.push_back(m2r[j]);
-        for (int i = nd - 1; i >= 0; --i) {
-            long double al = 1.0L;
-            int kk = 0;
-            for (size_t j = 0; j < c.size(); ++j) {
-                while (kk == i) ++kk;
-                al *= ((long double)div[i] - c[j]) / ((long double)div[i] - (long double)div[kk]);
-                ++kk;
-            }
-            for (; kk < nd; ++kk)
-                if (kk != i) al /= ((long double)div[i] - (long double)div[kk]);
-            ops.push_back(CrOp{div[i], (double)al, CR_PF, 0});
+// out_p = prod(num(p)) / prod_{k != p} (b_p - b_k): num(p) the numerator's
+// factors, paired with the denominator's
+template <typename Num>
+void pole_weights(int nd, const double *b, Num num, double *out, size_t stride)
+{
+    for (int p = 0; p < nd; ++p) {
+        const Factors f = num(p);
+        long double v = 1.0L;
+        int k = 0;
+        for (long double x : f) {
+            while (k == p) ++k;
+            v *= k < nd ? x / ((long double)b[p] - (long double)b[k]) : x;
+            ++k;
         }
-        p.nsolve = (int)ops.size() - p.off;
-        progs.push_back(p);
-        return (int)progs.size() - 1;
+        for (; k < nd; ++k)
+            if (k != p) v /= (long double)b[p] - (long double)b[k];
+        out[(size_t)p * stride] = (double)v;
     }
+}
 
-    // program of a product of scalar factors aa[na-1..0] and nd = na-1 divisors
-    int prog_scale(int nd, const double *div, int na, const double *aa, int sgn)
-    {
-        CrProg p{};
-        p.off = (int)ops.size();
-        p.sgn = (nd > 0 && sgn <= 0) ? -1.0 : 1.0;
-        p.has_pre = 1;
-        p.pre = aa[na - 1];
-        int id = nd, ia = na - 1;
-        while (id > 0) {
-            CrOp op{div[--id], aa[--ia], CR_SCALE, 0};
-            ops.push_back(op);
-        }
-        p.nsolve = (int)ops.size() - p.off;
-        progs.push_back(p);
-        return (int)progs.size() - 1;
+// the tables of the leaf whose first row is r0 (0-based): the block's
+// eigenvectors in 80-bit arithmetic, rounded once, each with BLKTRI's root
+int leaf_table(double *t, int r0, int rows, int n, const double *an, const double *bn, const double *cn,
+               const double *roots)
+{
+    std::vector<long double> d(rows), e(rows + 1, 0.0L), q, sc(rows, 1.0L);
+    for (int k = 0; k < rows; ++k) {
+        d[k] = bn[r0 + k];
+        if (k == 0) continue;
+        sc[k] = sc[k - 1] * std::sqrt((long double)cn[r0 + k - 1] / (long double)an[r0 + k]);
+        e[k] = std::sqrt((long double)an[r0 + k] * (long double)cn[r0 + k - 1]);
     }
-};
+    const int rc = symmetric_tridiag_eigen(rows, d, e, q);
+    if (rc != CHY_OK) return rc;
+    // eigenvector order[p] belongs to the p-th root by value
+    std::vector<int> order(rows);
+    std::iota(order.begin(), order.end(), 0);
+    std::sort(order.begin(), order.end(), [&](int a, int b) { return -d[a] < -d[b]; });
+    std::vector<double> rt(roots, roots + rows);
+    std::sort(rt.begin(), rt.end());
+    const bool left = r0 > 0, right = r0 + rows < n;
+    for (int p = 0; p < rows; ++p) {
+        auto u = [&](int k) { return sc[k] * q[(size_t)k * rows + order[p]]; };
+        auto v = [&](int k) { return q[(size_t)k * rows + order[p]] / sc[k]; };
+        for (int k = 0; k < rows; ++k) {
+            t[kLeafU + p * 20 + k] = (double)u(k);
+            t[kLeafV + k * 16 + p] = (double)v(k);
+        }
+        if (left) {
+            t[kLeafU + p * 20 + 16] = (double)(-(long double)an[r0] * u(0));
+            t[kLeafLeft + p] = (double)(-(long double)cn[r0 - 1] * v(0));
+        }
+        if (right) {
+            t[kLeafU + p * 20 + 17] = (double)(-(long double)cn[r0 + rows - 1] * u(rows - 1));
+            t[kLeafRight + p] = (double)(-(long double)an[r0 + rows] * v(rows - 1));
+        }
+        t[kLeafRoot + p] = rt[p];
+    }
+    for (int p = rows; p < 16; ++p) t[kLeafRoot + p] = t[kLeafRoot + rows - 1];
+    return CHY_OK;
+}
 
 }  // namespace
 
 int build_cr_plan(CrPlan &plan, int n, const double *an, const double *bn, const double *cn)
 {
-    Builder B;
     int kx = 0;
     while ((1 << kx) - 1 < n) ++kx;
     if ((1 << kx) - 1 != n || kx < 2) return CHY_EUNSUPPORTED;
-    B.n = n;
-    B.kx = kx;
     // squared symmetrised couplings, formed as the reference forms them:
     // the square of sqrt(AN(i) CN(i-1)) (pot/blktri.f:283-293, :360-362)
     std::vector<double> cpl2(n, 0.0);
@@ -179,81 +195,83 @@ int build_cr_plan(CrPlan &plan, int n, const double *an, const double *bn, const
         double e = std::sqrt(arg);
         cpl2[i] = e * e;
     }
+    // lev[lv][b * (2^(lv+1)-1) + i]: roots of block b of level lv (rows
+    // 1 + b 2^lv .. b 2^lv + 2^(lv+1) - 1), negated eigenvalues of the z
+    // sub-tridiagonal, by increasing magnitude
     const double machep = cr_machep();
-    B.lev.resize(kx);
-    B.lev[0].resize(n);
-    for (int i = 0; i < n; ++i) B.lev[0][i] = -bn[i];
+    std::vector<std::vector<double>> lev(kx);
+    lev[0].resize(n);
+    for (int i = 0; i < n; ++i) lev[0][i] = -bn[i];
     for (int lv = 1; lv < kx; ++lv) {
         const int step = 1 << lv, size = 2 * step - 1, nblk = (1 << (kx - lv)) - 1;
-        B.lev[lv].resize((size_t)size * nblk);
+        lev[lv].resize((size_t)size * nblk);
         std::vector<double> d(size), e2(size);
         for (int b = 0; b < nblk; ++b) {
             const int r0 = b * step;
             for (int i = 0; i < size; ++i) d[i] = bn[r0 + i];
             for (int i = 0; i + 1 < size; ++i) e2[i] = cpl2[r0 + i + 1];
             if (rational_ql(size, d.data(), e2.data(), machep) != 0) return CHY_ENUMERIC;
-            for (int i = 0; i < size; ++i) B.lev[lv][(size_t)b * size + i] = -d[i];
+            for (int i = 0; i < size; ++i) lev[lv][(size_t)b * size + i] = -d[i];
         }
     }
-    // CN shifted one row down, as BLKTRI hands it to its reduction
-    // (pot/blktri.f:46-51): cnp[i] couples row i to row i-1's equation
-    std::vector<double> cnp(n);
-    cnp[0] = cn[n - 1];
-    for (int i = 1; i < n; ++i) cnp[i] = cn[i - 1];
+    auto block = [&](int lv, int b) { return lev[lv].data() + (size_t)b * ((2 << lv) - 1); };
 
     plan.kx = kx;
     plan.phases.clear();
-    plan.rows.clear();
-    auto begin_phase = [&](int kind, int h) {
-        CrPhase ph{};
-        ph.kind = kind;
-        ph.h = h;
-        ph.row0 = (int)plan.rows.size();
-        plan.phases.push_back(ph);
+    const int lv0 = std::min(kx - 1, 4);  // the lowest nodes' level; the leaves lie between multiples of 2^lv0
+    plan.rows = (1 << lv0) - 1;
+    plan.nleaf = (n + 1) >> lv0;
+    plan.leaf.assign((size_t)plan.nleaf * kLeafStride, 0.0);
+    for (int b = 0; b < plan.nleaf; ++b) {
+        const int rc = leaf_table(&plan.leaf[(size_t)b * kLeafStride], b << lv0, plan.rows, n, an, bn, cn,
+                                  block(lv0 - 1, 2 * b));
+        if (rc != CHY_OK) return rc;
+    }
+    plan.nsolve = 2L * plan.nleaf * plan.rows;
+    // the nodes' records, level by level (h = 2^lv is even, so (-1)^h = 1)
+    std::vector<int> rec0(kx, 0);
+    plan.node.clear();
+    for (int lv = lv0; lv < kx; ++lv) {
+        const int h = 1 << lv, nd = 2 * h - 1, nnode = (n + 1) / (2 * h), np = node_roots(h);
+        rec0[lv] = (int)(plan.node.size() / kNodeRec);
+        plan.node.resize(plan.node.size() + (size_t)nnode * np * kNodeRec, 0.0);
+        for (int t = 0; t < nnode; ++t) {
+            const int i = (2 * t + 1) * h;  // 1-based row
+            const double *b = block(lv, 2 * t), *l = block(lv - 1, 4 * t), *r = block(lv - 1, 4 * t + 2);
+            double *rec = &plan.node[((size_t)rec0[lv] + (size_t)t * np) * kNodeRec];
+            for (int p = 0; p < np; ++p) rec[p * kNodeRec] = b[std::min(p, nd - 1)];
+            // half: a half block's roots; c: h couplings, c[0] the first (1-based row first)
+            auto weights = [&](int slot, const double *half, const double *half2, const double *c, int first) {
+                pole_weights(nd, b, [&](int p) {
+                    Factors f;
+                    for (int j = 0; j < h - 1; ++j) {
+                        f.push_back((long double)b[p] - (long double)half[j]);
+                        if (half2) f.push_back((long double)b[p] - (long double)half2[j]);
+                        else f.push_back(c[first - 1 + j]);
+                    }
+                    if (!half2) f.push_back(c[first - 1 + h - 1]);
+                    return f;
+                }, rec + slot, kNodeRec);
+            };
+            weights(3, l, r, nullptr, 0);
+            if (i + h <= n) {
+                weights(1, l, nullptr, an, i + 1);
+                weights(5, l, nullptr, cn, i);
+            }
+            if (i - h >= 1) {
+                weights(2, r, nullptr, cn, i - h);
+                weights(4, r, nullptr, an, i - h + 1);
+            }
+        }
+        plan.nsolve += (long)nnode * nd * (lv < kx - 1 ? 2 : 1);
+    }
+    auto nodes = [&](int kind, int lv) {
+        plan.phases.push_back(CrPhase{kind, 1 << lv, (n + 1) / (2 << lv), rec0[lv]});
     };
-    auto end_phase = [&]() { plan.phases.back().nrow = (int)plan.rows.size() - plan.phases.back().row0; };
-    // reduction (pot/blktri.f:72-120)
-    for (int lv = 0; lv < kx - 1; ++lv) {
-        const int h = 1 << lv, iim = h - 1, iiz = 2 * h - 1, sg = (lv & 1) ? -1 : 1;
-        begin_phase(CR_PHASE_ODD, h);
-        for (int o = h; o <= n; o += 2 * h) {
-            const int b = o / h - 1;
-            CrRow r{o, -1, -1, -1};
-            r.pm = B.prog_mult(iiz, B.blk(lv, b), iim, lv ? B.blk(lv - 1, 2 * b) : nullptr, iim,
-                               lv ? B.blk(lv - 1, 2 * b + 2) : nullptr, sg);
-            plan.rows.push_back(r);
-        }
-        end_phase();
-        begin_phase(CR_PHASE_EVEN, h);
-        for (int e = 2 * h; e + h <= n; e += 2 * h) {
-            const int s = e / (2 * h);
-            CrRow r{e, -1, -1, -1};
-            r.pa = B.prog_scale(iim, lv ? B.blk(lv - 1, 4 * s - 2) : nullptr, h, an + (e - h), -sg);
-            r.pc = B.prog_scale(iim, lv ? B.blk(lv - 1, 4 * s) : nullptr, h, cnp.data() + e, -sg);
-            plan.rows.push_back(r);
-        }
-        end_phase();
-    }
-    // back substitution (pot/blktri.f:122-170)
-    for (int lv = kx - 1; lv >= 0; --lv) {
-        const int h = 1 << lv, iim = h - 1, iiz = 2 * h - 1, sg = (lv & 1) ? -1 : 1;
-        const int nrow = (1 << (kx - lv)) - 1;
-        begin_phase(CR_PHASE_BACK, h);
-        for (int jj = 1; jj <= nrow; jj += 2) {
-            const int i = jj * h;
-            CrRow r{i, -1, -1, -1};
-            if (jj > 1)
-                r.pa = B.prog_scale(iim, lv ? B.blk(lv - 1, 2 * jj - 2) : nullptr, h, an + (i - h), -sg);
-            if (jj < nrow) r.pc = B.prog_scale(iim, lv ? B.blk(lv - 1, 2 * jj) : nullptr, h, cnp.data() + i, -sg);
-            r.pm = B.prog_mult(iiz, B.blk(lv, jj - 1), iim, lv ? B.blk(lv - 1, 2 * jj - 2) : nullptr, iim,
-                               lv ? B.blk(lv - 1, 2 * jj) : nullptr, sg);
-            plan.rows.push_back(r);
-        }
-        end_phase();
-    }
-    plan.ops = std::move(B.ops);
-    plan.progs = std::move(B.progs);
-    plan.nsolve = (long)plan.ops.size();
+    plan.phases.push_back(CrPhase{CR_LEAF_UP, 0, 0, 0});
+    for (int lv = lv0; lv < kx - 1; ++lv) nodes(CR_NODE_UP, lv);
+    for (int lv = kx - 1; lv >= lv0; --lv) nodes(CR_NODE_DOWN, lv);
+    plan.phases.push_back(CrPhase{CR_LEAF_DOWN, 0, 0, 0});
     return CHY_OK;
 }
 

@@ -325,7 +325,7 @@ int build_grid(chy_grid *g, const chy_grid_desc *desc, int isym)
             wi[(size_t)p * PP + k] = (double)(qv / dsc[k]);  // stored [p][k]: reduction index major
         }
 
-    // ---- BLKTRI's root tables and the cyclic reduction's programs (crplan.cpp) ----
+    // ---- BLKTRI's root tables and the cyclic reduction's weights (crplan.cpp) ----
     CHY_TRY(build_cr_plan(g->cr, NZ, an.data(), bn.data(), cn.data()));
     g->mode_solver = cr_supported(g) ? CHY_MODES_CR : CHY_MODES_EIGEN;
     // two orders per wavefront where the r system fits 32 lanes: measured
@@ -469,9 +469,8 @@ int build_grid(chy_grid *g, const chy_grid_desc *desc, int isym)
         CHY_TRY(upload(g, &d.bm, bmp));
     }
     CHY_TRY(upload(g, &d.zx, zx));
-    CHY_TRY(upload(g, &d.cr_ops, g->cr.ops));
-    CHY_TRY(upload(g, &d.cr_progs, g->cr.progs));
-    CHY_TRY(upload(g, &d.cr_rows, g->cr.rows));
+    CHY_TRY(upload(g, &d.cr_leaf, g->cr.leaf));
+    CHY_TRY(upload(g, &d.cr_node, g->cr.node));
     // the z operator of the same system for the refinement's spectral residuals
     CHY_TRY(upload(g, &d.rz_an, an));
     CHY_TRY(upload(g, &d.rz_cn, cn));
