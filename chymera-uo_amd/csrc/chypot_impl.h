@@ -52,11 +52,15 @@ enum { CR_LEAF_UP = 0, CR_NODE_UP = 1, CR_NODE_DOWN = 2, CR_LEAF_DOWN = 3 };
 struct CrPhase {
     int kind, h, nnode, rec0;  // nodes: their level's h, their number, the level's first root record
 };
-// a leaf's table, in doubles: U[16][20] (root p, row k; k = 16, 17: the
-// separators' part of the right-hand side), V[16][16] (row k, root p), the
-// roots, the weights of the messages to the right and left separator; zero
-// past the leaf's rows (roots: the last one repeated)
-constexpr int kLeafU = 0, kLeafV = 320, kLeafRoot = 576, kLeafRight = 592, kLeafLeft = 608, kLeafStride = 624;
+// a leaf's table in doubles, LS = kLeafSpan rows and roots: U[LS][LS+4] (root p,
+// row k; k = LS, LS + 1: the separators' part of the right-hand side),
+// V[LS][LS] (row k, root p), the roots, the weights of the messages to the
+// right and left separator; zero past the leaf's rows (roots: the last one
+// repeated)
+constexpr int kLeafSpan = 16;
+constexpr int kLeafU = 0, kLeafV = kLeafSpan * (kLeafSpan + 4), kLeafRoot = kLeafV + kLeafSpan * kLeafSpan,
+              kLeafRight = kLeafRoot + kLeafSpan, kLeafLeft = kLeafRight + kLeafSpan,
+              kLeafStride = kLeafLeft + kLeafSpan;
 // a node's record per root (node_roots(h) of them, past the block's 2h - 1
 // the last root with zero weights): root,
 // weight of the message to the right and to the left, weights of the node's

@@ -27,14 +27,15 @@
 // One block of a launch is one tree node (or leaf) of one order m: the cosine
 // and sine parts share T_m, so every solve has two right-hand sides; solves
 // run on groups of G lanes (rtri.h), 64/G roots per wavefront at a time.  The
-// leaves' changes of basis (16 roots x 15..17 rows) run on the FP64 matrix
-// cores through LDS.  The spectrum spec[q][k][j] (J contiguous) is the mode
+// leaves' changes of basis run on the FP64 matrix cores through LDS.  The spectrum spec[q][k][j] (J contiguous) is the mode
 // right-hand side on entry (with POT3's boundary terms applied) and the mode
-// solution on exit.  What a block adds to the row on its left goes to the
-// grid's second workspace buffer (yh), what it adds to the row on its right
-// into the spectrum itself, so every row has one writer per launch and the
-// order of every sum is fixed.
+// solution on exit.  What the blocks add to a separating row goes to the grid's
+// second workspace buffer (yh), from its right side into its own row there and
+// from its left side into the row before (unused inside a leaf), so every row
+// has one writer per launch and the order of every sum is fixed.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "chypot_impl.h"
 #include "rtri.h"
@@ -71,187 +72,207 @@ struct Plane {
     }
 };
 
-// LDS vectors of R*G values: element j = R g + r at r (G + 2) + g, so that
-// the lanes of a solve read consecutive words and 16 consecutive j (a matrix
-// operand) fall in 16 different 8-byte banks
-template <int R, int G>
-struct Vec {
-    static constexpr int PITCH = G + 2, SIZE = R * PITCH;
-    static __device__ __forceinline__ int at(int j) { return (j % R) * PITCH + j / R; }
-};
-
-// The two sums (to the right neighbour, to the left one) of a block's W
-// wavefronts, each lane holding its part for its root's group: added over the
-// wavefront's groups, then over the wavefronts in order, and handed to
-// out(sum, part, j, value) for j < M.
+// The sums of a node's block (one or two, two parts each): every lane holds
+// its root group's share; the W * 64/G shares of one sum at a time meet in LDS
+// and are added in order, out(sum, part, j, value) for j < M.  (Adding the
+// groups of a wavefront by lane exchanges first cost 300 instructions per
+// wavefront, two thirds of a solve.)
 template <int R, int G, int W, int NSUM, typename Out>
-__device__ __forceinline__ void block_sums(double (&s)[NSUM][2][R], double *lds, int M, Out out)
+__device__ __forceinline__ void block_sums(const double (&s)[NSUM][2][R], double *lds, int M, Out out)
 {
     typedef Vec<R, G> V;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, gl = lane % G;
-    const int lane4 = 4 * lane;
+    constexpr int SLOTS = W * 64 / G;
+    const int slot = threadIdx.x / G, gl = threadIdx.x % G;
 #pragma unroll
-    for (int n = 0; n < NSUM; ++n)
+    for (int n = 0; n < NSUM; ++n) {
+        __syncthreads();  // every wavefront is done with what lds held
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int r = 0; r < R; ++r) {
-                if constexpr (G <= 8) s[n][h][r] += lane_swap<8>(s[n][h][r], lane4);
-                if constexpr (G <= 16) s[n][h][r] += lane_swap<16>(s[n][h][r], lane4);
-                if constexpr (G <= 32) s[n][h][r] += lane_swap<32>(s[n][h][r], lane4);
-            }
-    __syncthreads();  // every wavefront is done with what lds held
-    if (lane < G) {
+            for (int r = 0; r < R; ++r) lds[(slot * 2 + h) * V::SIZE + r * V::PITCH + gl] = s[n][h][r];
+        __syncthreads();
+        for (int e = threadIdx.x; e < 2 * R * G; e += 64 * W) {
+            const int j = e % (R * G), h = e / (R * G);
+            const double *p = lds + h * V::SIZE + V::at(j);
+            double v = p[0];
 #pragma unroll
-        for (int n = 0; n < NSUM; ++n)
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int r = 0; r < R; ++r)
-                    lds[((wave * NSUM + n) * 2 + h) * V::SIZE + r * V::PITCH + gl] = s[n][h][r];
-    }
-    __syncthreads();
-    for (int e = threadIdx.x; e < NSUM * 2 * R * G; e += 64 * W) {
-        const int j = e % (R * G), nh = e / (R * G);
-        double v = lds[nh * V::SIZE + V::at(j)];
-#pragma unroll
-        for (int w = 1; w < W; ++w) v += lds[(w * NSUM * 2 + nh) * V::SIZE + V::at(j)];
-        if (j < M) out(nh / 2, nh % 2, j, v);
+            for (int t = 1; t < SLOTS; ++t) v += p[t * 2 * V::SIZE];
+            if (j < M) out(n, h, j, v);
+        }
     }
 }
 
-// A leaf: rows i0 .. i0 + rows - 1 (0-based, i0 = (rows + 1) b), the separating rows
-// i0 - 1 and i0 + rows beside it.  Up: the leaf's messages to the separators.
-// Down: its rows from the solved separators.  16 roots (zero-padded).
-//   gather   D[p][j] = sum_k U[p][k] Y[k][j]   (down: k = 16, 17 the separators)
+// Leaves: rows i0 .. i0 + rows - 1 (0-based, i0 = (rows + 1) b), the
+// separating rows i0 - 1 and i0 + rows beside them.  Up: a leaf's messages to
+// the separators.  Down: its rows from the solved separators.  LS roots
+// (zero-padded).
+//   gather   D[p][j] = sum_k U[p][k] Y[k][j]   (down: k = LS, LS + 1 the separators)
 //   solves   one root per group of lanes
 //   scatter  X[k][j] = sum_p V[k][p] D[p][j]   (down)
 // V_MFMA_F64_16X16X4F64: A lane l holds A[l%16][l/16], B lane l B[l/16][l%16],
-// the result D[l/16 + 4v][l%16].  LDS holds the 16 x 2 vectors: 70 KB at
-// JMAX <= 256 (two blocks per CU), 135 KB at 512.
+// the result D[l/16 + 4v][l%16].
+//
+// A block takes `run` leaves of one order one after the other.  It is bound by
+// HBM (up: the spectrum read once, down: read and written), while its solves
+// keep the VALU busy for about half as long, so the next leaf's rows are
+// loaded into registers (a matrix operand each) before the current one is
+// solved.  Loads and stores of a wavefront complete in order: nothing the
+// solves need is loaded after those rows (the roots and weights wait in LDS),
+// and the next leaf's U is loaded before the current one's results are
+// stored.  LDS holds the 16 x 2 vectors: 76 KB at JMAX <= 256 (two blocks of 4
+// wavefronts per CU), 148 KB at 512 (one of 8).  (Leaves of 31 rows need 146 KB
+// at JMAX <= 256 and twice the matrix products per row: one block per CU, its
+// phases one after another, 1.45 ms down and 1.2 ms up per 32 fields at
+// 256x128x256 against 1.0 and 1.0, more than the saved level of nodes gives.)
 template <int R, int G, int W, bool DOWN>
-__global__ __launch_bounds__(64 * W, 2) void k_cr_leaf(CrArgs a, const Fields F)
+__global__ __launch_bounds__(64 * W, 2) void k_cr_leaf(CrArgs a, const Fields F, int run)
 {
     typedef Vec<R, G> V;
-    constexpr int SPW = 64 / G, JP = R * G, CT = JP / 16, KS = DOWN ? 5 : 4;
-    __shared__ double lds[16 * 2 * V::SIZE];
+    constexpr int LS = kLeafSpan, SPW = 64 / G, JP = R * G, CT = JP / 16, KS = LS / 4 + (DOWN ? 1 : 0);
+    constexpr int NT = (2 * CT + W - 1) / W;  // column tiles per wavefront
+    __shared__ double lds[LS * 2 * V::SIZE], tri[3 * V::SIZE], wts[3 * LS];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int gl = lane % G, sub = lane / G, lr = lane & 15, lk = lane >> 4, lane4 = 4 * lane;
-    const int m = (int)blockIdx.x / a.nleaf, b = (int)blockIdx.x % a.nleaf;
-    const int M = a.M, nr = a.rows, i0 = b * (nr + 1);
-    const double *tab = a.leaf + (size_t)b * kLeafStride;
+    const int gl = lane % G, sub = lane / G, lr = lane & 15, lk = lane >> 4;
+    const int nrun = (a.nleaf + run - 1) / run;
+    const int m = (int)blockIdx.x / nrun, b0 = (int)blockIdx.x % nrun * run, b1 = min(b0 + run, a.nleaf);
+    const int M = a.M, nr = a.rows;
     const Plane<R, G> q(a, F, m);
 
-    double av[KS];
+    // this wavefront's column tiles of leaf b: row k of lane l, any valid row
+    // where U is zero
+    double y[NT][KS];
+    auto fetch = [&](int b) {
+        const int i0 = b * (nr + 1);
+        size_t off[KS];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) av[ks] = tab[kLeafU + lr * 20 + 4 * ks + lk];
-    int row[KS];  // the z row this lane loads for each k-step (any valid row where U is zero)
+        for (int ks = 0; ks < KS; ++ks) {
+            const int k = 4 * ks + lk;
+            const int row = k < LS ? i0 + min(k, nr - 1) : (k == LS ? max(i0 - 1, 0) : i0 + nr);
+            off[ks] = (size_t)row * a.J;
+        }
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-        const int k = 4 * ks + lk;
-        if (k < 16) row[ks] = i0 + (k < nr ? k : nr - 1);
-        else row[ks] = k == 16 ? (i0 > 0 ? i0 - 1 : 0) : i0 + nr;
-    }
-#pragma unroll 4
-    for (int t = wave; t < 2 * CT; t += W) {
-        const int h = t / CT, j = (t % CT) * 16 + lr, jc = j < M ? j : M - 1;
-        dx4 acc = dx4{0.0, 0.0, 0.0, 0.0};
-        if (h == 0 || q.two) {
-            const double *src = (h ? q.ss : q.sc) + jc;
-            double y[KS];
+        for (int t = 0; t < NT; ++t) {
+            const int tt = min(wave + t * W, 2 * CT - 1), h = tt / CT;  // the same for the wavefront
+            const int j = min((tt % CT) * 16 + lr, M - 1);
+            const double *src = (h ? q.ss : q.sc) + j;
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks) y[ks] = src[(size_t)row[ks] * a.J];
+            for (int ks = 0; ks < KS; ++ks) y[t][ks] = src[off[ks]];
+        }
+    };
+    double av[KS], wt;  // U's operands; this thread's root or weight
+    auto tables = [&](int b) {
+        const double *tab = a.leaf + (size_t)b * kLeafStride;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) av[ks] = tab[kLeafU + lr * (LS + 4) + 4 * ks + lk];
+        wt = tab[kLeafRoot + min((int)threadIdx.x, 3 * LS - 1)];
+    };
+    fetch(b0);
+    tables(b0);
+    rtri_load<R, G>(tri, a.am, a.cm, a.bm + (size_t)m * a.JP, M, 64 * W);
+    const Neigh at = neighbours<G>(lane);
+
+#pragma unroll 1
+    for (int b = b0; b < b1; ++b) {
+        const int i0 = b * (nr + 1);
+        if (threadIdx.x < 3 * LS) wts[threadIdx.x] = wt;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            const int tt = wave + t * W, h = tt / CT, j = (tt % CT) * 16 + lr;
+            if (tt >= 2 * CT) break;
+            const bool on = j < M && (h == 0 || q.two);
+            dx4 acc = dx4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks)
-                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[ks], j < M ? y[ks] : 0.0, acc, 0, 0, 0);
-        }
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[ks], on ? y[t][ks] : 0.0, acc, 0, 0, 0);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) lds[((lk + 4 * v) * 2 + h) * V::SIZE + V::at(j)] = acc[v];
-    }
-    double ca[R], cb[R], cc[R];
-    rtri_rows<R>(a.am, a.cm, a.bm + (size_t)m * a.JP, gl * R, M, ca, cb, cc);
-    __syncthreads();
+            for (int v = 0; v < 4; ++v) lds[((lk + 4 * v) * 2 + h) * V::SIZE + V::at(j)] = acc[v];
+        }
+        __syncthreads();
+        if (b + 1 < b1) fetch(b + 1);
 
-    double s[2][2][R];
-    if constexpr (!DOWN) {
-#pragma unroll
-        for (int r = 0; r < R; ++r) s[0][0][r] = s[0][1][r] = s[1][0][r] = s[1][1][r] = 0.0;
-    }
 #pragma unroll 1
-    for (int p0 = wave * SPW; p0 < nr; p0 += W * SPW) {
-        const int p = p0 + sub;
-        const double rt = tab[kLeafRoot + p];
-        double d0[R], d1[R];
-        double *v0 = lds + (size_t)(p * 2) * V::SIZE + gl, *v1 = v0 + V::SIZE;
+        for (int p0 = wave * SPW; p0 < nr; p0 += W * SPW) {
+            const int p = p0 + sub;
+            const double rt = wts[p];
+            asm volatile("" ::: "memory");  // T's rows are read anew in every round, not kept in registers
+            double d0[R], d1[R];
+            double *v0 = lds + (size_t)(p * 2) * V::SIZE + gl, *v1 = v0 + V::SIZE;
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            d0[r] = v0[r * V::PITCH];
-            d1[r] = v1[r * V::PITCH];
-        }
-        rtri_solve<R, G>(ca, cb, cc, rt, lane4, d0, d1);
-        if constexpr (DOWN) {
+            for (int r = 0; r < R; ++r) {
+                d0[r] = v0[r * V::PITCH];
+                d1[r] = v1[r * V::PITCH];
+            }
+            rtri_solve<R, G>(tri + gl, rt, at, d0, d1);
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 v0[r * V::PITCH] = d0[r];
                 v1[r * V::PITCH] = d1[r];
             }
-        } else {
-            const double wr = tab[kLeafRight + p], wl = tab[kLeafLeft + p];
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                s[0][0][r] = __builtin_fma(wr, d0[r], s[0][0][r]);
-                s[0][1][r] = __builtin_fma(wr, d1[r], s[0][1][r]);
-                s[1][0][r] = __builtin_fma(wl, d0[r], s[1][0][r]);
-                s[1][1][r] = __builtin_fma(wl, d1[r], s[1][1][r]);
-            }
         }
-    }
 
-    if constexpr (!DOWN) {
-        block_sums<R, G, W, 2>(s, lds, M, [&](int n, int h, int j, double v) {
-            if (h == 1 && !q.two) return;
-            if (n == 0) {
-                if (b + 1 < a.nleaf) (h ? q.ss : q.sc)[(size_t)(i0 + nr) * a.J + j] += v;
-            } else if (b > 0) {
-                (h ? q.ps : q.pc)[(size_t)(i0 - 1) * a.JP + j] = v;
+        if constexpr (!DOWN) {
+            if (b + 1 < b1) tables(b + 1);
+            __syncthreads();
+            // to the right separator through the second buffer's row before
+            // it, to the left one through its own
+            for (int e = threadIdx.x; e < 2 * JP; e += 64 * W) {
+                const int h = e / JP, j = e % JP;
+                const double *x = lds + h * V::SIZE + V::at(j);
+                double right = 0.0, left = 0.0;
+#pragma unroll
+                for (int p = 0; p < LS; ++p) {
+                    const double v = x[(size_t)(p * 2) * V::SIZE];
+                    right = __builtin_fma(wts[LS + p], v, right);
+                    left = __builtin_fma(wts[2 * LS + p], v, left);
+                }
+                if (j >= M || (h == 1 && !q.two)) continue;
+                double *out = (h ? q.ps : q.pc) + j;
+                if (b + 1 < a.nleaf) out[(size_t)(i0 + nr - 1) * a.JP] = right;
+                if (b > 0) out[(size_t)(i0 - 1) * a.JP] = left;
             }
-        });
-    } else {
-        double vv[4];
+        } else {
+            double vv[LS / 4];
+            {
+                const double *tab = a.leaf + (size_t)b * kLeafStride + kLeafV;
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) vv[ks] = tab[kLeafV + lr * 16 + 4 * ks + lk];
-        __syncthreads();
+                for (int ks = 0; ks < LS / 4; ++ks) vv[ks] = tab[lr * LS + 4 * ks + lk];
+            }
+            if (b + 1 < b1) tables(b + 1);
+            __syncthreads();
 #pragma unroll 4
-        for (int t = wave; t < 2 * CT; t += W) {
-            const int h = t / CT, j = (t % CT) * 16 + lr;
-            if (h == 1 && !q.two) break;  // the same for the wavefront, and for every later t
-            dx4 acc = dx4{0.0, 0.0, 0.0, 0.0};
+            for (int t = wave; t < 2 * CT; t += W) {
+                const int h = t / CT, j = (t % CT) * 16 + lr;
+                if (h == 1 && !q.two) break;  // the same for the wavefront, and for every later t
+                dx4 acc = dx4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-            for (int ks = 0; ks < 4; ++ks)
-                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                    vv[ks], lds[((4 * ks + lk) * 2 + h) * V::SIZE + V::at(j)], acc, 0, 0, 0);
-            double *dst = (h ? q.ss : q.sc) + (size_t)i0 * a.J + j;
+                for (int ks = 0; ks < LS / 4; ++ks)
+                    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                        vv[ks], lds[((4 * ks + lk) * 2 + h) * V::SIZE + V::at(j)], acc, 0, 0, 0);
+                double *dst = (h ? q.ss : q.sc) + (size_t)i0 * a.J + j;
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int k = lk + 4 * v;
-                if (k < nr && j < M) dst[(size_t)k * a.J] = acc[v];
+                for (int v = 0; v < 4; ++v) {
+                    const int k = lk + 4 * v;
+                    if (k < nr && j < M) dst[(size_t)k * a.J] = acc[v];
+                }
             }
         }
+        __syncthreads();  // lds is free for the next leaf
     }
 }
 
 // A node of the tree: row i = (2 n + 1) h (1-based) with its block of 2h - 1
 // rows; the roots are dealt to the block's W wavefronts in turn.  Its
-// right-hand side is the spectrum's row plus the second buffer's.
+// right-hand side is the spectrum's row plus the messages from its right (the
+// second buffer's row) and from its left (the row before).
 template <int R, int G, int W, bool DOWN>
-__global__ __launch_bounds__(64 * W, 2) void k_cr_node(CrArgs a, const Fields F, CrPhase ph)
+__global__ __launch_bounds__(64 * W, R == 8 ? 3 : 4) void k_cr_node(CrArgs a, const Fields F, CrPhase ph)
 {
     typedef Vec<R, G> V;
     constexpr int SPW = 64 / G, JP = R * G, NIN = DOWN ? 3 : 1, NSUM = DOWN ? 1 : 2;
-    constexpr int NV = NIN * 2 > W * NSUM * 2 ? NIN * 2 : W * NSUM * 2;
-    __shared__ double lds[NV * V::SIZE];
+    constexpr int NV = NIN > W * SPW ? NIN * 2 : W * SPW * 2;
+    __shared__ double lds[NV * V::SIZE], tri[3 * V::SIZE];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int gl = lane % G, sub = lane / G, lane4 = 4 * lane;
+    const int gl = lane % G, sub = lane / G;
     const int m = (int)blockIdx.x / ph.nnode, n = (int)blockIdx.x % ph.nnode;
     const int h = ph.h, M = a.M;
     const int i = (2 * n + 1) * h - 1;          // this row, 0-based
@@ -264,25 +285,20 @@ __global__ __launch_bounds__(64 * W, 2) void k_cr_node(CrArgs a, const Fields F,
         double v = 0.0;
         if (j < M && (c == 0 || q.two)) {
             const double *S = (c ? q.ss : q.sc) + j, *Pv = (c ? q.ps : q.pc) + j;
-            if (w == 0) v = S[(size_t)i * a.J] + Pv[(size_t)i * a.JP];
+            if (w == 0) v = S[(size_t)i * a.J] + (Pv[(size_t)i * a.JP] + Pv[(size_t)(i - 1) * a.JP]);
             else if (w == 1 ? left : right) v = S[(size_t)(w == 1 ? i - h : i + h) * a.J];
         }
         lds[(w * 2 + c) * V::SIZE + V::at(j)] = v;
     }
-    double ca[R], cb[R], cc[R];
-    rtri_rows<R>(a.am, a.cm, a.bm + (size_t)m * a.JP, gl * R, M, ca, cb, cc);
+    rtri_load<R, G>(tri, a.am, a.cm, a.bm + (size_t)m * a.JP, M, 64 * W);
+    const Neigh at = neighbours<G>(lane);
     __syncthreads();
 
-    double s[NSUM][2][R], x0[R], x1[R];
+    double s[NSUM][2][R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
+    for (int r = 0; r < R; ++r)
 #pragma unroll
         for (int t = 0; t < NSUM; ++t) s[t][0][r] = s[t][1][r] = 0.0;
-        if constexpr (!DOWN) {
-            x0[r] = lds[r * V::PITCH + gl];
-            x1[r] = lds[V::SIZE + r * V::PITCH + gl];
-        }
-    }
     const double *rec = a.node + ((size_t)ph.rec0 + (size_t)n * node_roots(h) + sub) * kNodeRec;
     double rt = rec[(size_t)wave * SPW * kNodeRec];
 #pragma unroll 1
@@ -291,19 +307,20 @@ __global__ __launch_bounds__(64 * W, 2) void k_cr_node(CrArgs a, const Fields F,
         const double w0 = rp[DOWN ? 3 : 1], w1 = rp[DOWN ? 4 : 2], w2 = DOWN ? rp[5] : 0.0;
         const int pn = p + W * SPW < 2 * h ? p + W * SPW : p;
         const double rt_next = rec[(size_t)pn * kNodeRec];
+        asm volatile("" ::: "memory");  // the LDS operands are read anew in every round, not kept in registers
         double d0[R], d1[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
+            const double *l = lds + r * V::PITCH + gl;
             if constexpr (DOWN) {
-                const double *l = lds + r * V::PITCH + gl;
                 d0[r] = __builtin_fma(w2, l[4 * V::SIZE], __builtin_fma(w1, l[2 * V::SIZE], w0 * l[0]));
                 d1[r] = __builtin_fma(w2, l[5 * V::SIZE], __builtin_fma(w1, l[3 * V::SIZE], w0 * l[V::SIZE]));
             } else {
-                d0[r] = x0[r];
-                d1[r] = x1[r];
+                d0[r] = l[0];
+                d1[r] = l[V::SIZE];
             }
         }
-        rtri_solve<R, G>(ca, cb, cc, rt, lane4, d0, d1);
+        rtri_solve<R, G>(tri + gl, rt, at, d0, d1);
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             if constexpr (DOWN) {
@@ -323,7 +340,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_cr_node(CrArgs a, const Fields F,
         if constexpr (DOWN) {
             (c ? q.ss : q.sc)[(size_t)i * a.J + j] = v;
         } else if (t == 0) {
-            if (right) (c ? q.ss : q.sc)[(size_t)(i + h) * a.J + j] += v;
+            if (right) (c ? q.ps : q.pc)[(size_t)(i + h - 1) * a.JP + j] += v;
         } else if (left) {
             (c ? q.ps : q.pc)[(size_t)(i - h) * a.JP + j] += v;
         }
@@ -340,27 +357,46 @@ void launch_node(const CrPhase &ph, const CrArgs &a, const Fields &F, hipStream_
         hipLaunchKernelGGL((k_cr_node<R, G, W, false>), grid, dim3(64 * W), 0, s, a, F, ph);
 }
 
+template <int R, int G>
+void launch_leaf(const CrPhase &ph, const chy_grid *g, const CrArgs &a, const Fields &F, hipStream_t s)
+{
+    // wavefronts: two rounds of 64/G roots each, at most 8
+    constexpr int rounds = kLeafSpan * G / 64, W = rounds >= 16 ? 8 : rounds / 2;
+    // leaves per block: the fewest rounds of blocks over the CUs, each a run
+    // and the exposed first load (about half a leaf's time)
+    constexpr int lds = (2 * kLeafSpan + 3) * Vec<R, G>::SIZE * 8;
+    const long slots = (long)g->ncu * std::max(1, std::min(160 * 1024 / lds, 8 / W));
+    auto cost = [&](int run) {
+        const long blocks = (long)(g->N + 1) * ((a.nleaf + run - 1) / run) * F.nf;
+        return (blocks + slots - 1) / slots * (2 * run + 1);
+    };
+    int run = 1;
+    for (int r = 2; r <= a.nleaf; r *= 2)
+        if (cost(r) <= cost(run)) run = r;
+    const dim3 grid((unsigned)((g->N + 1) * ((a.nleaf + run - 1) / run)), F.nf);
+    if (ph.kind == CR_LEAF_UP)
+        hipLaunchKernelGGL((k_cr_leaf<R, G, W, false>), grid, dim3(64 * W), 0, s, a, F, run);
+    else
+        hipLaunchKernelGGL((k_cr_leaf<R, G, W, true>), grid, dim3(64 * W), 0, s, a, F, run);
+}
+
 // One launch per phase.  Wavefronts per node: four rounds of 64/G roots each,
-// at most 8, so that a single field's launch of any level holds about one
-// wavefront per SIMD (N+1 orders x nodes x W).
+// at most 4, so that three blocks share a CU (296 us per level and 32 fields
+// at 256x128x256; with 8 wavefronts only one block fits the registers beside
+// itself, 382 us; one field alone takes 20-25 us either way).
 template <int R, int G>
 int launch_phases(const chy_grid *g, const CrArgs &a, const Fields &F, hipStream_t s)
 {
     constexpr int SPW = 64 / G;
-    constexpr int WL = G == 64 ? 8 : (G == 8 ? 2 : 4);
-    const dim3 leaves((unsigned)((g->N + 1) * a.nleaf), F.nf);
     for (const CrPhase &ph : g->cr.phases) {
-        if (ph.kind == CR_LEAF_UP) {
-            hipLaunchKernelGGL((k_cr_leaf<R, G, WL, false>), leaves, dim3(64 * WL), 0, s, a, F);
-        } else if (ph.kind == CR_LEAF_DOWN) {
-            hipLaunchKernelGGL((k_cr_leaf<R, G, WL, true>), leaves, dim3(64 * WL), 0, s, a, F);
+        if (ph.kind == CR_LEAF_UP || ph.kind == CR_LEAF_DOWN) {
+            launch_leaf<R, G>(ph, g, a, F, s);
         } else {
-            switch (2 * ph.h / (4 * SPW)) {
+            switch (std::min(4, 2 * ph.h / (4 * SPW))) {
             case 0:
             case 1: launch_node<R, G, 1>(ph, a, F, s); break;
             case 2: launch_node<R, G, 2>(ph, a, F, s); break;
-            case 4: launch_node<R, G, 4>(ph, a, F, s); break;
-            default: launch_node<R, G, 8>(ph, a, F, s); break;
+            default: launch_node<R, G, 4>(ph, a, F, s); break;
             }
         }
     }

@@ -28,9 +28,9 @@
 // at once, with their exact eigenvectors and BLKTRI's roots, and stay within
 // 7e-14 of the reference's result; at 63 rows the roots' errors no longer fit
 // those of the blocks inside and around them (4e-12; KMAX = 32..512).  The
-// leaves have 15 rows, and fewer than half of the column: solved as one leaf,
-// a whole column on a grid much finer in r than in z (512x16) lands 9e-13
-// away, with one node above the leaves 1.5e-13.
+// leaves have at most 15 rows (cr.hip), and fewer than half of the column:
+// solved as one leaf, a whole column on a grid much finer in r than in z
+// (512x16) lands 9e-13 away, with one node above the leaves 1.5e-13.
 #include <algorithm>
 #include <cmath>
 #include <numeric>
@@ -115,24 +115,23 @@ int rational_ql(int n, double *d, double *e2, double machep)
     return 0;
 }
 
-typedef std::vector<long double> Factors;
-
-// out_p = prod(num(p)) / prod_{k != p} (b_p - b_k): num(p) the numerator's
-// factors, paired with the denominator's
+// out_p = prod(num(p, f)) / prod_{k != p} (b_p - b_k): num fills f with the
+// numerator's factors and returns their number; they are paired with the
+// denominator's
 template <typename Num>
-void pole_weights(int nd, const double *b, Num num, double *out, size_t stride)
+void pole_weights(int nd, const double *b, std::vector<long double> &f, Num num, double *out, size_t stride)
 {
     for (int p = 0; p < nd; ++p) {
-        const Factors f = num(p);
+        const int nf = num(p, f.data());
+        const long double bp = b[p];
         long double v = 1.0L;
         int k = 0;
-        for (long double x : f) {
-            while (k == p) ++k;
-            v *= k < nd ? x / ((long double)b[p] - (long double)b[k]) : x;
-            ++k;
+        for (int i = 0; i < nf; ++i, ++k) {
+            if (k == p) ++k;
+            v *= k < nd ? f[i] / (bp - (long double)b[k]) : f[i];
         }
         for (; k < nd; ++k)
-            if (k != p) v /= (long double)b[p] - (long double)b[k];
+            if (k != p) v /= bp - (long double)b[k];
         out[(size_t)p * stride] = (double)v;
     }
 }
@@ -162,20 +161,20 @@ int leaf_table(double *t, int r0, int rows, int n, const double *an, const doubl
         auto u = [&](int k) { return sc[k] * q[(size_t)k * rows + order[p]]; };
         auto v = [&](int k) { return q[(size_t)k * rows + order[p]] / sc[k]; };
         for (int k = 0; k < rows; ++k) {
-            t[kLeafU + p * 20 + k] = (double)u(k);
-            t[kLeafV + k * 16 + p] = (double)v(k);
+            t[kLeafU + p * (kLeafSpan + 4) + k] = (double)u(k);
+            t[kLeafV + k * kLeafSpan + p] = (double)v(k);
         }
         if (left) {
-            t[kLeafU + p * 20 + 16] = (double)(-(long double)an[r0] * u(0));
+            t[kLeafU + p * (kLeafSpan + 4) + kLeafSpan] = (double)(-(long double)an[r0] * u(0));
             t[kLeafLeft + p] = (double)(-(long double)cn[r0 - 1] * v(0));
         }
         if (right) {
-            t[kLeafU + p * 20 + 17] = (double)(-(long double)cn[r0 + rows - 1] * u(rows - 1));
+            t[kLeafU + p * (kLeafSpan + 4) + kLeafSpan + 1] = (double)(-(long double)cn[r0 + rows - 1] * u(rows - 1));
             t[kLeafRight + p] = (double)(-(long double)an[r0 + rows] * v(rows - 1));
         }
         t[kLeafRoot + p] = rt[p];
     }
-    for (int p = rows; p < 16; ++p) t[kLeafRoot + p] = t[kLeafRoot + rows - 1];
+    for (int p = rows; p < kLeafSpan; ++p) t[kLeafRoot + p] = rt[rows - 1];
     return CHY_OK;
 }
 
@@ -218,7 +217,7 @@ int build_cr_plan(CrPlan &plan, int n, const double *an, const double *bn, const
 
     plan.kx = kx;
     plan.phases.clear();
-    const int lv0 = std::min(kx - 1, 4);  // the lowest nodes' level; the leaves lie between multiples of 2^lv0
+    const int lv0 = std::min(kx - 1, 4);  // the lowest nodes' level: leaves of 2^lv0 - 1 rows
     plan.rows = (1 << lv0) - 1;
     plan.nleaf = (n + 1) >> lv0;
     plan.leaf.assign((size_t)plan.nleaf * kLeafStride, 0.0);
@@ -230,6 +229,7 @@ int build_cr_plan(CrPlan &plan, int n, const double *an, const double *bn, const
     plan.nsolve = 2L * plan.nleaf * plan.rows;
     // the nodes' records, level by level (h = 2^lv is even, so (-1)^h = 1)
     std::vector<int> rec0(kx, 0);
+    std::vector<long double> factors(n + 1);
     plan.node.clear();
     for (int lv = lv0; lv < kx; ++lv) {
         const int h = 1 << lv, nd = 2 * h - 1, nnode = (n + 1) / (2 * h), np = node_roots(h);
@@ -242,15 +242,15 @@ int build_cr_plan(CrPlan &plan, int n, const double *an, const double *bn, const
             for (int p = 0; p < np; ++p) rec[p * kNodeRec] = b[std::min(p, nd - 1)];
             // half: a half block's roots; c: h couplings, c[0] the first (1-based row first)
             auto weights = [&](int slot, const double *half, const double *half2, const double *c, int first) {
-                pole_weights(nd, b, [&](int p) {
-                    Factors f;
+                pole_weights(nd, b, factors, [&](int p, long double *f) {
+                    const long double bp = b[p];
+                    int nf = 0;
                     for (int j = 0; j < h - 1; ++j) {
-                        f.push_back((long double)b[p] - (long double)half[j]);
-                        if (half2) f.push_back((long double)b[p] - (long double)half2[j]);
-                        else f.push_back(c[first - 1 + j]);
+                        f[nf++] = bp - (long double)half[j];
+                        f[nf++] = half2 ? bp - (long double)half2[j] : (long double)c[first - 1 + j];
                     }
-                    if (!half2) f.push_back(c[first - 1 + h - 1]);
-                    return f;
+                    if (!half2) f[nf++] = c[first - 1 + h - 1];
+                    return nf;
                 }, rec + slot, kNodeRec);
             };
             weights(3, l, r, nullptr, 0);

@@ -50,36 +50,50 @@ __device__ __forceinline__ T lane_next(T x)
 
 // x of the lane at byte address addr (4 * lane, modulo the wavefront) through
 // the LDS crossbar
-__device__ __forceinline__ double crossbar(double x, int addr)
+__device__ __forceinline__ int crossbar_word(int v, int addr) { return __builtin_amdgcn_ds_bpermute(addr, v); }
+
+// f applied to both words of x (double: low, then high)
+template <typename F>
+__device__ __forceinline__ double by_word(double x, F f)
 {
     const long long v = __double_as_longlong(x);
-    const int lo = __builtin_amdgcn_ds_bpermute(addr, (int)(v & 0xffffffffll));
-    const int hi = __builtin_amdgcn_ds_bpermute(addr, (int)(v >> 32));
+    const int lo = f((int)(v & 0xffffffffll)), hi = f((int)(v >> 32));
     return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
 
-// x of lane i ^ S, S a power of two; lane4 = 4 * lane.  Within a row of 16
-// lanes by DPP: quad permutations for 1 and 2, for 4 and 8 a shift either way,
-// the second written to its own half only.
-template <int S>
-__device__ __forceinline__ int lane_swap_word(int v)
+// a DPP move within a row of 16 lanes, 0 where it reads past the row
+template <int CTRL>
+__device__ __forceinline__ double row_move(double x)
 {
-    if constexpr (S == 1) return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false);  // quad [1,0,3,2]
-    if constexpr (S == 2) return __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false);  // quad [2,3,0,1]
-    constexpr int lower = S == 4 ? 0x5 : 0x3;  // banks of 4 lanes that read upwards
-    const int up = __builtin_amdgcn_update_dpp(0, v, kDppRowShr + S, 0xF, 0xF, false);
-    return __builtin_amdgcn_update_dpp(up, v, kDppRowShl + S, 0xF, lower, false);
+    return by_word(x, [](int v) { return __builtin_amdgcn_mov_dpp(v, CTRL, 0xF, 0xF, true); });
 }
 
+// x of lane i ^ S, S = 4 or 8 (within a row of 16 lanes): a shift either way,
+// the second written to its own half only
 template <int S>
-__device__ __forceinline__ double lane_swap(double x, int lane4)
+__device__ __forceinline__ double row_swap(double x)
 {
-    if constexpr (S <= 8) {
-        const long long v = __double_as_longlong(x);
-        const int lo = lane_swap_word<S>((int)(v & 0xffffffffll)), hi = lane_swap_word<S>((int)(v >> 32));
-        return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+    static_assert(S == 4 || S == 8, "halves of 8 or 16 lanes");
+    return by_word(x, [](int v) {
+        const int up = __builtin_amdgcn_mov_dpp(v, kDppRowShr + S, 0xF, 0xF, true);
+        // the banks of 4 lanes that read upwards
+        return __builtin_amdgcn_update_dpp(up, v, kDppRowShl + S, 0xF, S == 4 ? 0x5 : 0x3, false);
+    });
+}
+
+// x of lane i ^ S, S = 16 or 32: the halves of the pair of rows (or of the
+// wavefront) change places
+template <int S>
+__device__ __forceinline__ void half_pair(int v, int &even, int &odd)
+{
+    if constexpr (S == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+        even = (int)r[0];
+        odd = (int)r[1];
     } else {
-        return crossbar(x, lane4 ^ (4 * S));
+        const auto r = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+        even = (int)r[0];
+        odd = (int)r[1];
     }
 }
 

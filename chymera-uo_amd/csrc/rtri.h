@@ -1,7 +1,7 @@
 // The r-tridiagonal solves of the mode systems on a group of G lanes of a
 // wavefront (64/G systems per wavefront), two right-hand sides per system.
 //
-// Lane gl of a group owns rows [R gl, R gl + R).  Rows 0..R-2 are eliminated
+// The lane at position p of a group owns rows [R p, R p + R).  Rows 0..R-2 are eliminated
 // inside the lane from both ends towards the middle row (two independent
 // chains of R/2 - 1 reciprocals instead of one of R - 1), with the two
 // neighbouring interface unknowns kept symbolic; the interface rows R-1 of the
@@ -34,31 +34,86 @@ __device__ __forceinline__ double rcp_full(double x)
     return __builtin_fma(r, __builtin_fma(e, e, e), r);
 }
 
-// x of lane i - S / i + S of a group of G lanes (any finite value past the
-// group's edges): DPP moves where the group lies in a row of 16 lanes, the
-// LDS crossbar otherwise; distance 1 by DPP for every group
-template <int S, int G>
-__device__ __forceinline__ double lane_lo(double x, int lane4)
+// Where the lanes of a group stand along r.  Up to 16 lanes: in lane order,
+// inside one row of 16 lanes.  32 and 64 lanes: row b of a group's 2 or 4
+// rows holds the positions b modulo the number of rows, so that after one or
+// two reduction steps the rows are independent systems and every later step
+// is a DPP move within a row (no LDS crossbar: at 32 lanes its 54 accesses
+// per solve kept the wavefronts waiting 40% of the time).
+template <int G>
+struct Group {
+    static constexpr int ROWS = G <= 16 ? 1 : G / 16;
+    static __device__ __forceinline__ int pos(int gl) { return ROWS == 1 ? gl : ROWS * (gl & 15) + (gl >> 4); }
+    static __device__ __forceinline__ int lane(int p) { return ROWS == 1 ? p : (p % ROWS) * 16 + p / ROWS; }
+};
+
+// Values of the positions p - 1 (lo) and p + 1 (hi) of a group; any finite
+// value past its ends.  at: the crossbar addresses of both (64 lanes).
+struct Neigh {
+    int lo, hi;
+};
+
+template <int G>
+__device__ __forceinline__ Neigh neighbours(int lane)
 {
-    if constexpr (S == 1) {
-        return lane_prev(x);
-    } else if constexpr (G <= 16) {
-        return dpp_move<kDppRowShr + S>(x);
+    if constexpr (G < 64) {
+        return Neigh{0, 0};
     } else {
-        return crossbar(x, lane4 - 4 * S);
+        const int p = Group<64>::pos(lane);
+        return Neigh{4 * Group<64>::lane((p + 63) & 63), 4 * Group<64>::lane((p + 1) & 63)};
     }
 }
 
-template <int S, int G>
-__device__ __forceinline__ double lane_hi(double x, int lane4)
+// Even and odd halves S lanes apart, position p of the even half between
+// p - 1 and p of the odd one: each half's neighbours lie in the other, one of
+// them at the same lane of the row.
+template <int S>
+__device__ __forceinline__ int half_lo(int v)
 {
-    if constexpr (S == 1) {
-        return lane_next(x);
-    } else if constexpr (G <= 16) {
-        return dpp_move<kDppRowShl + S>(x);
-    } else {
-        return crossbar(x, lane4 + 4 * S);
-    }
+    int e, o;
+    half_pair<S>(v, e, o);
+    return __builtin_amdgcn_update_dpp(e, o, kDppRowShr + 1, S == 16 ? 0x5 : 0x3, 0xF, false);
+}
+
+template <int S>
+__device__ __forceinline__ int half_hi(int v)
+{
+    int e, o;
+    half_pair<S>(v, e, o);
+    return __builtin_amdgcn_update_dpp(o, e, kDppRowShl + 1, S == 16 ? 0xA : 0xC, 0xF, false);
+}
+
+template <int G>
+__device__ __forceinline__ double pos_prev(double x, Neigh at)
+{
+    if constexpr (G <= 16) return row_move<kDppRowShr + 1>(x);
+    else if constexpr (G == 32) return by_word(x, [](int v) { return half_lo<16>(v); });
+    else return by_word(x, [&](int v) { return crossbar_word(v, at.lo); });
+}
+
+template <int G>
+__device__ __forceinline__ double pos_next(double x, Neigh at)
+{
+    if constexpr (G <= 16) return row_move<kDppRowShl + 1>(x);
+    else if constexpr (G == 32) return by_word(x, [](int v) { return half_hi<16>(v); });
+    else return by_word(x, [&](int v) { return crossbar_word(v, at.hi); });
+}
+
+// values S positions down and up
+template <int S, int G>
+__device__ __forceinline__ double step_lo(double x, Neigh at)
+{
+    if constexpr (S == 1) return pos_prev<G>(x, at);
+    else if constexpr (G == 64 && S == 2) return by_word(x, [](int v) { return half_lo<32>(v); });
+    else return row_move<kDppRowShr + S / Group<G>::ROWS>(x);
+}
+
+template <int S, int G>
+__device__ __forceinline__ double step_hi(double x, Neigh at)
+{
+    if constexpr (S == 1) return pos_next<G>(x, at);
+    else if constexpr (G == 64 && S == 2) return by_word(x, [](int v) { return half_hi<32>(v); });
+    else return row_move<kDppRowShl + S / Group<G>::ROWS>(x);
 }
 
 // One row of the interface system, scaled to diagonal 1:
@@ -68,13 +123,13 @@ struct Iface {
 };
 
 template <int S, int G>
-__device__ __forceinline__ void pcr_steps(Iface &r, int lane4)
+__device__ __forceinline__ void pcr_steps(Iface &r, Neigh at)
 {
     if constexpr (2 * S < G) {
-        const double lal = lane_lo<S, G>(r.al, lane4), lga = lane_lo<S, G>(r.ga, lane4);
-        const double ld0 = lane_lo<S, G>(r.d0, lane4), ld1 = lane_lo<S, G>(r.d1, lane4);
-        const double hal = lane_hi<S, G>(r.al, lane4), hga = lane_hi<S, G>(r.ga, lane4);
-        const double hd0 = lane_hi<S, G>(r.d0, lane4), hd1 = lane_hi<S, G>(r.d1, lane4);
+        const double lal = step_lo<S, G>(r.al, at), lga = step_lo<S, G>(r.ga, at);
+        const double ld0 = step_lo<S, G>(r.d0, at), ld1 = step_lo<S, G>(r.d1, at);
+        const double hal = step_hi<S, G>(r.al, at), hga = step_hi<S, G>(r.ga, at);
+        const double hd0 = step_hi<S, G>(r.d0, at), hd1 = step_hi<S, G>(r.d1, at);
         const double be = __builtin_fma(-r.ga, hal, __builtin_fma(-r.al, lga, 1.0));
         const double inv = rcp_full(be);
         const double t0 = __builtin_fma(-r.ga, hd0, __builtin_fma(-r.al, ld0, r.d0));
@@ -83,18 +138,36 @@ __device__ __forceinline__ void pcr_steps(Iface &r, int lane4)
         r.ga = -(r.ga * hga) * inv;
         r.d0 = t0 * inv;
         r.d1 = t1 * inv;
-        pcr_steps<2 * S, G>(r, lane4);
+        pcr_steps<2 * S, G>(r, at);
     }
 }
 
-// (T - rt) x = d in place in d0, d1.  ca, cb, cc: the lane's rows of T (sub,
-// diagonal, super), rows past the system with ca = cc = 0, a large cb and
-// d = 0 (their x is 0); lane4: 4 * lane (byte address in the crossbar).
+// LDS vectors of R*G values: element j = R p + r (position p) at
+// r (G + 2) + lane(p), so that the lanes of a solve read consecutive words and
+// 16 consecutive j (a matrix operand) fall in 16 different 8-byte banks
 template <int R, int G>
-__device__ __forceinline__ void rtri_solve(const double (&ca)[R], const double (&cb)[R], const double (&cc)[R],
-                                           double rt, int lane4, double (&d0)[R], double (&d1)[R])
+struct Vec {
+    static constexpr int PITCH = G + 2, SIZE = R * PITCH;
+    static __device__ __forceinline__ int at(int j) { return (j % R) * PITCH + Group<G>::lane(j / R); }
+};
+
+// (T - rt) x = d in place in d0, d1.  tri: this lane's rows of T in LDS (Vec
+// layout; sub-diagonal, diagonal, super-diagonal one after the other), rows
+// past the system with zero off-diagonals, a large diagonal and d = 0 (their x
+// is 0).  The rows are read here, where they are used, and not kept in
+// registers: 48 registers less at R = 8 let a third wavefront run per SIMD.
+template <int R, int G>
+__device__ __forceinline__ void rtri_solve(const double *tri, double rt, Neigh at, double (&d0)[R], double (&d1)[R])
 {
-    static_assert(G >= 2, "group");
+    static_assert(G >= 8, "group");
+    typedef Vec<R, G> V;
+    double ca[R], cb[R], cc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        ca[r] = tri[r * V::PITCH];
+        cb[r] = tri[V::SIZE + r * V::PITCH];
+        cc[r] = tri[2 * V::SIZE + r * V::PITCH];
+    }
     constexpr int MID = R / 2 - 1, LAST = R - 2;
     // x_i = d_i + P_i XL + Q_i XR for i < R-1 (XL, XR: the last rows of the
     // previous lane and of this one); before the inner substitution Q_i of the
@@ -175,8 +248,8 @@ __device__ __forceinline__ void rtri_solve(const double (&ca)[R], const double (
             P[i] = -P[i] * P[i - 1];
         }
         // interface row: the next lane's first row enters through its D, P, Q
-        const double nP = lane_next(P[0]), nQ = lane_next(Q[0]);
-        const double n0 = lane_next(d0[0]), n1 = lane_next(d1[0]);
+        const double nP = pos_next<G>(P[0], at), nQ = pos_next<G>(Q[0], at);
+        const double n0 = pos_next<G>(d0[0], at), n1 = pos_next<G>(d1[0], at);
         const double a = ca[R - 1], c = cc[R - 1];
         f.al = a * P[LAST];
         be = __builtin_fma(c, nP, __builtin_fma(a, Q[LAST], be));
@@ -191,20 +264,20 @@ __device__ __forceinline__ void rtri_solve(const double (&ca)[R], const double (
         f.d0 = d0[R - 1] * inv;
         f.d1 = d1[R - 1] * inv;
     }
-    pcr_steps<1, G>(f, lane4);
-    // last step: a row's one partner lies G/2 lanes away (al is zero in the
-    // lower half of the group, ga in the upper)
+    pcr_steps<1, G>(f, at);
+    // last step: a row's one partner lies G/2 positions away (al is zero in
+    // the lower half of the group, ga in the upper)
     {
+        constexpr int H = G < 16 ? G / 2 : 8;  // in lanes of a row
         const double c = f.al + f.ga;
-        const double pc = lane_swap<G / 2>(c, lane4), p0 = lane_swap<G / 2>(f.d0, lane4);
-        const double p1 = lane_swap<G / 2>(f.d1, lane4);
+        const double pc = row_swap<H>(c), p0 = row_swap<H>(f.d0), p1 = row_swap<H>(f.d1);
         const double inv = rcp_full(__builtin_fma(-c, pc, 1.0));
         d0[R - 1] = __builtin_fma(-c, p0, f.d0) * inv;
         d1[R - 1] = __builtin_fma(-c, p1, f.d1) * inv;
     }
     if constexpr (R > 1) {
-        // XL: for a group's first lane any finite value (its P is zero)
-        const double xl0 = lane_prev(d0[R - 1]), xl1 = lane_prev(d1[R - 1]);
+        // XL: at a group's first position any finite value (its P is zero)
+        const double xl0 = pos_prev<G>(d0[R - 1], at), xl1 = pos_prev<G>(d1[R - 1], at);
 #pragma unroll
         for (int i = 0; i <= LAST; ++i) {
             d0[i] = __builtin_fma(P[i], xl0, __builtin_fma(Q[i], d0[R - 1], d0[i]));
@@ -213,18 +286,18 @@ __device__ __forceinline__ void rtri_solve(const double (&ca)[R], const double (
     }
 }
 
-// The rows of T_m one lane owns (am, cm, bm of the grid, padded to whole
-// groups), rows >= M made inert.
+// The rows of T_m (am, cm, bm of the grid, padded to R G rows) into LDS for
+// rtri_solve by a block of nt threads, rows >= M made inert.
 constexpr double kInertDiag = 1e150;
-template <int R>
-__device__ __forceinline__ void rtri_rows(const double *am, const double *cm, const double *bm, int f, int M,
-                                          double (&ca)[R], double (&cb)[R], double (&cc)[R])
+template <int R, int G>
+__device__ __forceinline__ void rtri_load(double *tri, const double *am, const double *cm, const double *bm, int M,
+                                          int nt)
 {
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        ca[r] = am[f + r];
-        cc[r] = cm[f + r];
-        cb[r] = f + r < M ? bm[f + r] : kInertDiag;
+    typedef Vec<R, G> V;
+    for (int j = threadIdx.x; j < R * G; j += nt) {
+        tri[V::at(j)] = am[j];
+        tri[V::SIZE + V::at(j)] = j < M ? bm[j] : kInertDiag;
+        tri[2 * V::SIZE + V::at(j)] = cm[j];
     }
 }
 
