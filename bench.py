@@ -558,6 +558,9 @@ def main():
         kind = "refined" if steps else ("cr" if solver == chypot.MODES_CR else "eigen")
         if steps and st.get("planes", (0, 0))[1]:
             kind = "refined_fused"
+        elif steps and st.get("cr", (0, 0))[1]:
+            kind = "cr"  # the refined solve by the plain solve's binary64 mode solves
+        res["mode_solves"] = {"cr": "binary64, cyclic reduction", "eigen": "binary64, z eigenbasis"}.get(kind, "binary32")
         work = stage_work(g, kind, steps)
         res["rooflines"] = rooflines(st, work, B * args.steps, B, args.steps, f"potsolve_{g.name}_{kind}", copy_gbs)
         if n_lat > 0:
@@ -669,7 +672,7 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "f32+f64" if refined is not None else "f64",
+        "dtype": "f32+f64" if head["mode_solves"] == "binary32" else "f64",
         "data": "synthetic",
         "config": {"workload": "refined potential solve (BDYGEN+POT3), batched, spiral-arm torus"
                    if refined is not None else "plain FP64 potential solve (BDYGEN+POT3), batched, spiral-arm torus",

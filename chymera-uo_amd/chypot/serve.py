@@ -19,9 +19,9 @@ a grid shape and a device-resident density; the server
     until the next arrival;
   * records per-request latency from arrival to the host seeing completion.
 
-refine_steps > 0 serves the refined solve (binary32 correction solves on the
-FP32 matrix cores, binary64 residuals) on grids it supports (KMAX <= 256);
-other grids get the plain binary64 solve.  Each request records its path.
+refine_steps > 0 serves the refined solve (within 1e-10 of the plain one, by
+whichever mode solves are the faster on the grid) on grids it supports (KMAX <=
+256); other grids get the plain binary64 solve.  Each request records its path.
 A chypot.autotune table (tune_table) sets the launch shapes of every grid
 the server prepares.
 

@@ -425,8 +425,12 @@ static int run_pot3(chy_grid *g, int npoint, const double *rho, double *phi, dou
     return run_pot3_tail(g, s, npoint, phi, klocat_in, true);
 }
 
-// Buffers of the refined solve, allocated on first use.
-static int ensure_refine(chy_grid *g)
+// True where refined solves on g may run the binary32 mode solves: the
+// one-kernel-per-plane form is on, or the binary64 tree does not take the grid.
+static bool refine_may_use32(const chy_grid *g) { return g->refine_fused > 0 || !cr_supported(g); }
+
+// Buffers of the refined solve's binary32 mode solves, allocated on first use.
+static int ensure_refine(chy_grid *g, bool use32)
 {
     auto get = [&](void **p, size_t bytes) -> int {
         if (*p) return CHY_OK;
@@ -437,6 +441,7 @@ static int ensure_refine(chy_grid *g)
         return CHY_OK;
     };
     if (!refine_supported(g)) return CHY_EUNSUPPORTED;
+    if (!use32) return CHY_OK;
     int rc = get((void **)&g->d.spec32, sizeof(float) * (size_t)g->L * g->K * g->J);
     if (!rc) rc = get((void **)&g->d.yh32, sizeof(float) * (size_t)g->L * g->PP * g->JP);
     if (!rc) rc = get((void **)&g->d.rstat, sizeof(unsigned long long) * 2 * kMaxRefine);
@@ -474,7 +479,13 @@ static int rhs_spectrum_f(chy_grid *g, const Fields &F, hipStream_t s, int maxtr
 }
 
 // Refined solve of every field of F (grids[f] owns field f's workspace; g's
-// tables), by iterative refinement of the mode systems in the azimuthal
+// tables).  Where the binary64 tree takes the grid (cr.hip) and neither the
+// per-step statistics nor the one-kernel form is asked for, the tree solves
+// the mode systems in one pass: it moves a third of the bytes of two
+// binary32 solves and the residual between them, and binary32 r solves run no
+// faster than binary64 ones on this VALU (mode work of 32 fields at
+// 256x128x256: 3.3 against 4.8 ms; of one, 200 against 230 us).  Otherwise by
+// iterative refinement of the mode systems in the azimuthal
 // spectrum, where the 7-point operator is block diagonal by mode:
 //   B = the right-hand side spectrum (binary64, as the plain solve forms it);
 //   X = 0; for each step: R = B - A X (binary64, per mode, rounded to
@@ -509,13 +520,22 @@ static int run_refined_fields(chy_grid *g, const std::vector<chy_grid *> &grids,
     Profiler *p = g->ctx->prof.on ? &g->ctx->prof : nullptr;
     // the fused per-plane kernel where it applies (it collects no per-step
     // statistics: those calls take the kernel-per-stage path)
-    if (F.nf <= g->refine_fused && g->d.fac32 && !with_stats && refine_planes_ok(g, steps)) {
+    bool have32 = true;
+    for (int f = 0; f < F.nf; ++f) have32 = have32 && grids[f]->d.yh32;
+    if (F.nf <= g->refine_fused && g->d.fac32 && have32 && !with_stats && refine_planes_ok(g, steps)) {
         Fields Fp = F;
         for (int f = 0; f < F.nf; ++f) Fp.aux[f] = grids[f]->d.yh32;
         if (p) p->begin(CHY_STAGE_PLANES, s);
         if (!rc) rc = dev_rc(launch_refine_planes_f(g, Fp, steps, g->refine_m64, s), "refined mode planes launch");
         if (p) p->end(s);
         steps = 0;  // the mode work is done
+    } else if (!with_stats && cr_supported(g)) {
+        if (p) p->begin(CHY_STAGE_CR, s);
+        if (!rc) rc = dev_rc(launch_cr_solve_f(g, F, s), "mode solve launch");
+        if (p) p->end(s);
+        steps = 0;
+    } else if (!have32) {
+        return CHY_ESTATE;  // not reached: the callers allocate the buffers where this path may run
     }
     // two steps: the first iterate, a binary32 value, is kept in binary32
     const bool x32 = steps == 2;
@@ -548,7 +568,7 @@ static int run_refined(chy_grid *g, hipStream_t s, int maxtrm, int isym, double 
                        const double *rho, double *phi, double *coef, int coef_mode, int steps, int klocat_in,
                        bool with_stats)
 {
-    int rc = ensure_refine(g);
+    int rc = ensure_refine(g, with_stats || refine_may_use32(g));
     if (rc) return rc;
     const Fields F = one_field(g, rho, phi, coef, klocat_in);
     return run_refined_fields(g, std::vector<chy_grid *>{g}, F, s, maxtrm, isym, redge, npoint, coef_mode, steps,
@@ -939,7 +959,9 @@ static int solve_batch(chy_ctx *ctx, const chy_solve_item *items, int n, int ste
     DeviceScope ds(ctx->device);
     int rc = ensure_workers(ctx);
     if (rc) return rc;
-    for (int i = 0; i < n && steps > 0 && rc == CHY_OK; ++i) rc = ensure_refine(items[i].grid);
+    bool use32 = false;
+    for (int i = 0; i < n; ++i) use32 = use32 || refine_may_use32(items[i].grid);
+    for (int i = 0; i < n && steps > 0 && rc == CHY_OK; ++i) rc = ensure_refine(items[i].grid, use32);
     if (rc) return rc;
     if (any_diag && ctx->diag_cap < n) {
         drop_graphs_of(ctx->batch_graphs, kBatchKeyHead, kBatchKeyPerItem, nullptr);  // they copy into the old staging

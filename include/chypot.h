@@ -108,8 +108,9 @@ size_t chy_grid_device_bytes(const chy_grid *g);
 /* How POT3's per-mode 2-D solves (pot/pot3.f:233-239) are done on a grid.
  *   CHY_MODES_CR    (default) BLKTRI's generalised cyclic reduction
  *                   (pot/blktri.f:60-260) with BLKTRI's own root tables
- *                   (COMPB/TQLRAT, pot/blktri.f:264-423, the same arithmetic):
- *                   the reference's results to rounding (2.2e-13 relative at
+ *                   (COMPB/TQLRAT, pot/blktri.f:264-423, the same arithmetic),
+ *                   its products as sums of independent solves: the
+ *                   reference's results to rounding (2.2e-13 relative at
  *                   256x128x256).
  *   CHY_MODES_EIGEN the m-independent z operator diagonalised once per grid
  *                   (80-bit arithmetic) and r-tridiagonal solves per z
@@ -125,20 +126,18 @@ int chy_grid_set_mode_solver(chy_grid *g, int kind);
 int chy_grid_mode_solver(const chy_grid *g);
 
 /* Kernel shapes and precision split of a grid (no reference counterpart).
- *   CHY_TUNE_CR_LANES    lanes per r system in the cyclic reduction: 64 (one
- *                        order per wavefront) or 32 (two orders per
- *                        wavefront, JMAX-1 <= 256)
- *   CHY_TUNE_REFINE_M64  refined solves: the r solves of orders m <= this
- *                        value run in binary64, the others in binary32
- *                        (-1..LMAX/2; default 4)
+ *   CHY_TUNE_CR_LANES    r systems of the cyclic reduction per wavefront: 64
+ *                        (64 lanes, one system) or 32 (8 rows per lane, so 8
+ *                        to 32 lanes, up to 8 systems; JMAX-1 <= 256)
+ *   CHY_TUNE_REFINE_M64  refined solves in binary32: the r solves of orders
+ *                        m <= this value run in binary64 (-1..LMAX/2;
+ *                        default 4)
  *   CHY_TUNE_REFINE_FUSED refined solves of 1 or 2 steps launched for at
  *                        most this many fields (0..32; default 0) run all
  *                        mode work of a mode plane in one kernel with the
  *                        binary32 plane in LDS, where it fits (KMAX <= 129,
- *                        JMAX <= 257): a third of the HBM traffic, but one
- *                        block per CU runs its phases one after another, so
- *                        it wins for few fields per launch and loses for
- *                        many; larger launches run one kernel per stage
+ *                        JMAX <= 257) instead of the mode solves that
+ *                        chy_solve_refined otherwise uses
  * Results do not depend on the shapes beyond rounding.  Changing a value
  * drops the grid's captured solve graphs.  CHY_EINVAL for a value the grid
  * cannot take. */
@@ -224,19 +223,25 @@ int chy_pot3_host(chy_grid *g, int npoint, const double *rho_h, double *phi_h, d
 
 /* ---- refined solve (no reference counterpart) ----
  * The same results as chy_solve (PHI, COEF, diagnostics) to a stated
- * accuracy, by iterative refinement of the mode systems in the azimuthal
- * spectrum: BDYGEN, COEF and the forward transform in binary64 as chy_solve
- * computes them; then `steps` (1..8) mode solves in binary32 (z transforms
- * on the FP32 matrix cores, r solves in binary32 except the orders
- * m <= CHY_TUNE_REFINE_M64, which are solved in binary64), the first of the
- * right-hand side, each later one of the binary64 residual of the mode
- * systems (pot/pot3.f:203-231) at the binary64 solution so far, rounded to
- * binary32, its solution added in binary64; then the inverse transform,
- * POT3's ghost cells and ZAXPHI as in chy_solve.  Two steps put PHI within
- * ~1e-11 of chy_solve's at 256x128x256.  KMAX <= 256 (CHY_EUNSUPPORTED
- * otherwise).  rel_corr (host, may be NULL) receives, per step, the largest
- * correction relative to the largest |solution| after it (1 for the first
- * step).  Waits when diag or rel_corr is non-NULL. */
+ * accuracy: within 1e-10 of chy_solve's for 2 or more steps.  BDYGEN, COEF,
+ * both transforms, POT3's ghost cells and ZAXPHI in binary64 as chy_solve
+ * computes them; the mode systems in one of two ways:
+ *   - JMAX-1 <= 512, rel_corr NULL and no one-kernel form in force
+ *     (CHY_TUNE_REFINE_FUSED): by CHY_MODES_CR's binary64 solves, which are
+ *     the faster way there and give chy_solve's own results whatever `steps`
+ *     is;
+ *   - otherwise by iterative refinement in the azimuthal spectrum: `steps`
+ *     (1..8) mode solves in binary32 (z transforms on the FP32 matrix cores,
+ *     r solves in binary32 except the orders m <= CHY_TUNE_REFINE_M64, which
+ *     are solved in binary64), the first of the right-hand side, each later
+ *     one of the binary64 residual of the mode systems (pot/pot3.f:203-231) at
+ *     the binary64 solution so far, rounded to binary32, its solution added
+ *     in binary64.  One step puts PHI within ~1e-6 of chy_solve's, two within
+ *     ~1e-11 at 256x128x256.
+ * KMAX <= 256 (CHY_EUNSUPPORTED otherwise).  rel_corr (host, may be NULL)
+ * receives, per step, the largest correction relative to the largest
+ * |solution| after it (1 for the first step).  Waits when diag or rel_corr is
+ * non-NULL. */
 int chy_solve_refined(chy_grid *g, int maxtrm, int isym, double redge, int npoint, const double *rho_d,
                       double *phi_d, double *coef_d, int coef_mode, int steps, chy_diag *diag,
                       double *rel_corr);

@@ -49,3 +49,55 @@ def test_tree_against_oracle(jkl, lanes):
     finally:
         po.use_cyclic_reduction(False)
     assert rel_max(phi, want["phi"]) < 1e-12
+
+
+@pytest.mark.parametrize("jkl", [(5, 4, 4), (64, 32, 24), (130, 64, 40), (257, 16, 32), (300, 8, 24)])
+def test_refined_by_the_tree(jkl):
+    """A refined solve that reports no corrections takes the plain solve's mode
+    solves: bit for bit chy_solve's PHI, one step or two, LMAX/2 below and
+    above MAXTRM (boundary values through PHI or in the spectrum); one that
+    reports them still refines in binary32, within 1e-10."""
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    g = fields.unit_grid(*jkl)
+    print(f"[gpu] refined by the tree {g.name}", flush=True)
+    ctx = chypot.Context(0)
+    pg = chypot.PreparedGrid(ctx, g)
+    rho = chypot.to_device(fields.density_spiral_torus(g, seed=8))
+    plain = torch.zeros_like(rho)
+    pg.solve(rho, plain, npoint=4)
+    for steps in (1, 2):
+        phi = torch.zeros_like(rho)
+        pg.solve_refined(rho, phi, steps=steps, npoint=4)
+        ctx.sync()
+        assert torch.equal(phi, plain)
+    phi = torch.zeros_like(rho)
+    _, rel = pg.solve_refined(rho, phi, steps=2, npoint=4, report=True)
+    assert 0.0 < rel[1] < 1e-5
+    assert float((phi - plain).abs().max()) < 1e-10 * float(plain.abs().max())
+    pg.close()
+
+
+def test_refined_group_of_unlike_tunings():
+    """Fields of one group on grid objects with and without the one-kernel form
+    (whose buffers only some objects would have asked for by themselves)."""
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    g = fields.unit_grid(64, 32, 64)
+    print("[gpu] refined group of unlike tunings", flush=True)
+    ctx = chypot.Context(0)
+    for first in (0, 1):
+        jobs = []
+        for i in range(3):
+            pg = chypot.PreparedGrid(ctx, g)
+            pg.refine_fused = 32 if i == first else 0
+            rho = chypot.to_device(fields.density_spiral_torus(g, seed=20 + i))
+            jobs.append(dict(grid=pg, rho=rho, phi=torch.zeros_like(rho)))
+        ctx.solve_batch(jobs, refine_steps=2)
+        ctx.sync()
+        for j in jobs:
+            plain = torch.zeros_like(j["rho"])
+            j["grid"].solve(j["rho"], plain)
+            ctx.sync()
+            assert float((j["phi"] - plain).abs().max()) < 1e-10 * float(plain.abs().max())
+            j["grid"].close()
