@@ -108,19 +108,22 @@ __device__ __forceinline__ double zax_phac(const double (&ph)[PPT], int l0, int 
 // PHICHK/KLOCAT (pot3.f:391-399) by the last of `nblocks` blocks to finish:
 // each block has stored its PHAC(K) in dscal[4+K]; the one that takes the
 // last ticket reduces them (largest |PHAC|, first K wins; KLOCAT unchanged
-// when every PHAC is 0) and resets the ticket for the next launch.
+// when every PHAC is 0) and resets the ticket for the next launch.  The one
+// value that crosses blocks is stored and loaded with device scope (past the
+// XCDs' L2 caches) and waited for before the ticket, so no fence is needed: a
+// __threadfence writes back the whole L2, and one per block took most of
+// ZAXPHI's time (32 fields at 256x128x256: 205 us).
 __device__ inline void zax_finish(double *dscal, int K_phac, double phac, unsigned *ticket, unsigned nblocks,
                                   int kmax, int klocat_in, double *sv, int *si)
 {
     __shared__ bool last;
     if (threadIdx.x == 0) {
-        dscal[4 + K_phac] = phac;
-        __threadfence();
-        last = atomicAdd(ticket, 1u) == nblocks - 1;
+        __hip_atomic_store(&dscal[4 + K_phac], phac, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nblocks - 1;
     }
     __syncthreads();
     if (!last) return;
-    __threadfence();
     double best2 = 0.0;
     int bk = 0x7fffffff;
     for (int kk = 2 + (int)threadIdx.x; kk <= kmax + 1; kk += blockDim.x) {
