@@ -693,7 +693,6 @@ int chy_ctx_destroy(chy_ctx *ctx)
     if (ctx->h_diag) (void)hipHostFree(ctx->h_diag);
     for (const chy_ctx::TrigTable &t : ctx->trig) (void)hipFree(t.d);
     if (ctx->force_part) (void)hipFree(ctx->force_part);
-    if (ctx->force_out) (void)hipFree(ctx->force_out);
     if (ctx->force_h) (void)hipHostFree(ctx->force_h);
     if (ctx->own) (void)hipStreamDestroy(ctx->own);
     delete ctx;
@@ -1342,20 +1341,11 @@ int chy_find_force(chy_ctx *ctx, const chy_force_desc *d, const double *rhf_d, c
         if (hipMalloc(&ctx->force_part, sizeof(double) * 2 * (size_t)nb) != hipSuccess) return CHY_ENOMEM;
         ctx->force_cap = nb;
     }
-    if (!ctx->force_out) {
-        if (hipMalloc(&ctx->force_out, sizeof(double) * 2) != hipSuccess) return CHY_ENOMEM;
-        if (hipHostMalloc(&ctx->force_h, sizeof(double) * 2) != hipSuccess) {
-            (void)hipFree(ctx->force_out);
-            ctx->force_out = nullptr;
-            return CHY_ENOMEM;
-        }
-    }
+    // the total is written straight into pinned host memory
+    if (!ctx->force_h && hipHostMalloc(&ctx->force_h, sizeof(double) * 2) != hipSuccess) return CHY_ENOMEM;
     hipStream_t s = ctx->stream;
-    rc = dev_rc(launch_find_force(d, rhf_d, zhf_d, cs, rho_d, x, y, ctx->force_part, ctx->force_out, s),
+    rc = dev_rc(launch_find_force(d, rhf_d, zhf_d, cs, rho_d, x, y, ctx->force_part, ctx->force_h, s),
                 "find_force launch");
-    if (!rc)
-        rc = dev_rc((int)hipMemcpyAsync(ctx->force_h, ctx->force_out, 2 * sizeof(double), hipMemcpyDeviceToHost, s),
-                    "force readback");
     if (!rc) rc = dev_rc((int)hipStreamSynchronize(s), "hipStreamSynchronize");
     if (!rc) {
         f_h[0] = ctx->force_h[0];

@@ -184,8 +184,8 @@ struct chy_ctx {
         double *d;
     };
     std::vector<TrigTable> trig;
-    // chy_find_force: block partials and the (fx, fy) result
-    double *force_part = nullptr, *force_out = nullptr, *force_h = nullptr;
+    // chy_find_force: block partials and the (fx, fy) result (pinned host memory)
+    double *force_part = nullptr, *force_h = nullptr;
     int force_cap = 0;
     // chy_find_force_noalloc: the device's fixed scratch (force.hip)
     double *force_scratch = nullptr;
