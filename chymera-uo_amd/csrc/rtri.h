@@ -122,9 +122,27 @@ struct Iface {
     double al, ga, d0, d1;
 };
 
-template <int S, int G>
-__device__ __forceinline__ void pcr_steps(Iface &r, Neigh at)
+// False when no row of the wavefront is coupled to another any more: a row's
+// couplings (relative to its diagonal) square with every step, and below
+// kUncoupled a partner changes nothing within binary64.  The larger a system's
+// root, the sooner: on a grid alike in r and z the roots of a column need 2.9
+// of the 5 steps of 32 lanes on average.
+constexpr double kUncoupled = 1e-20;
+__device__ __forceinline__ bool coupled(const Iface &r)
 {
+    return __any(fmax(fabs(r.al), fabs(r.ga)) > kUncoupled);
+}
+
+// The steps of distance S, 2S, .. < G/2; false once uncoupled.  A right-hand
+// side with an infinity or NaN takes every step (all: found at the first
+// check), so that it reaches every row of its system as the reference's
+// sweeps carry it.
+template <int S, int G>
+__device__ __forceinline__ bool pcr_steps(Iface &r, Neigh at, bool all = false)
+{
+    if constexpr (S == 4) all = __any(!__builtin_isfinite(fabs(r.d0) + fabs(r.d1)));
+    if constexpr (S >= 4)
+        if (!all && !coupled(r)) return false;
     if constexpr (2 * S < G) {
         const double lal = step_lo<S, G>(r.al, at), lga = step_lo<S, G>(r.ga, at);
         const double ld0 = step_lo<S, G>(r.d0, at), ld1 = step_lo<S, G>(r.d1, at);
@@ -138,8 +156,9 @@ __device__ __forceinline__ void pcr_steps(Iface &r, Neigh at)
         r.ga = -(r.ga * hga) * inv;
         r.d0 = t0 * inv;
         r.d1 = t1 * inv;
-        pcr_steps<2 * S, G>(r, at);
+        return pcr_steps<2 * S, G>(r, at, all);
     }
+    return true;
 }
 
 // LDS vectors of R*G values: element j = R p + r (position p) at
@@ -264,10 +283,12 @@ __device__ __forceinline__ void rtri_solve(const double *tri, double rt, Neigh a
         f.d0 = d0[R - 1] * inv;
         f.d1 = d1[R - 1] * inv;
     }
-    pcr_steps<1, G>(f, at);
-    // last step: a row's one partner lies G/2 positions away (al is zero in
-    // the lower half of the group, ga in the upper)
-    {
+    const bool more = pcr_steps<1, G>(f, at);
+    d0[R - 1] = f.d0;
+    d1[R - 1] = f.d1;
+    if (more) {
+        // last step: a row's one partner lies G/2 positions away (al is zero
+        // in the lower half of the group, ga in the upper)
         constexpr int H = G < 16 ? G / 2 : 8;  // in lanes of a row
         const double c = f.al + f.ga;
         const double pc = row_swap<H>(c), p0 = row_swap<H>(f.d0), p1 = row_swap<H>(f.d1);

@@ -101,3 +101,30 @@ def test_refined_group_of_unlike_tunings():
             ctx.sync()
             assert float((j["phi"] - plain).abs().max()) < 1e-10 * float(plain.abs().max())
             j["grid"].close()
+
+
+@pytest.mark.parametrize("lanes", [64, 32])
+@pytest.mark.parametrize("jkl", [(64, 32, 8), (250, 8, 6), (257, 16, 4), (513, 4, 4)])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_tree_spreads_what_is_not_finite(jkl, lanes, bad):
+    """One density value that is not finite leaves no finite PHI, as it does
+    through the reference's sweeps, also on flat grids, where the reduction
+    along r ends early for finite right-hand sides."""
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    if lanes == 32 and jkl[0] - 1 > 256:
+        pytest.skip("64 lanes only")
+    g = fields.unit_grid(*jkl)
+    print(f"[gpu] tree not finite {g.name} lanes {lanes}", flush=True)
+    ctx = chypot.Context(0)
+    pg = chypot.PreparedGrid(ctx, g)
+    pg.cr_lanes = lanes
+    rho = chypot.to_device(fields.density_spiral_torus(g, seed=6))
+    phi = torch.zeros_like(rho)
+    pg.solve(rho, phi, npoint=4)
+    rho[0, 1, g.jmax // 2] = bad
+    pg.pot3(rho, phi, npoint=4)
+    ctx.sync()
+    inner = phi[:, 1:g.kmax, 1:g.jmax]
+    assert not bool(torch.isfinite(inner).any())
+    pg.close()
