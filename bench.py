@@ -71,14 +71,22 @@ def cr_solves_per_mode(n):
     """r solves of the cyclic reduction of one mode with n = 2^k - 1 z rows as
     the GPU runs it: leaves of 2^l - 1 rows (l = 4, or k - 1 where that is
     less), each root solved once up and once down the tree, and every row at an
-    odd multiple of h >= 2^l with the 2h - 1 roots of its block, up (below the
-    top level) and down."""
+    odd multiple of h = 2^j >= 2^l with its block's roots, up (below the top
+    level) and down.  A block of 2h - 1 >= 31 rows has about 16 + 6.3 (j - 4)
+    of them on a uniform grid, the first of a level 6 more, the top one
+    15 + 3 (j - 4)."""
     kx = int(round(np.log2(n + 1)))
     l0 = min(kx - 1, 4)
     tot = 2 * ((n + 1) >> l0) * ((1 << l0) - 1)
     for lv in range(l0, kx):
         h = 1 << lv
-        tot += (n + 1) // (2 * h) * (2 * h - 1) * (2 if lv < kx - 1 else 1)
+        nodes = (n + 1) // (2 * h)
+        if lv < 4:
+            tot += nodes * (2 * h - 1) * (2 if lv < kx - 1 else 1)
+        elif lv < kx - 1:
+            tot += 2 * int(nodes * (16 + 6.3 * (lv - 4)) + 6)
+        else:
+            tot += 15 + 3 * (lv - 4)
     return tot
 
 

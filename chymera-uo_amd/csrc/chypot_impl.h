@@ -50,7 +50,7 @@ const Term *terms_table(int *count);  // the kMaxTerms terms, l-major, m ascendi
 // leaves' solutions.
 enum { CR_LEAF_UP = 0, CR_NODE_UP = 1, CR_NODE_DOWN = 2, CR_LEAF_DOWN = 3 };
 struct CrPhase {
-    int kind, h, nnode, rec0;  // nodes: their level's h, their number, the level's first root record
+    int kind, h, nnode, rec0, np;  // nodes: their level's h, their number, the level's first record, root records per node
 };
 // a leaf's table in doubles, LS = kLeafSpan rows and roots: U[LS][LS+4] (root p,
 // row k; k = LS, LS + 1: the separators' part of the right-hand side),
@@ -61,12 +61,11 @@ constexpr int kLeafSpan = 16;
 constexpr int kLeafU = 0, kLeafV = kLeafSpan * (kLeafSpan + 4), kLeafRoot = kLeafV + kLeafSpan * kLeafSpan,
               kLeafRight = kLeafRoot + kLeafSpan, kLeafLeft = kLeafRight + kLeafSpan,
               kLeafStride = kLeafLeft + kLeafSpan;
-// a node's record per root (node_roots(h) of them, past the block's 2h - 1
-// the last root with zero weights): root,
-// weight of the message to the right and to the left, weights of the node's
-// right-hand side, the left and the right solved row
-constexpr int kNodeRec = 8;
-__host__ __device__ constexpr int node_roots(int h) { return h < 4 ? 8 : 2 * h; }
+// a node's records: the first holds the number of its roots, then one per root
+// (the last root with zero weights up to the level's np, a multiple of
+// kNodePad): root, weight of the message to the right and to the left, weights
+// of the node's right-hand side, the left and the right solved row
+constexpr int kNodeRec = 8, kNodePad = 8;
 struct CrPlan {
     int kx = 0;
     int rows = 0, nleaf = 0;

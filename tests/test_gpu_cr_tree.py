@@ -21,8 +21,13 @@ SHAPES = [(5, 4, 4), (9, 8, 6), (65, 16, 4), (64, 32, 8), (66, 64, 4), (128, 4, 
           (257, 16, 4), (250, 64, 6), (256, 4, 4), (258, 8, 4), (513, 32, 4), (400, 16, 6)]
 
 
+# columns of up to 511 rows (nodes with far fewer roots than rows), cells up to
+# 16 times flatter than wide and the reverse
+TALL = [(17, 512, 4), (33, 256, 6), (65, 512, 4), (200, 128, 8), (513, 128, 4)]
+
+
 @pytest.mark.parametrize("lanes", [64, 32])
-@pytest.mark.parametrize("jkl", SHAPES)
+@pytest.mark.parametrize("jkl", SHAPES + TALL)
 def test_tree_against_oracle(jkl, lanes):
     import pyoracle as po
     if not torch.cuda.is_available():
