@@ -114,9 +114,11 @@ __device__ __forceinline__ void block_sums(const double (&s)[NSUM][2][R], double
 // V_MFMA_F64_16X16X4F64: A lane l holds A[l%16][l/16], B lane l B[l/16][l%16],
 // the result D[l/16 + 4v][l%16].
 //
-// A block takes `run` leaves of one order one after the other.  It is bound by
-// HBM (up: the spectrum read once, down: read and written), while its solves
-// keep the VALU busy for about half as long, so the next leaf's rows are
+// A block takes `run` leaves (one or two) of one order one after the other.  It
+// is bound by HBM (up: the spectrum read once, down: read and written: 0.63 and
+// 0.99 ms per 32 fields at 256x128x256, 0.44 and 0.87 at the rate of a copy),
+// while its solves keep the VALU busy for about half as long, so the next
+// leaf's rows are
 // loaded into registers (a matrix operand each) before the current one is
 // solved.  Loads and stores of a wavefront complete in order: nothing the
 // solves need is loaded after those rows (the roots and weights wait in LDS),
@@ -125,7 +127,7 @@ __device__ __forceinline__ void block_sums(const double (&s)[NSUM][2][R], double
 // wavefronts per CU), 148 KB at 512 (one of 8).  (Leaves of 31 rows need 146 KB
 // at JMAX <= 256 and twice the matrix products per row: one block per CU, its
 // phases one after another, 1.45 ms down and 1.2 ms up per 32 fields at
-// 256x128x256 against 1.0 and 1.0, more than the saved level of nodes gives.)
+// 256x128x256, more than the saved level of nodes gives.)
 template <int R, int G, int W, bool DOWN>
 __global__ __launch_bounds__(64 * W, 2) void k_cr_leaf(CrArgs a, const Fields F, int run)
 {
@@ -369,19 +371,18 @@ void launch_node(const CrPhase &ph, const CrArgs &a, const Fields &F, hipStream_
 template <int R, int G>
 void launch_leaf(const CrPhase &ph, const chy_grid *g, const CrArgs &a, const Fields &F, hipStream_t s)
 {
-    // wavefronts: two rounds of 64/G roots each, at most 8
-    constexpr int rounds = kLeafSpan * G / 64, W = rounds >= 16 ? 8 : rounds / 2;
-    // leaves per block: the fewest rounds of blocks over the CUs, each a run
-    // and the exposed first load (about half a leaf's time)
+    // wavefronts: all roots in one round of 64/G each for short r systems (at
+    // JMAX 64 one round 4.7 + 6.4 us, two rounds 5.8 + 8.8), two rounds at 32 and
+    // 64 lanes (twice the wavefronts at 32: 1.08 instead of 1.00 ms down per 32
+    // fields at 256x128x256, and no faster alone)
+    constexpr int rounds = kLeafSpan * G / 64, W = rounds >= 16 ? 8 : rounds >= 8 ? rounds / 2 : rounds;
+    // leaves per block: two hide a part of each other's loads once the chip has
+    // its blocks eight times over (8 fields at 256x128x256 279 + 185 us, one leaf
+    // 285 + 188, four 293 + 192); below that more blocks are better (one field
+    // 40 + 30 us with one, 43 + 33 with two, 49 + 38 with four)
     constexpr int lds = (2 * kLeafSpan + 3) * Vec<R, G>::SIZE * 8;
     const long slots = (long)g->ncu * std::max(1, std::min(160 * 1024 / lds, 8 / W));
-    auto cost = [&](int run) {
-        const long blocks = (long)(g->N + 1) * ((a.nleaf + run - 1) / run) * F.nf;
-        return (blocks + slots - 1) / slots * (2 * run + 1);
-    };
-    int run = 1;
-    for (int r = 2; r <= a.nleaf; r *= 2)
-        if (cost(r) <= cost(run)) run = r;
+    const int run = (long)(g->N + 1) * a.nleaf * F.nf >= 8 * slots ? 2 : 1;
     const dim3 grid((unsigned)((g->N + 1) * ((a.nleaf + run - 1) / run)), F.nf);
     if (ph.kind == CR_LEAF_UP)
         hipLaunchKernelGGL((k_cr_leaf<R, G, W, false>), grid, dim3(64 * W), 0, s, a, F, run);
