@@ -138,20 +138,20 @@ struct FftArgs {
 };
 
 // lane index -> (j,k), j = J-2 (0..JMAX-1), k = K-2 (0..KMAX-1)
-__device__ __forceinline__ void lane_jk(const FftArgs &a, long lg, int &j, int &k)
+__device__ __forceinline__ void lane_jk(const FftArgs &a, int lg, int &j, int &k)
 {
     if (a.lanes == LANES_ALL) {
-        j = (int)(lg % a.J);
-        k = (int)(lg / a.J);
+        k = (int)((unsigned)lg / (unsigned)a.J);
+        j = lg - k * a.J;
     } else if (a.lanes == LANES_INTERIOR) {
-        j = (int)(lg % (a.J - 1));
-        k = (int)(lg / (a.J - 1));
+        k = (int)((unsigned)lg / (unsigned)(a.J - 1));
+        j = lg - k * (a.J - 1);
     } else if (lg < a.J) {  // top row K=KMAX+1, J=2..JMAX+1
-        j = (int)lg;
+        j = lg;
         k = a.K - 1;
     } else {                // outer column J=JMAX+1, K=2..KMAX
         j = a.J - 1;
-        k = (int)(lg - a.J);
+        k = lg - a.J;
     }
 }
 
@@ -178,9 +178,9 @@ __device__ __forceinline__ void forward_outputs(const FftArgs &a, const double2 
                                                 size_t base, size_t plane)
 {
     // A_m = 2 Re X_m, B_m = 2 Im X_m
-    auto xm = [&](int m) -> double2 {
-        double2 zm = lds[(m % N) * NL + lane];
-        double2 zc = lds[((N - m) % N) * NL + lane];
+    auto xm = [&](int m) -> double2 {  // m = 0..N
+        double2 zm = lds[(m == N ? 0 : m) * NL + lane];
+        double2 zc = lds[(m == 0 ? 0 : N - m) * NL + lane];
         zc.y = -zc.y;
         double2 e = make_double2(0.5 * (zm.x + zc.x), 0.5 * (zm.y + zc.y));
         double2 d = csub(zm, zc);
@@ -195,7 +195,7 @@ __device__ __forceinline__ void forward_outputs(const FftArgs &a, const double2 
         const int ir = j + (a.J - 1) * k;
         const double dv = a.dv[ir];
         for (int mm = sub; mm <= kMaxTrm; mm += NS) {
-            const int r = mm % a.L;
+            const int r = mm < a.L ? mm : mm % a.L;
             double2 X = r <= N ? xm(r) : xm(a.L - r);
             if (r > N) X.y = -X.y;
             const double2 w = a.twh[mm];
@@ -216,12 +216,15 @@ __device__ __forceinline__ void forward_outputs(const FftArgs &a, const double2 
     const double ys = interior ? a.ys : 1.0;
     double A0 = 0.0;
     if (want_coef) A0 = 2.0 * xm(0).x;
+    TS *sp = spec ? spec + sidx + (size_t)sub * JK : nullptr;
+    const size_t step = JK * (size_t)NS, half = JK * (size_t)N;
     for (int m = sub; m <= N; m += NS) {
         const double2 X = xm(m);
         const double A = 2.0 * X.x, B = 2.0 * X.y;
-        if (spec) {
-            spec[(size_t)m * JK + sidx] = (TS)(A * a.sf1 * ys);
-            if (m >= 1 && m <= N - 1) spec[(size_t)(N + m) * JK + sidx] = (TS)(B * a.sf1 * ys);
+        if (sp) {
+            sp[0] = (TS)(A * a.sf1 * ys);
+            if (m >= 1 && m <= N - 1) sp[half] = (TS)(B * a.sf1 * ys);
+            sp += step;
         }
         if (want_coef && m >= 1) {
             // COEF(J,K,m,1) amplitude, COEF(J,K,m,2) phase (pot3.f:105-132)
@@ -317,7 +320,7 @@ __global__ __launch_bounds__(NL *N2) void k_fft_forward(FftArgs a, const Fields 
     const int sub = tid / NL;
     const int chunk = xcd_chunk((a.nlanes + NL - 1) / NL);
     if (chunk * NL >= a.nlanes) return;  // whole block
-    const long lg = (long)chunk * NL + lane;
+    const int lg = chunk * NL + lane;
     const bool active = lg < a.nlanes;
     int j = 0, k = 0;
     lane_jk(a, active ? lg : 0, j, k);  // inactive lanes read lane 0's data and store nothing
@@ -383,7 +386,7 @@ __global__ __launch_bounds__(NL *N2) void k_fft_inverse(FftArgs a, const Fields 
     const int sub = tid / NL;
     const int chunk = xcd_chunk((a.nlanes + NL - 1) / NL);
     if (chunk * NL >= a.nlanes) return;  // whole block
-    const long lg = (long)chunk * NL + lane;
+    const int lg = chunk * NL + lane;
     const bool active = lg < a.nlanes;
     int j = 0, k = 0;
     lane_jk(a, active ? lg : 0, j, k);  // inactive lanes read lane 0's data and store nothing
@@ -517,8 +520,9 @@ __device__ __forceinline__ void stockham_pass(const double2 *src, double2 *dst, 
 {
     const int nb = N / P;
     const int tstep = 2 * (N / (Ns * P));  // table step of exp(2 pi i/(Ns P)); r kk tstep < L
+    const float per = 1.0f / (float)Ns;    // b < 512: (b + 1/2)/Ns is further than its rounding from a whole number
     for (int b = sub; b < nb; b += NS) {
-        const int kk = b % Ns;
+        const int kk = b - Ns * (int)(((float)b + 0.5f) * per);
         double2 v[P];
 #pragma unroll
         for (int r = 0; r < P; ++r) v[r] = src[(b + r * nb) * NL + lane];
@@ -573,21 +577,28 @@ __device__ __forceinline__ double2 *stockham(const RadixPlan &rp, double2 *src, 
     return src;
 }
 
-// NL lanes per block, NS threads per lane, N <= NMAX (two buffers of
-// NMAX*NL values and the table of L = 2N twiddles in static LDS)
+// NL lanes per block, NS threads per lane, N <= NMAX = 8 NS; in LDS two buffers of
+// N*NL values and the table of L = 2N twiddles (as many as N needs, so that three
+// blocks share a CU at two thirds of NMAX).  What the time goes into is the
+// chain load, passes, store of a block, so a thread's (at most 8) loads are all
+// in flight at once and the index arithmetic has no division: 1000x32x96 (N = 48)
+// forward 24.3 -> 20.2 us, inverse 24.5 -> 19.9, 200x64x192 forward 23 -> 20,
+// inverse 26 -> 20 (a power of two's kernel would take 17).  In place, with
+// one buffer and every butterfly in registers, 266 registers leave one
+// wavefront per SIMD: 36 and 30 us.
 template <int NL, int NS, int NMAX>
 __global__ __launch_bounds__(NL *NS) void k_fft_forward_mr(FftArgs a, const Fields F, RadixPlan rp)
 {
     bind(a, F, blockIdx.y);
-    __shared__ double2 buf[2][NMAX * NL];
-    __shared__ double2 tw[2 * NMAX];
+    extern __shared__ double2 lds[];
     const int L = a.L, N = L / 2;
+    double2 *buf = lds, *tw = lds + 2 * N * NL;
     const int tid = threadIdx.x;
     const int lane = tid % NL;
     const int sub = tid / NL;
     const int chunk = xcd_chunk((a.nlanes + NL - 1) / NL);
     if (chunk * NL >= a.nlanes) return;  // whole block
-    const long lg = (long)chunk * NL + lane;
+    const int lg = chunk * NL + lane;
     const bool active = lg < a.nlanes;
     int j = 0, k = 0;
     lane_jk(a, active ? lg : 0, j, k);  // inactive lanes read lane 0's data and store nothing
@@ -595,14 +606,21 @@ __global__ __launch_bounds__(NL *NS) void k_fft_forward_mr(FftArgs a, const Fiel
     const double *rho = static_cast<const double *>(a.rho);
     const size_t plane = (size_t)a.JS * a.KS;
     const size_t base = (size_t)(j + 1) + (size_t)a.JS * (size_t)(k + 1);
-    // z_n = x_{2n} + i x_{2n+1}
-    for (int n = sub; n < N; n += NS) {
-        const size_t i0 = base + plane * (size_t)(2 * n), i1 = i0 + plane;
-        buf[0][n * NL + lane] = interior ? make_double2(rho[i0], rho[i1]) : make_double2(a.phi[i0], a.phi[i1]);
+    // z_n = x_{2n} + i x_{2n+1}; every load is issued before any is used
+    const double *src = interior ? rho : a.phi;
+    double2 x[NMAX / NS];
+#pragma unroll
+    for (int t = 0; t < NMAX / NS; ++t) {
+        const int n = min(sub + NS * t, N - 1);
+        const size_t i0 = base + plane * (size_t)(2 * n);
+        x[t] = make_double2(src[i0], src[i0 + plane]);
     }
     for (int e = tid; e < L; e += NL * NS) tw[e] = a.twL[e];
+#pragma unroll
+    for (int t = 0; t < NMAX / NS; ++t)
+        if (sub + NS * t < N) buf[(sub + NS * t) * NL + lane] = x[t];
     __syncthreads();
-    const double2 *z = stockham<+1>(rp, buf[0], buf[1], N, NL, NS, lane, sub, tw, a.tw64, L);
+    const double2 *z = stockham<+1>(rp, buf, buf + N * NL, N, NL, NS, lane, sub, tw, a.tw64, L);
     if (!active) return;
     forward_outputs<double>(a, z, tw, N, NL, NS, lane, sub, j, k, interior, base, plane);
 }
@@ -611,15 +629,15 @@ template <int NL, int NS, int NMAX>
 __global__ __launch_bounds__(NL *NS) void k_fft_inverse_mr(FftArgs a, const Fields F, RadixPlan rp)
 {
     bind(a, F, blockIdx.y);
-    __shared__ double2 buf[2][NMAX * NL];
-    __shared__ double2 tw[2 * NMAX];
+    extern __shared__ double2 lds[];
     const int L = a.L, N = L / 2;
+    double2 *buf = lds, *tw = lds + 2 * N * NL;
     const int tid = threadIdx.x;
     const int lane = tid % NL;
     const int sub = tid / NL;
     const int chunk = xcd_chunk((a.nlanes + NL - 1) / NL);
     if (chunk * NL >= a.nlanes) return;  // whole block
-    const long lg = (long)chunk * NL + lane;
+    const int lg = chunk * NL + lane;
     const bool active = lg < a.nlanes;
     int j = 0, k = 0;
     lane_jk(a, active ? lg : 0, j, k);  // inactive lanes read lane 0's data and store nothing
@@ -627,18 +645,26 @@ __global__ __launch_bounds__(NL *NS) void k_fft_inverse_mr(FftArgs a, const Fiel
     const size_t sidx = (size_t)k * a.J + j;
     // C_0 = a_0/2 and C_N = a_N/2 packed in slot 0, C_m = (a_m + i b_m)/2
     const double *spec = static_cast<const double *>(a.spec);
-    for (int m = sub; m <= N; m += NS) {
-        const double am = spec[(size_t)m * JK + sidx];
-        if (m == 0) buf[0][lane].x = 0.5 * am;
-        else if (m == N) buf[0][lane].y = 0.5 * am;
-        else buf[0][m * NL + lane] = make_double2(0.5 * am, 0.5 * spec[(size_t)(N + m) * JK + sidx]);
+    double av[NMAX / NS + 1], bv[NMAX / NS + 1];  // every load is issued before any is used
+#pragma unroll
+    for (int t = 0; t <= NMAX / NS; ++t) {
+        const int m = min(sub + NS * t, N);
+        av[t] = spec[(size_t)m * JK + sidx];
+        bv[t] = spec[(size_t)(m >= 1 && m < N ? N + m : 0) * JK + sidx];
     }
     for (int e = tid; e < L; e += NL * NS) tw[e] = a.twL[e];
+#pragma unroll
+    for (int t = 0; t <= NMAX / NS; ++t) {
+        const int m = sub + NS * t;
+        if (m == 0) buf[lane].x = 0.5 * av[t];
+        else if (m == N) buf[lane].y = 0.5 * av[t];
+        else if (m < N) buf[m * NL + lane] = make_double2(0.5 * av[t], 0.5 * bv[t]);
+    }
     __syncthreads();
-    inverse_presplit(buf[0], tw, N, NL, NS, lane, sub);
+    inverse_presplit(buf, tw, N, NL, NS, lane, sub);
     __syncthreads();
     // z_n = sum_k Z_k e^{-2 pi i k n/N}, x_{2n} = Re z_n, x_{2n+1} = Im z_n
-    const double2 *z = stockham<-1>(rp, buf[0], buf[1], N, NL, NS, lane, sub, tw, a.tw64, L);
+    const double2 *z = stockham<-1>(rp, buf, buf + N * NL, N, NL, NS, lane, sub, tw, a.tw64, L);
     if (!active) return;
     const size_t plane = (size_t)a.JS * a.KS;
     const size_t base = (size_t)(j + 1) + (size_t)a.JS * (size_t)(k + 1);
@@ -664,16 +690,17 @@ int launch_one(const FftArgs &a, const Fields &F, hipStream_t s)
     return (int)hipGetLastError();
 }
 
-// mixed-radix sizes: NL lanes per block with N*NL <= 2048 (two 32 KB buffers)
+// mixed-radix sizes: NL lanes per block with N*NL <= 2048 (two buffers of up to 32 KB)
 template <int NL, int KIND>
 int launch_mr(const FftArgs &a, const Fields &F, const RadixPlan &rp, hipStream_t s)
 {
     constexpr int NS = 256 / NL, NMAX = 2048 / NL;
+    const size_t lds = sizeof(double2) * ((size_t)a.L * NL + a.L);
     const int chunks = (a.nlanes + NL - 1) / NL;
     const int blocks = (chunks + kXcds - 1) / kXcds * kXcds;
     const dim3 grid(blocks, F.nf), block(NL * NS);
-    if (KIND == FWD64) hipLaunchKernelGGL((k_fft_forward_mr<NL, NS, NMAX>), grid, block, 0, s, a, F, rp);
-    if (KIND == INV64) hipLaunchKernelGGL((k_fft_inverse_mr<NL, NS, NMAX>), grid, block, 0, s, a, F, rp);
+    if (KIND == FWD64) hipLaunchKernelGGL((k_fft_forward_mr<NL, NS, NMAX>), grid, block, lds, s, a, F, rp);
+    if (KIND == INV64) hipLaunchKernelGGL((k_fft_inverse_mr<NL, NS, NMAX>), grid, block, lds, s, a, F, rp);
     return (int)hipGetLastError();
 }
 
