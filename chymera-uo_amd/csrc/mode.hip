@@ -161,7 +161,7 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void k_zgemm(ModeArgs a, const Fie
             }
 }
 
-// The same products for PP <= 128 (KMAX <= 128) with the weight table held in
+// The same products for KMAX <= 128 (binary32: 256) with the weight table held in
 // registers.  Persistent blocks (MINB per CU) walk output tiles of PPT rows x
 // PCT columns (tile = (q, column block)); wave w owns rows 16w..16w+15, keeps
 // its 16 x PPT slice of the weights as MFMA A operands for the whole run, and
@@ -737,18 +737,48 @@ ModeArgs make_args(const chy_grid *g)
 template <bool FWD, typename TI, typename TO, typename AT = double, int EPI = EPI_SPEC>
 void launch_zgemm(const chy_grid *g, const ModeArgs &a, const Fields &F, hipStream_t s)
 {
-    // 64-column tiles, one persistent block per CU (128 KB / 64 KB of LDS);
-    // the last binary32 inverse (binary32 X read, the binary64 spectrum
-    // written) in 32-column tiles, whose epilogue fits two blocks per CU
-    // (993 against 1147 us per 32-field launch at 256x128x256)
+    // 64-column tiles of persistent blocks; the last binary32 inverse (binary32
+    // X read, the binary64 spectrum written) in 32-column tiles, whose epilogue
+    // fits two blocks per CU (993 against 1147 us per 32-field launch at 256x128x256)
     constexpr int PCT = EPI == EPI_XFIN32 ? 32 : 64;
-    if (g->PP == 128 || g->PP == 64) {
-        // binary32 forward products and binary32-X inverses: two blocks per
-        // CU (half the LDS of a binary64 block; the binary64-X inverses'
-        // epilogues need more than the 128 registers that would leave)
-        constexpr int MB = (sizeof(AT) == 4 && (FWD || EPI == EPI_XSET32 || EPI == EPI_XFIN32)) ? 2 : 1;
-        const int col_tiles = ((FWD ? g->JP : g->M) + PCT - 1) / PCT;
-        const int ntiles = col_tiles * g->L * F.nf;
+    const int cols = FWD ? g->JP : g->M;  // k_rsolve reads zeros from M to JP
+    if constexpr (sizeof(AT) == 8) {
+        if (g->NZ <= 128) {
+            // the fewest rows of 16, 32, 64, 128 that hold the column (64 for
+            // every shorter one spent 28 us on a product at KMAX = 32,
+            // 1000x32x96, where 32 spend 16), 8 wavefronts (128 KB of LDS) per CU
+            const int col_tiles = (cols + PCT - 1) / PCT, ntiles = col_tiles * g->L * F.nf;
+            auto launch = [&](auto rows) {
+                constexpr int R = decltype(rows)::value, MB = 128 / R;
+                const int blocks = std::min(ntiles, MB * g->ncu);
+                hipLaunchKernelGGL((k_zgemm_reg<FWD, R, PCT, MB, TI, TO, AT, EPI>), dim3(blocks), dim3(R * 4), 0, s,
+                                   a, F, col_tiles, ntiles);
+            };
+            if (g->NZ <= 16) launch(std::integral_constant<int, 16>());
+            else if (g->NZ <= 32) launch(std::integral_constant<int, 32>());
+            else if (g->NZ <= 64) launch(std::integral_constant<int, 64>());
+            else launch(std::integral_constant<int, 128>());
+        } else if (FWD) {
+            dim3 gf((g->JP + CT - 1) / CT, (g->PP + RT - 1) / RT, g->L * F.nf);
+            hipLaunchKernelGGL((k_zgemm<true, TO>), gf, dim3(GEMM_THREADS), 0, s, a, F);
+        } else {
+            dim3 gi((g->M + CT - 1) / CT, (g->NZ + RT - 1) / RT, g->L * F.nf);
+            hipLaunchKernelGGL((k_zgemm<false, TO>), gi, dim3(GEMM_THREADS), 0, s, a, F);
+        }
+    } else if (g->PP == 256) {
+        // binary32 products of KMAX = 256 (the refined solve): 16 wavefronts
+        // of 16 rows, 16-column tiles (wider tiles spill the 64 A operands'
+        // neighbours out of the 128 registers a wavefront has), one block per CU
+        constexpr int PCT2 = 16;
+        const int col_tiles = (cols + PCT2 - 1) / PCT2, ntiles = col_tiles * g->L * F.nf;
+        hipLaunchKernelGGL((k_zgemm_reg<FWD, 256, PCT2, 1, TI, TO, AT, EPI>), dim3(std::min(ntiles, g->ncu)),
+                           dim3(1024), 0, s, a, F, col_tiles, ntiles);
+    } else {
+        // forward products and binary32-X inverses: two blocks per CU (the
+        // binary64-X inverses' epilogues need more than the 128 registers that
+        // would leave); PP is 64 or 128 here (refine_supported)
+        constexpr int MB = (FWD || EPI == EPI_XSET32 || EPI == EPI_XFIN32) ? 2 : 1;
+        const int col_tiles = (cols + PCT - 1) / PCT, ntiles = col_tiles * g->L * F.nf;
         const int blocks = std::min(ntiles, MB * g->ncu);
         if (g->PP == 128)
             hipLaunchKernelGGL((k_zgemm_reg<FWD, 128, PCT, MB, TI, TO, AT, EPI>), dim3(blocks), dim3(512), 0, s, a, F,
@@ -756,24 +786,6 @@ void launch_zgemm(const chy_grid *g, const ModeArgs &a, const Fields &F, hipStre
         else
             hipLaunchKernelGGL((k_zgemm_reg<FWD, 64, PCT, MB, TI, TO, AT, EPI>), dim3(blocks), dim3(256), 0, s, a, F,
                                col_tiles, ntiles);
-    } else if (g->PP == 256 && sizeof(AT) == 4) {
-        // binary32 products of KMAX = 256 (the refined solve): 16 wavefronts
-        // of 16 rows, 16-column tiles (wider tiles spill the 64 A operands'
-        // neighbours out of the 128 registers a wavefront has), one block per CU
-        if constexpr (sizeof(AT) == 4) {
-            constexpr int PCT2 = 16;
-            const int col_tiles = ((FWD ? g->JP : g->M) + PCT2 - 1) / PCT2;
-            const int ntiles = col_tiles * g->L * F.nf;
-            const int blocks = std::min(ntiles, g->ncu);
-            hipLaunchKernelGGL((k_zgemm_reg<FWD, 256, PCT2, 1, TI, TO, AT, EPI>), dim3(blocks), dim3(1024), 0, s, a,
-                               F, col_tiles, ntiles);
-        }
-    } else if (FWD) {
-        dim3 gf((g->JP + CT - 1) / CT, (g->PP + RT - 1) / RT, g->L * F.nf);
-        hipLaunchKernelGGL((k_zgemm<true, TO>), gf, dim3(GEMM_THREADS), 0, s, a, F);
-    } else {
-        dim3 gi((g->M + CT - 1) / CT, (g->NZ + RT - 1) / RT, g->L * F.nf);
-        hipLaunchKernelGGL((k_zgemm<false, TO>), gi, dim3(GEMM_THREADS), 0, s, a, F);
     }
 }
 
