@@ -615,7 +615,7 @@ def main():
     if refined is not None and args.coef_full_steps > 0:
         # the same batched refined solve writing COEF for every K, as the
         # reference's POT3 does (the timed region above writes the K=2 plane),
-        # beside the K=2 form timed the same way (HIP graph replays)
+        # beside the K=2 form timed the same way
         cf = {}
         for mode, key in ((chypot.COEF_K2, "k2_plane"), (chypot.COEF_FULL, "every_k")):
             for j in jobs:

@@ -197,7 +197,7 @@ class Context:
         _check(lib().chy_ctx_profile(self.handle, int(enable)), "chy_ctx_profile")
 
     def graphs(self, enable: bool = True):
-        """Replay chy_solve from captured HIP graphs (default on)."""
+        """Replay batches of several groups from captured HIP graphs (default on)."""
         _check(lib().chy_ctx_graphs(self.handle, int(enable)), "chy_ctx_graphs")
 
     def workers(self, n: int):

@@ -8,6 +8,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <new>
+#include <numeric>
 #include <string>
 #include <vector>
 
@@ -22,10 +23,6 @@ void set_device_error(hipError_t e, const char *where)
     g_last_error = std::string(where) + ": " + hipGetErrorString(e);
 }
 
-// a captured group's key: kGroupKeyHead argument words, then per field its
-// grid, density, PHI, COEF and KLOCAT
-constexpr size_t kGroupKeyHead = 8, kGroupKeyPerField = 5;
-constexpr size_t kGroupGraphCache = 16;
 // a captured batch's key: kBatchKeyHead words, then per item its grid,
 // arrays, arguments, KLOCAT in and whether it wants diagnostics
 constexpr size_t kBatchKeyHead = 6, kBatchKeyPerItem = 11;
@@ -220,7 +217,7 @@ static void wait_done(hipEvent_t done)
 }
 
 // waits for the entry's last launch, then frees it
-static void retire_graph(chy_grid::GraphEntry &e)
+static void retire_graph(chy_ctx::BatchGraph &e)
 {
     wait_done(e.done);
     if (e.exec) (void)hipGraphExecDestroy(e.exec);
@@ -228,36 +225,21 @@ static void retire_graph(chy_grid::GraphEntry &e)
     e.exec = nullptr;
 }
 
-static void retire_group_graph(chy_ctx::GroupGraph &e)
+// drops the captured batches that launch work on grid g (all with g null)
+static void drop_graphs(chy_ctx *c, const chy_grid *g)
 {
-    wait_done(e.done);
-    if (e.exec) (void)hipGraphExecDestroy(e.exec);
-    e.done = nullptr;
-    e.exec = nullptr;
-}
-
-// drops the cached graphs of v whose keys (head words, then per item a
-// record whose first word is the grid) name grid g (all with g null)
-static void drop_graphs_of(std::vector<chy_ctx::GroupGraph> &v, size_t head, size_t per, const chy_grid *g)
-{
+    auto &v = c->batch_graphs;
     for (size_t i = 0; i < v.size();) {
         bool hit = g == nullptr;
-        for (size_t k = head; !hit && k < v[i].key.size(); k += per) hit = v[i].key[k] == (uintptr_t)g;
+        for (size_t k = kBatchKeyHead; !hit && k < v[i].key.size(); k += kBatchKeyPerItem)
+            hit = v[i].key[k] == (uintptr_t)g;
         if (hit) {
-            retire_group_graph(v[i]);
+            retire_graph(v[i]);
             v.erase(v.begin() + (long)i);
         } else {
             ++i;
         }
     }
-}
-
-// drops the captured group and batch graphs that launch work on grid g (all
-// with g null)
-static void drop_group_graphs(chy_ctx *c, const chy_grid *g)
-{
-    drop_graphs_of(c->group_graphs, kGroupKeyHead, kGroupKeyPerField, g);
-    drop_graphs_of(c->batch_graphs, kBatchKeyHead, kBatchKeyPerItem, g);
 }
 
 // true while s records into a graph (a capture of ours or of the caller's):
@@ -311,7 +293,7 @@ static int run_pot3_tail(chy_grid *g, hipStream_t s, int npoint, double *phi, in
 // both the spectrum and the ring moments; BDYGEN then writes the boundary
 // lanes' spectrum directly (a Fourier series of order <= MAXTRM).  For
 // LMAX/2 <= 10 the boundary values go through PHI and a transform instead.
-static int run_solve_eager(chy_grid *g, hipStream_t s, int maxtrm, int isym, double redge, int npoint,
+static int run_solve(chy_grid *g, hipStream_t s, int maxtrm, int isym, double redge, int npoint,
                            const double *rho, double *phi, double *coef, int coef_mode, int klocat_in)
 {
     Profiler *p = g->ctx->prof.on ? &g->ctx->prof : nullptr;
@@ -336,57 +318,8 @@ static int run_solve_eager(chy_grid *g, hipStream_t s, int maxtrm, int isym, dou
     return run_pot3_tail(g, s, npoint, phi, klocat_in, !spectral);
 }
 
-// The same sequence replayed from a HIP graph (captured on first use for a
-// given set of arguments) when stage timing is off: one launch per solve.
-static int run_solve(chy_grid *g, hipStream_t s, int maxtrm, int isym, double redge, int npoint,
-                     const double *rho, double *phi, double *coef, int coef_mode, int klocat_in)
-{
-    if (!bdygen_args_ok(maxtrm, isym, redge)) return CHY_EINVAL;
-    chy_ctx *c = g->ctx;
-    if (c->prof.on || !c->graphs || capturing(s))
-        return run_solve_eager(g, s, maxtrm, isym, redge, npoint, rho, phi, coef, coef_mode, klocat_in);
-    SolveKey key{rho, phi, coef, coef_mode, maxtrm, isym, npoint, klocat_in, redge, s};
-    hipGraphExec_t exec = nullptr;
-    for (size_t i = 0; i < g->graphs.size(); ++i) {
-        if (g->graphs[i].key == key) {
-            chy_grid::GraphEntry hit = g->graphs[i];
-            g->graphs.erase(g->graphs.begin() + (long)i);
-            g->graphs.push_back(hit);
-            exec = hit.exec;
-            break;
-        }
-    }
-    if (!exec) {
-        hipGraph_t graph = nullptr;
-        hipError_t e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
-        if (e != hipSuccess) return dev_rc((int)e, "hipStreamBeginCapture");
-        int rc = run_solve_eager(g, s, maxtrm, isym, redge, npoint, rho, phi, coef, coef_mode, klocat_in);
-        e = hipStreamEndCapture(s, &graph);
-        if (rc) {
-            if (graph) (void)hipGraphDestroy(graph);
-            return rc;
-        }
-        if (e != hipSuccess) return dev_rc((int)e, "hipStreamEndCapture");
-        e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(graph);
-        if (e != hipSuccess) return dev_rc((int)e, "hipGraphInstantiate");
-        hipEvent_t done = nullptr;
-        e = hipEventCreateWithFlags(&done, hipEventDisableTiming);
-        if (e != hipSuccess) {
-            (void)hipGraphExecDestroy(exec);
-            return dev_rc((int)e, "hipEventCreate");
-        }
-        if ((int)g->graphs.size() >= kGraphCache) retire_graph(g->graphs.front());
-        if ((int)g->graphs.size() >= kGraphCache) g->graphs.erase(g->graphs.begin());
-        g->graphs.push_back(chy_grid::GraphEntry{key, exec, done});
-    }
-    int rc = dev_rc((int)hipGraphLaunch(exec, s), "hipGraphLaunch");
-    if (rc == CHY_OK) rc = dev_rc((int)hipEventRecord(g->graphs.back().done, s), "hipEventRecord");
-    return rc;
-}
-
 // BDYGEN + POT3 of every field in F (spectral BDYGEN), one launch per kernel
-// on grid g's tables: the sequence of run_solve_eager, field by field the
+// on grid g's tables: the sequence of run_solve, field by field the
 // same arithmetic, so each field's result equals its own chy_solve's.
 static int run_solve_fields(chy_grid *g, const Fields &F, hipStream_t s, int maxtrm, int isym, double redge,
                             int npoint, int coef_mode)
@@ -686,7 +619,7 @@ int chy_ctx_destroy(chy_ctx *ctx)
     DeviceScope ds(ctx->device);
     ctx->prof.collect();
     ctx->prof.release();
-    drop_group_graphs(ctx, nullptr);
+    drop_graphs(ctx, nullptr);
     release_workers(ctx);
     if (ctx->fork_ev) (void)hipEventDestroy(ctx->fork_ev);
     if (ctx->d_diag) (void)hipFree(ctx->d_diag);
@@ -711,69 +644,58 @@ int chy_ctx_workers(chy_ctx *ctx, int n)
 }
 
 // chy_solve_batch (steps = 0) and chy_solve_batch_refined (steps > 0)
-// One group of a batch (fields on identically described grids, one launch per
-// kernel), replayed from a captured HIP graph when the same group with the
-// same arrays and arguments ran before on the same stream (graphs on, stage
-// timing off); the capture holds kernel launches only.
-static int run_group(chy_ctx *ctx, const chy_solve_item &lead, const std::vector<chy_grid *> &grids,
-                     const Fields &F, hipStream_t s, int np, int steps)
+
+// items that may run together, one launch per kernel
+static bool batchable(const chy_solve_item &a, const chy_solve_item &b)
 {
-    auto eager = [&]() {
-        if (steps > 0)
-            return run_refined_fields(lead.grid, grids, F, s, lead.maxtrm, lead.isym, lead.redge, np,
-                                      lead.coef_mode, steps, false);
-        return run_solve_fields(lead.grid, F, s, lead.maxtrm, lead.isym, lead.redge, np, lead.coef_mode);
-    };
-    if (ctx->prof.on || !ctx->graphs || capturing(s)) return eager();
-    std::vector<uintptr_t> key(kGroupKeyHead + kGroupKeyPerField * (size_t)F.nf);
-    uint64_t rbits;
-    std::memcpy(&rbits, &lead.redge, sizeof(rbits));
-    key[0] = (uintptr_t)steps; key[1] = (uintptr_t)lead.maxtrm; key[2] = (uintptr_t)(lead.isym + 8);
-    key[3] = (uintptr_t)np; key[4] = (uintptr_t)lead.coef_mode; key[5] = (uintptr_t)rbits;
-    key[6] = (uintptr_t)s; key[7] = (uintptr_t)F.nf;
-    for (int f = 0; f < F.nf; ++f) {
-        uintptr_t *k = key.data() + kGroupKeyHead + kGroupKeyPerField * f;
-        k[0] = (uintptr_t)grids[f]; k[1] = (uintptr_t)F.rho[f]; k[2] = (uintptr_t)F.phi[f];
-        k[3] = (uintptr_t)F.coef[f]; k[4] = (uintptr_t)(uint32_t)F.klocat_in[f];
-    }
-    auto &cache = ctx->group_graphs;
-    size_t hit = cache.size();
-    for (size_t i = 0; i < cache.size(); ++i)
-        if (cache[i].key == key) hit = i;
-    if (hit == cache.size()) {
-        hipGraph_t graph = nullptr;
-        hipError_t e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
-        if (e != hipSuccess) return dev_rc((int)e, "hipStreamBeginCapture");
-        int rc = eager();
-        e = hipStreamEndCapture(s, &graph);
-        if (rc) {
-            if (graph) (void)hipGraphDestroy(graph);
-            return rc;
-        }
-        if (e != hipSuccess) return dev_rc((int)e, "hipStreamEndCapture");
-        chy_ctx::GroupGraph g;
-        g.key = std::move(key);
-        e = hipGraphInstantiate(&g.exec, graph, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(graph);
-        if (e != hipSuccess) return dev_rc((int)e, "hipGraphInstantiate");
-        e = hipEventCreateWithFlags(&g.done, hipEventDisableTiming);
-        if (e != hipSuccess) {
-            (void)hipGraphExecDestroy(g.exec);
-            return dev_rc((int)e, "hipEventCreate");
-        }
-        if (cache.size() >= kGroupGraphCache) {
-            retire_group_graph(cache.front());
-            cache.erase(cache.begin());
-        }
-        cache.push_back(std::move(g));
-        hit = cache.size() - 1;
+    return same_tables(a.grid, b.grid) && bdygen_spectral_ok(a.grid) && a.maxtrm == b.maxtrm && a.isym == b.isym &&
+           a.redge == b.redge && std::min(a.npoint, 10) == std::min(b.npoint, 10) && a.coef_mode == b.coef_mode;
+}
+
+// One group of a batch (items grp of identically described grids, one launch
+// per kernel) on stream s, with its diagnostics.
+static int run_group(chy_ctx *ctx, const chy_solve_item *items, const std::vector<int> &grp, hipStream_t s, int steps)
+{
+    const chy_solve_item &lead = items[grp[0]];
+    const int np = std::min(lead.npoint, 10);
+    int rc;
+    if (grp.size() == 1 && steps == 0) {
+        rc = run_solve(lead.grid, s, lead.maxtrm, lead.isym, lead.redge, np, lead.rho_d, lead.phi_d, lead.coef_d,
+                       lead.coef_mode, lead.diag ? lead.diag->klocat : 0);
     } else {
-        std::rotate(cache.begin() + (long)hit, cache.begin() + (long)hit + 1, cache.end());
-        hit = cache.size() - 1;
+        Fields F{};
+        F.nf = (int)grp.size();
+        std::vector<chy_grid *> grids(F.nf);
+        for (int f = 0; f < F.nf; ++f) {
+            const chy_solve_item &it = items[grp[f]];
+            set_field(F, f, it.grid, it.rho_d, it.phi_d, it.coef_d, it.diag ? it.diag->klocat : 0);
+            grids[f] = it.grid;
+        }
+        rc = steps > 0 ? run_refined_fields(lead.grid, grids, F, s, lead.maxtrm, lead.isym, lead.redge, np,
+                                            lead.coef_mode, steps, false)
+                       : run_solve_fields(lead.grid, F, s, lead.maxtrm, lead.isym, lead.redge, np, lead.coef_mode);
     }
-    int rc = dev_rc((int)hipGraphLaunch(cache[hit].exec, s), "hipGraphLaunch");
-    if (rc == CHY_OK) rc = dev_rc((int)hipEventRecord(cache[hit].done, s), "hipEventRecord");
+    for (size_t f = 0; f < grp.size() && rc == CHY_OK; ++f) {
+        const chy_solve_item &it = items[grp[f]];
+        if (it.diag)
+            rc = dev_rc((int)hipMemcpyAsync(ctx->d_diag + 3 * grp[f], it.grid->d.dscal, 3 * sizeof(double),
+                                            hipMemcpyDeviceToDevice, s),
+                        "diagnostics copy");
+    }
     return rc;
+}
+
+// True when the batch is one group: every item on a grid object of its own,
+// all of them together in one launch per kernel.
+static bool one_group(const chy_solve_item *items, int n)
+{
+    if (n > kMaxBatch) return false;
+    for (int i = 1; i < n; ++i) {
+        if (!batchable(items[0], items[i])) return false;
+        for (int j = 0; j < i; ++j)
+            if (items[j].grid == items[i].grid) return false;
+    }
+    return true;
 }
 
 // The fork from the context's stream, the groups on the worker streams and
@@ -795,11 +717,6 @@ static int issue_batch(chy_ctx *ctx, const chy_solve_item *items, int n, int ste
             if (items[j].grid == items[i].grid) ++round[i];
         nrounds = std::max(nrounds, round[i] + 1);
     }
-    auto batchable = [](const chy_solve_item &a, const chy_solve_item &b) {
-        return same_tables(a.grid, b.grid) && bdygen_spectral_ok(a.grid) && a.maxtrm == b.maxtrm &&
-               a.isym == b.isym && a.redge == b.redge && std::min(a.npoint, 10) == std::min(b.npoint, 10) &&
-               a.coef_mode == b.coef_mode;
-    };
     const int nw = ctx->nworkers;
     std::vector<chy_grid *> seen;      // grid objects in order of first appearance (worker = index % nw)
     std::vector<int> last_w;           // worker of each seen grid's latest use, -1 before it
@@ -842,28 +759,7 @@ static int issue_batch(chy_ctx *ctx, const chy_solve_item *items, int n, int ste
                     waited.push_back(v);
                 }
             }
-            const int np = std::min(lead.npoint, 10);
-            if (rc == CHY_OK && grp.size() == 1 && steps == 0) {
-                rc = run_solve(lead.grid, s, lead.maxtrm, lead.isym, lead.redge, np, lead.rho_d, lead.phi_d,
-                               lead.coef_d, lead.coef_mode, lead.diag ? lead.diag->klocat : 0);
-            } else if (rc == CHY_OK) {
-                Fields F{};
-                F.nf = (int)grp.size();
-                std::vector<chy_grid *> grids(F.nf);
-                for (int f = 0; f < F.nf; ++f) {
-                    const chy_solve_item &it = items[grp[f]];
-                    set_field(F, f, it.grid, it.rho_d, it.phi_d, it.coef_d, it.diag ? it.diag->klocat : 0);
-                    grids[f] = it.grid;
-                }
-                rc = run_group(ctx, lead, grids, F, s, np, steps);
-            }
-            for (size_t f = 0; f < grp.size() && rc == CHY_OK; ++f) {
-                const chy_solve_item &it = items[grp[f]];
-                if (it.diag)
-                    rc = dev_rc((int)hipMemcpyAsync(ctx->d_diag + 3 * grp[f], it.grid->d.dscal, 3 * sizeof(double),
-                                                    hipMemcpyDeviceToDevice, s),
-                                "diagnostics copy");
-            }
+            if (rc == CHY_OK) rc = run_group(ctx, items, grp, s, steps);
             // this worker's progress so far, for later groups that reuse these grids elsewhere
             if (rc == CHY_OK) rc = dev_rc((int)hipEventRecord(ctx->worker_ev[w], s), "hipEventRecord");
             for (int i : grp) last_w[grid_index(items[i].grid)] = w;
@@ -879,10 +775,13 @@ static int issue_batch(chy_ctx *ctx, const chy_solve_item *items, int n, int ste
     return rc;
 }
 
-// A batch replayed from a HIP graph of the whole fork, groups and join when
-// the same batch (grids, arrays, arguments, worker count, stream, diagnostics
-// staging) ran before; captured on first use.  Work on different grids stays
-// on different branches of the graph, as on the worker streams.
+// A batch of several groups replayed from a HIP graph of the whole fork,
+// groups and join when the same batch (grids, arrays, arguments, worker count,
+// stream, diagnostics staging) ran before: its first run is issued to the
+// streams, its second one captured (a capture costs two to three runs, which
+// callers with other arrays each time would pay every time).  Work on
+// different grids stays on different branches of the graph, as on the worker
+// streams.
 static int run_batch_graph(chy_ctx *ctx, const chy_solve_item *items, int n, int steps, bool any_diag)
 {
     std::vector<uintptr_t> key(kBatchKeyHead + kBatchKeyPerItem * (size_t)n);
@@ -903,6 +802,14 @@ static int run_batch_graph(chy_ctx *ctx, const chy_solve_item *items, int n, int
     for (size_t i = 0; i < cache.size(); ++i)
         if (cache[i].key == key) hit = i;
     if (hit == cache.size()) {
+        auto &before = ctx->batch_seen;
+        const auto known = std::find(before.begin(), before.end(), key);
+        if (known == before.end()) {
+            if (before.size() >= kBatchGraphCache) before.erase(before.begin());
+            before.push_back(std::move(key));
+            return issue_batch(ctx, items, n, steps);
+        }
+        before.erase(known);
         hipGraph_t graph = nullptr;
         hipError_t e = hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal);
         if (e != hipSuccess) return dev_rc((int)e, "hipStreamBeginCapture");
@@ -913,7 +820,7 @@ static int run_batch_graph(chy_ctx *ctx, const chy_solve_item *items, int n, int
             return rc;
         }
         if (e != hipSuccess) return dev_rc((int)e, "hipStreamEndCapture");
-        chy_ctx::GroupGraph b;
+        chy_ctx::BatchGraph b;
         b.key = std::move(key);
         e = hipGraphInstantiate(&b.exec, graph, nullptr, nullptr, 0);
         (void)hipGraphDestroy(graph);
@@ -924,7 +831,7 @@ static int run_batch_graph(chy_ctx *ctx, const chy_solve_item *items, int n, int
             return dev_rc((int)e, "hipEventCreate");
         }
         if (cache.size() >= kBatchGraphCache) {
-            retire_group_graph(cache.front());
+            retire_graph(cache.front());
             cache.erase(cache.begin());
         }
         cache.push_back(std::move(b));
@@ -963,7 +870,7 @@ static int solve_batch(chy_ctx *ctx, const chy_solve_item *items, int n, int ste
     for (int i = 0; i < n && steps > 0 && rc == CHY_OK; ++i) rc = ensure_refine(items[i].grid, use32);
     if (rc) return rc;
     if (any_diag && ctx->diag_cap < n) {
-        drop_graphs_of(ctx->batch_graphs, kBatchKeyHead, kBatchKeyPerItem, nullptr);  // they copy into the old staging
+        drop_graphs(ctx, nullptr);  // they copy into the old staging
         if (ctx->d_diag) (void)hipFree(ctx->d_diag);
         if (ctx->h_diag) (void)hipHostFree(ctx->h_diag);
         ctx->d_diag = ctx->h_diag = nullptr;
@@ -972,12 +879,18 @@ static int solve_batch(chy_ctx *ctx, const chy_solve_item *items, int n, int ste
         if (hipHostMalloc(&ctx->h_diag, sizeof(double) * 3 * n) != hipSuccess) return CHY_ENOMEM;
         ctx->diag_cap = n;
     }
-    // one graph launch for the whole batch unless stage timing is on, graphs
-    // are off or the caller is capturing the context's stream
-    if (ctx->graphs && !ctx->prof.on && !capturing(ctx->stream))
+    // one group: plain launches on the context's own stream.  Several: one graph
+    // launch unless stage timing is on, graphs are off or the caller is
+    // capturing the context's stream
+    if (one_group(items, n)) {
+        std::vector<int> all(n);
+        std::iota(all.begin(), all.end(), 0);
+        rc = run_group(ctx, items, all, ctx->stream, steps);
+    } else if (ctx->graphs && !ctx->prof.on && !capturing(ctx->stream)) {
         rc = run_batch_graph(ctx, items, n, steps, any_diag);
-    else
+    } else {
         rc = issue_batch(ctx, items, n, steps);
+    }
     if (rc || !any_diag) return rc;
     hipError_t e = hipMemcpyAsync(ctx->h_diag, ctx->d_diag, sizeof(double) * 3 * n, hipMemcpyDeviceToHost,
                                   ctx->stream);
@@ -1069,9 +982,7 @@ int chy_grid_set_mode_solver(chy_grid *g, int kind)
     if (kind == CHY_MODES_CR && !cr_supported(g)) return CHY_EUNSUPPORTED;
     if (kind == g->mode_solver) return CHY_OK;
     DeviceScope ds(g->ctx->device);
-    for (auto &e : g->graphs) retire_graph(e);
-    g->graphs.clear();
-    drop_group_graphs(g->ctx, g);
+    drop_graphs(g->ctx, g);
     g->mode_solver = kind;
     return CHY_OK;
 }
@@ -1088,9 +999,7 @@ int chy_grid_set_tune(chy_grid *g, int param, int value)
     if (!slot) return CHY_EINVAL;
     if (*slot == value) return CHY_OK;
     DeviceScope ds(g->ctx->device);
-    for (auto &e : g->graphs) retire_graph(e);
-    g->graphs.clear();
-    drop_group_graphs(g->ctx, g);
+    drop_graphs(g->ctx, g);
     *slot = value;
     return CHY_OK;
 }
@@ -1112,9 +1021,7 @@ int chy_grid_destroy(chy_grid *g)
         (void)hipGetLastError();
         (void)hipDeviceSynchronize();
     }
-    for (auto &e : g->graphs) retire_graph(e);
-    g->graphs.clear();
-    drop_group_graphs(g->ctx, g);
+    drop_graphs(g->ctx, g);
     free_grid_memory(g);
     delete g;
     (void)hipGetLastError();  // a failed release must not surface at the caller's next launch check

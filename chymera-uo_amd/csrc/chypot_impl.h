@@ -28,8 +28,6 @@ constexpr int kTermM[kMaxTerms] = {0, 1, 0, 2, 1, 3, 0, 2, 4, 1, 3, 5, 0, 2, 4, 
                                    5, 7, 0, 2, 4, 6, 8, 1, 3, 5, 7, 9, 0, 2, 4, 6, 8, 10};
 // Rings per boundary chunk (the unit of the deterministic radial reduction).
 constexpr int kChunkRings = 64;
-// Captured solve graphs kept per grid (one per distinct argument set).
-constexpr int kGraphCache = 8;
 // Most refinement steps of chy_solve_refined.
 constexpr int kMaxRefine = 8;
 
@@ -165,7 +163,7 @@ struct chy_ctx {
     int device = 0;
     hipStream_t own = nullptr;
     hipStream_t stream = nullptr;
-    bool graphs = true;  // replay chy_solve from captured HIP graphs
+    bool graphs = true;  // replay batches of several groups from captured HIP graphs
     chy::Profiler prof;
     // chy_solve_batch: worker streams (default priority), fork/join events,
     // per-item diagnostics staging
@@ -188,36 +186,17 @@ struct chy_ctx {
     int force_cap = 0;
     // chy_find_force_noalloc: the device's fixed scratch (force.hip)
     double *force_scratch = nullptr;
-    // chy_solve_batch: captured graphs of multi-field groups, keyed on the
-    // group's grids, arrays and arguments, most recently used last
-    struct GroupGraph {
+    // chy_solve_batch: captured graphs of whole batches (fork, groups, join),
+    // keyed on every item, the worker count, the stream and the diagnostics
+    // staging, most recently used last; the keys of batches run once so far
+    struct BatchGraph {
         std::vector<uintptr_t> key;
         hipGraphExec_t exec = nullptr;
         hipEvent_t done = nullptr;
     };
-    std::vector<GroupGraph> group_graphs;
-    // chy_solve_batch: captured graphs of whole batches (fork, groups, join),
-    // keyed on every item, the worker count, the stream and the diagnostics
-    // staging, most recently used last
-    std::vector<GroupGraph> batch_graphs;
+    std::vector<BatchGraph> batch_graphs;
+    std::vector<std::vector<uintptr_t>> batch_seen;
 };
-
-namespace chy {
-// Arguments a captured solve graph was recorded with.
-struct SolveKey {
-    const void *rho;
-    void *phi, *coef;
-    int coef_mode, maxtrm, isym, npoint, klocat_in;
-    double redge;
-    hipStream_t stream;
-    bool operator==(const SolveKey &o) const
-    {
-        return rho == o.rho && phi == o.phi && coef == o.coef && coef_mode == o.coef_mode &&
-               maxtrm == o.maxtrm && isym == o.isym && npoint == o.npoint && klocat_in == o.klocat_in &&
-               redge == o.redge && stream == o.stream;
-    }
-};
-}  // namespace chy
 
 struct chy_grid {
     chy_ctx *ctx = nullptr;
@@ -240,14 +219,6 @@ struct chy_grid {
     size_t device_bytes = 0;
     std::vector<void *> allocations;
     chy::DeviceGrid d;
-    // captured chy_solve graphs, most recently used last (at most kGraphCache);
-    // `done` is recorded after every launch so an entry can be retired safely
-    struct GraphEntry {
-        chy::SolveKey key;
-        hipGraphExec_t exec;
-        hipEvent_t done;
-    };
-    std::vector<GraphEntry> graphs;
 };
 
 namespace chy {

@@ -119,8 +119,8 @@ size_t chy_grid_device_bytes(const chy_grid *g);
  *                   (whose root tables put it up to a few 1e-12 from it at
  *                   256x128x256), and faster.
  * CHY_MODES_CR needs JMAX-1 <= 512 (CHY_EUNSUPPORTED otherwise; such grids
- * start with CHY_MODES_EIGEN).  Changing the solver drops the grid's captured
- * solve graphs. */
+ * start with CHY_MODES_EIGEN).  Changing the solver drops the captured batches
+ * that use the grid. */
 enum { CHY_MODES_CR = 0, CHY_MODES_EIGEN = 1 };
 int chy_grid_set_mode_solver(chy_grid *g, int kind);
 int chy_grid_mode_solver(const chy_grid *g);
@@ -139,7 +139,7 @@ int chy_grid_mode_solver(const chy_grid *g);
  *                        JMAX <= 257) instead of the mode solves that
  *                        chy_solve_refined otherwise uses
  * Results do not depend on the shapes beyond rounding.  Changing a value
- * drops the grid's captured solve graphs.  CHY_EINVAL for a value the grid
+ * drops the captured batches that use the grid.  CHY_EINVAL for a value the grid
  * cannot take. */
 enum { CHY_TUNE_CR_LANES = 0, CHY_TUNE_REFINE_M64 = 1, CHY_TUNE_REFINE_FUSED = 2 };
 int chy_grid_set_tune(chy_grid *g, int param, int value);
@@ -169,15 +169,14 @@ int chy_pot3(chy_grid *g, int npoint, const double *rho_d, double *phi_d, double
              int coef_mode, chy_diag *diag);
 
 /* BDYGEN followed by POT3: one potential solve, device-resident, one stream.
- * Writes the same cells of phi_d as chy_bdygen then chy_pot3 would.  Unless
- * stage timing is on or graphs are off (chy_ctx_graphs), the kernel sequence
- * is captured into a HIP graph on the first call with a given set of
- * arguments (pointers, scalars, stream) and replayed by later calls with the
- * same set; a call with different arguments re-captures. */
+ * Writes the same cells of phi_d as chy_bdygen then chy_pot3 would.  The
+ * kernels are launched one after another: replayed as a HIP graph (captured
+ * per set of arguments) a solve took 5-8 us longer behind earlier work, for
+ * the graph's start and the event that guards its release, and no less
+ * alone. */
 int chy_solve(chy_grid *g, int maxtrm, int isym, double redge, int npoint, const double *rho_d,
               double *phi_d, double *coef_d, int coef_mode, chy_diag *diag);
-/* Enable (default) or disable graph replay of chy_solve and chy_solve_batch
- * on this context. */
+/* Enable (default) or disable graph replay of chy_solve_batch on this context. */
 int chy_ctx_graphs(chy_ctx *ctx, int enable);
 
 /* ---- batched solves (no reference counterpart: the reference solves one
@@ -192,11 +191,12 @@ int chy_ctx_graphs(chy_ctx *ctx, int enable);
  * worker streams.  Each item's results are bitwise those of chy_solve on the
  * same arguments.  If any item has a diag pointer the call waits and fills
  * every such diag.  Every item is checked before anything is launched.
- * Unless stage timing is on, graphs are off or the caller is capturing the
- * context's stream, the whole batch (fork, groups, join) is captured into one
- * HIP graph the first time a given batch runs (same grids, arrays, arguments,
- * worker count and stream) and replayed as one launch by later calls; a
- * change to a grid's solver or tuning drops the graphs that use it. */
+ * A batch whose items all run together goes to the context's stream itself.
+ * Any other one is captured into one HIP graph (fork, groups, join) the second
+ * time it runs (same grids, arrays, arguments, worker count and stream) and
+ * replayed as one launch by later calls, unless stage timing is on, graphs are
+ * off or the caller is capturing the context's stream; a change to a grid's
+ * solver or tuning drops the graphs that use it. */
 typedef struct {
     chy_grid *grid;
     const double *rho_d;
