@@ -97,7 +97,7 @@ class Server:
         self.tune_table = tune_table or {}  # chypot.autotune table applied to every new slot's grid
         ctx.workers(workers)
         # eager launches: each request brings its own density buffer, so a
-        # captured single-field graph (keyed on its pointers) would rarely replay
+        # captured batch (keyed on its pointers) would rarely replay
         ctx.graphs(False)
         # the context's stream: batches fork from and join back to it
         self.stream = torch.cuda.Stream()

@@ -456,15 +456,16 @@ int build_cr_plan(CrPlan &plan, int n, const double *an, const double *bn, const
     // lev[lv][b * (2^(lv+1)-1) + i]: roots of block b of level lv (rows
     // 1 + b 2^lv .. b 2^lv + 2^(lv+1) - 1), negated eigenvalues of the z
     // sub-tridiagonal, by increasing magnitude
+    const int lv0 = std::min(kx - 1, 4);  // the lowest nodes' level: leaves of 2^lv0 - 1 rows
     const double machep = cr_machep();
     std::vector<std::vector<double>> lev(kx);
     lev[0].resize(n);
     for (int i = 0; i < n; ++i) lev[0][i] = -bn[i];
-    for (int lv = 1; lv < kx; ++lv) {
+    for (int lv = std::max(1, lv0 - 1); lv < kx; ++lv) {
         const int step = 1 << lv, size = 2 * step - 1, nblk = (1 << (kx - lv)) - 1;
         lev[lv].resize((size_t)size * nblk);
         std::vector<double> d(size), e2(size);
-        for (int b = 0; b < nblk; ++b) {
+        for (int b = 0; b < nblk; b += 2) {  // the others lie across the tree's blocks
             const int r0 = b * step;
             for (int i = 0; i < size; ++i) d[i] = bn[r0 + i];
             for (int i = 0; i + 1 < size; ++i) e2[i] = cpl2[r0 + i + 1];
@@ -476,7 +477,6 @@ int build_cr_plan(CrPlan &plan, int n, const double *an, const double *bn, const
 
     plan.kx = kx;
     plan.phases.clear();
-    const int lv0 = std::min(kx - 1, 4);  // the lowest nodes' level: leaves of 2^lv0 - 1 rows
     plan.rows = (1 << lv0) - 1;
     plan.nleaf = (n + 1) >> lv0;
     plan.leaf.assign((size_t)plan.nleaf * kLeafStride, 0.0);

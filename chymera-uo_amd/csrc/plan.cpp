@@ -350,7 +350,8 @@ int build_grid(chy_grid *g, const chy_grid_desc *desc, int isym)
         }
 
     // ---- BLKTRI's root tables and the cyclic reduction's weights (crplan.cpp) ----
-    CHY_TRY(build_cr_plan(g->cr, NZ, an.data(), bn.data(), cn.data()));
+    // (r systems too long for its kernels: no tables)
+    if (JP <= 512) CHY_TRY(build_cr_plan(g->cr, NZ, an.data(), bn.data(), cn.data()));
     g->mode_solver = cr_supported(g) ? CHY_MODES_CR : CHY_MODES_EIGEN;
     // two orders per wavefront where the r system fits 32 lanes: measured
     // faster or equal on every grid class tried (chypot/tuned_mi355x.json)
