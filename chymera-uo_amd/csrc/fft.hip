@@ -82,10 +82,10 @@ __device__ __forceinline__ void dft_reg(double2 (&v)[P], const double2 *__restri
 // then fetched (or written back) once.  The grid is rounded up to a multiple
 // of 8; blocks past the last chunk leave at once.
 constexpr int kXcds = 8;
-__device__ __forceinline__ int xcd_chunk(int nchunks)
+__device__ __forceinline__ int xcd_chunk(int nchunks, int block)
 {
     const int per = (nchunks + kXcds - 1) / kXcds;
-    return (int)(blockIdx.x % kXcds) * per + (int)(blockIdx.x / kXcds);
+    return block % kXcds * per + block / kXcds;
 }
 
 // the radices of a mixed-radix transform, first pass first
@@ -131,11 +131,34 @@ struct FftArgs {
     int lanes;            // LANES_ALL / LANES_INTERIOR / LANES_BOUNDARY
     int nlanes;
     int coef_mode;
+    int coef_blocks;      // forward: leading blocks that form COEF alone, coef_parts per chunk of lanes (or 0)
+    int coef_parts;
     double sf1, pi;
     double ys;            // factor on the interior lanes' spectrum (4 pi G)
     int ghosts;           // inverse: also write POT3's axis/midplane ghost cells
     double *zsamp;        // inverse: [KMAX][kZaxSamples][L] copy of PHI(J=2..6,K,L) for ZAXPHI, or null
 };
+
+// The forward transform's block: its chunk of lanes, with a's outputs cut down
+// to what the block forms, and the part of the orders it forms COEF for (the
+// part-th of every `parts` rounds of the block's threads).  The launch's leading
+// coef_blocks form COEF alone, the others everything else.
+__device__ __forceinline__ int forward_chunk(FftArgs &a, int nl, int &part, int &parts)
+{
+    const int nchunks = (a.nlanes + nl - 1) / nl;
+    part = 0;
+    parts = 1;
+    if (a.coef_blocks == 0) return xcd_chunk(nchunks, (int)blockIdx.x);
+    if ((int)blockIdx.x >= a.coef_blocks) {
+        a.coef = nullptr;
+        return xcd_chunk(nchunks, (int)blockIdx.x - a.coef_blocks);
+    }
+    a.spec = nullptr;
+    a.mom = nullptr;
+    parts = a.coef_parts;
+    part = (int)blockIdx.x % parts;
+    return (int)blockIdx.x / parts;
+}
 
 // lane index -> (j,k), j = J-2 (0..JMAX-1), k = K-2 (0..KMAX-1)
 __device__ __forceinline__ void lane_jk(const FftArgs &a, int lg, int &j, int &k)
@@ -167,6 +190,8 @@ __device__ __forceinline__ void bind(FftArgs &a, const Fields &F, int f)
     a.coef = a.coef_mode == CHY_COEF_NONE ? nullptr : F.coef[f];
 }
 
+constexpr int kCoefOrders = 2;  // COEF's orders at a time per thread
+
 // Phase 3 of the forward transform, shared by both kernel families: the real
 // split X_m = E_m + e^{2 pi i m/L} O_m of the complex result Z in lds
 // ([element][lane], lane fastest), then the ring moments, the spectrum and
@@ -175,7 +200,7 @@ __device__ __forceinline__ void bind(FftArgs &a, const Fields &F, int f)
 template <typename TS>
 __device__ __forceinline__ void forward_outputs(const FftArgs &a, const double2 *lds, const double2 *tw, int N,
                                                 int NL, int NS, int lane, int sub, int j, int k, bool interior,
-                                                size_t base, size_t plane)
+                                                size_t base, size_t plane, int part, int parts)
 {
     // A_m = 2 Re X_m, B_m = 2 Im X_m
     auto xm = [&](int m) -> double2 {  // m = 0..N
@@ -214,36 +239,45 @@ __device__ __forceinline__ void forward_outputs(const FftArgs &a, const double2 
     TS *spec = static_cast<TS *>(a.spec);
     // interior lanes feed the mode right-hand side Y = 4 pi G PHI~ (pot3.f:212)
     const double ys = interior ? a.ys : 1.0;
-    double A0 = 0.0;
-    if (want_coef) A0 = 2.0 * xm(0).x;
     TS *sp = spec ? spec + sidx + (size_t)sub * JK : nullptr;
     const size_t step = JK * (size_t)NS, half = JK * (size_t)N;
-    for (int m = sub; m <= N; m += NS) {
-        const double2 X = xm(m);
-        const double A = 2.0 * X.x, B = 2.0 * X.y;
-        if (sp) {
-            sp[0] = (TS)(A * a.sf1 * ys);
-            if (m >= 1 && m <= N - 1) sp[half] = (TS)(B * a.sf1 * ys);
-            sp += step;
+    if (sp) {
+        TS *p = sp;
+        for (int m = sub; m <= N; m += NS, p += step) {
+            const double2 X = xm(m);
+            p[0] = (TS)(2.0 * X.x * a.sf1 * ys);
+            if (m >= 1 && m <= N - 1) p[half] = (TS)(2.0 * X.y * a.sf1 * ys);
         }
-        if (want_coef && m >= 1) {
-            // COEF(J,K,m,1) amplitude, COEF(J,K,m,2) phase (pot3.f:105-132)
-            const double x1 = fabs(A0);
-            double *c1 = a.coef + base + plane * (size_t)(m - 1);
-            double *c2 = c1 + plane * (size_t)N;
-            if (m < N) {
-                if (x1 != 0.0) *c1 = 2.0 * sqrt(A * A + B * B) / x1;
-                double philag;
-                if (A > 0.0) philag = atan(B / A);
-                else if (A < 0.0) philag = atan(B / A) + a.pi;
-                else if (B > 0.0) philag = 0.5 * a.pi;
-                else if (B < 0.0) philag = -0.5 * a.pi;
-                else philag = 4.0 * a.pi;
-                *c2 = philag * 180.0 / a.pi;
-            } else {
-                if (x1 != 0.0) *c1 = fabs(A) / x1;
-                *c2 = A0;
-            }
+    }
+    if (!want_coef) return;
+    // COEF(J,K,m,1) amplitude, COEF(J,K,m,2) phase (pot3.f:105-132), two
+    // orders at a time without branches (the chain of the square root, the
+    // divisions and the arc tangent takes 0.6 us)
+    const double A0 = 2.0 * xm(0).x, x1 = fabs(A0), two_x1 = 2.0 / x1, deg = 180.0 / a.pi;
+    const size_t cstep = plane * (size_t)NS, chalf = plane * (size_t)N;
+    constexpr int U = kCoefOrders;
+    for (int m0 = sub + part * U * NS; m0 <= N; m0 += parts * U * NS) {
+        double *c1 = a.coef + base + plane * (size_t)m0 - plane;
+        double A[U], B[U], amp[U], ph[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const double2 X = xm(min(m0 + u * NS, N));
+            A[u] = 2.0 * X.x;
+            B[u] = 2.0 * X.y;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            amp[u] = two_x1 * sqrt(A[u] * A[u] + B[u] * B[u]);
+            const double t = atan(B[u] / A[u]);
+            ph[u] = A[u] > 0.0 ? t : A[u] < 0.0 ? t + a.pi : B[u] > 0.0 ? 0.5 * a.pi : B[u] < 0.0 ? -0.5 * a.pi : 4.0 * a.pi;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int m = m0 + u * NS;
+            if (m < 1 || m > N) continue;
+            double *c = c1 + (size_t)u * cstep;
+            if (x1 != 0.0) c[0] = m < N ? amp[u] : fabs(A[u]) / x1;
+            c[chalf] = m < N ? ph[u] * deg : A0;
         }
     }
 }
@@ -318,7 +352,8 @@ __global__ __launch_bounds__(NL *N2) void k_fft_forward(FftArgs a, const Fields 
     const int tid = threadIdx.x;
     const int lane = tid % NL;
     const int sub = tid / NL;
-    const int chunk = xcd_chunk((a.nlanes + NL - 1) / NL);
+    int part, parts;
+    const int chunk = forward_chunk(a, NL, part, parts);
     if (chunk * NL >= a.nlanes) return;  // whole block
     const int lg = chunk * NL + lane;
     const bool active = lg < a.nlanes;
@@ -368,7 +403,7 @@ __global__ __launch_bounds__(NL *N2) void k_fft_forward(FftArgs a, const Fields 
     __syncthreads();
     if (!active) return;
 
-    forward_outputs<TS>(a, lds, tw, N, NL, N2, lane, sub, j, k, interior, base, plane);
+    forward_outputs<TS>(a, lds, tw, N, NL, N2, lane, sub, j, k, interior, base, plane, part, parts);
 }
 
 // TS: storage type of the spectrum.
@@ -384,7 +419,7 @@ __global__ __launch_bounds__(NL *N2) void k_fft_inverse(FftArgs a, const Fields 
     const int tid = threadIdx.x;
     const int lane = tid % NL;
     const int sub = tid / NL;
-    const int chunk = xcd_chunk((a.nlanes + NL - 1) / NL);
+    const int chunk = xcd_chunk((a.nlanes + NL - 1) / NL, (int)blockIdx.x);
     if (chunk * NL >= a.nlanes) return;  // whole block
     const int lg = chunk * NL + lane;
     const bool active = lg < a.nlanes;
@@ -596,7 +631,8 @@ __global__ __launch_bounds__(NL *NS) void k_fft_forward_mr(FftArgs a, const Fiel
     const int tid = threadIdx.x;
     const int lane = tid % NL;
     const int sub = tid / NL;
-    const int chunk = xcd_chunk((a.nlanes + NL - 1) / NL);
+    int part, parts;
+    const int chunk = forward_chunk(a, NL, part, parts);
     if (chunk * NL >= a.nlanes) return;  // whole block
     const int lg = chunk * NL + lane;
     const bool active = lg < a.nlanes;
@@ -622,7 +658,7 @@ __global__ __launch_bounds__(NL *NS) void k_fft_forward_mr(FftArgs a, const Fiel
     __syncthreads();
     const double2 *z = stockham<+1>(rp, buf, buf + N * NL, N, NL, NS, lane, sub, tw, a.tw64, L);
     if (!active) return;
-    forward_outputs<double>(a, z, tw, N, NL, NS, lane, sub, j, k, interior, base, plane);
+    forward_outputs<double>(a, z, tw, N, NL, NS, lane, sub, j, k, interior, base, plane, part, parts);
 }
 
 template <int NL, int NS, int NMAX>
@@ -635,7 +671,7 @@ __global__ __launch_bounds__(NL *NS) void k_fft_inverse_mr(FftArgs a, const Fiel
     const int tid = threadIdx.x;
     const int lane = tid % NL;
     const int sub = tid / NL;
-    const int chunk = xcd_chunk((a.nlanes + NL - 1) / NL);
+    const int chunk = xcd_chunk((a.nlanes + NL - 1) / NL, (int)blockIdx.x);
     if (chunk * NL >= a.nlanes) return;  // whole block
     const int lg = chunk * NL + lane;
     const bool active = lg < a.nlanes;
@@ -675,15 +711,35 @@ __global__ __launch_bounds__(NL *NS) void k_fft_inverse_mr(FftArgs a, const Fiel
     }
 }
 
+// Leading blocks for COEF (forward_chunk) where the launch leaves CUs idle: nl
+// lanes and ns threads per lane in a block.  A lane's orders are then spread over
+// as many blocks as give each thread one round of them (each repeats the lane's
+// transform): with COEF's K=2 plane formed by the blocks that hold its lanes,
+// those two worked on it for 9 us of a 65.4 us solve at 64x32x64 (56.5 so, 55.8
+// without COEF).
+int coef_split(FftArgs &a, const Fields &F, int ncu, int nl, int ns)
+{
+    a.coef_blocks = 0;
+    if (a.coef_mode == CHY_COEF_NONE || a.lanes == LANES_BOUNDARY) return 0;
+    const int chunks = (a.nlanes + nl - 1) / nl, row = a.lanes == LANES_ALL ? a.J : a.J - 1;
+    const int with = a.coef_mode == CHY_COEF_K2 ? (row + nl - 1) / nl : chunks;
+    const int parts = (a.L / 2 + 1 + kCoefOrders * ns - 1) / (kCoefOrders * ns);
+    if (parts < 2 || (long)(chunks + with * parts) * F.nf > ncu) return 0;
+    a.coef_parts = parts;
+    a.coef_blocks = (with * parts + kXcds - 1) / kXcds * kXcds;
+    return a.coef_blocks;
+}
+
 // transform variants (the refinement works in the spectrum and uses the
 // binary64 transforms)
 enum { FWD64 = 0, INV64 = 2 };
 
 template <int N1, int N2, int NL, int KIND>
-int launch_one(const FftArgs &a, const Fields &F, hipStream_t s)
+int launch_one(FftArgs a, const Fields &F, int ncu, hipStream_t s)
 {
     const int chunks = (a.nlanes + NL - 1) / NL;
-    const int blocks = (chunks + kXcds - 1) / kXcds * kXcds;
+    int blocks = (chunks + kXcds - 1) / kXcds * kXcds;
+    if (KIND == FWD64) blocks += coef_split(a, F, ncu, NL, N2);
     const dim3 grid(blocks, F.nf), block(NL * N2);
     if (KIND == FWD64) hipLaunchKernelGGL((k_fft_forward<N1, N2, NL, double, double>), grid, block, 0, s, a, F);
     if (KIND == INV64) hipLaunchKernelGGL((k_fft_inverse<N1, N2, NL, double>), grid, block, 0, s, a, F);
@@ -692,12 +748,13 @@ int launch_one(const FftArgs &a, const Fields &F, hipStream_t s)
 
 // mixed-radix sizes: NL lanes per block with N*NL <= 2048 (two buffers of up to 32 KB)
 template <int NL, int KIND>
-int launch_mr(const FftArgs &a, const Fields &F, const RadixPlan &rp, hipStream_t s)
+int launch_mr(FftArgs a, const Fields &F, int ncu, const RadixPlan &rp, hipStream_t s)
 {
     constexpr int NS = 256 / NL, NMAX = 2048 / NL;
     const size_t lds = sizeof(double2) * ((size_t)a.L * NL + a.L);
     const int chunks = (a.nlanes + NL - 1) / NL;
-    const int blocks = (chunks + kXcds - 1) / kXcds * kXcds;
+    int blocks = (chunks + kXcds - 1) / kXcds * kXcds;
+    if (KIND == FWD64) blocks += coef_split(a, F, ncu, NL, NS);
     const dim3 grid(blocks, F.nf), block(NL * NS);
     if (KIND == FWD64) hipLaunchKernelGGL((k_fft_forward_mr<NL, NS, NMAX>), grid, block, lds, s, a, F, rp);
     if (KIND == INV64) hipLaunchKernelGGL((k_fft_inverse_mr<NL, NS, NMAX>), grid, block, lds, s, a, F, rp);
@@ -710,10 +767,10 @@ int dispatch(int N, int ncu, const FftArgs &a, const Fields &F, hipStream_t s)
     if (N & (N - 1)) {
         RadixPlan rp;
         if (N > 512 || !radix_plan(N, rp)) return (int)hipErrorInvalidValue;
-        if (N <= 64) return launch_mr<32, KIND>(a, F, rp, s);
-        if (N <= 128) return launch_mr<16, KIND>(a, F, rp, s);
-        if (N <= 256) return launch_mr<8, KIND>(a, F, rp, s);
-        return launch_mr<4, KIND>(a, F, rp, s);
+        if (N <= 64) return launch_mr<32, KIND>(a, F, ncu, rp, s);
+        if (N <= 128) return launch_mr<16, KIND>(a, F, ncu, rp, s);
+        if (N <= 256) return launch_mr<8, KIND>(a, F, ncu, rp, s);
+        return launch_mr<4, KIND>(a, F, ncu, rp, s);
     }
     // Fewer lanes per block (a quarter, a half at N = 128, where pieces of 8
     // lanes per plane cost more than they give) where the usual blocks fill
@@ -723,24 +780,24 @@ int dispatch(int N, int ncu, const FftArgs &a, const Fields &F, hipStream_t s)
     const int usual = N >= 16 && N <= 128 ? 4096 / N : 1;  // lanes per block below
     if ((long)((a.nlanes + usual - 1) / usual) * F.nf < ncu / 2) {
         switch (N) {
-        case 16: return launch_one<16, 1, 64, KIND>(a, F, s);
-        case 32: return launch_one<16, 2, 32, KIND>(a, F, s);
-        case 64: return launch_one<16, 4, 16, KIND>(a, F, s);
-        case 128: return launch_one<16, 8, 16, KIND>(a, F, s);
+        case 16: return launch_one<16, 1, 64, KIND>(a, F, ncu, s);
+        case 32: return launch_one<16, 2, 32, KIND>(a, F, ncu, s);
+        case 64: return launch_one<16, 4, 16, KIND>(a, F, ncu, s);
+        case 128: return launch_one<16, 8, 16, KIND>(a, F, ncu, s);
         default: break;
         }
     }
     switch (N) {
-    case 1: return launch_one<1, 1, 256, KIND>(a, F, s);
-    case 2: return launch_one<2, 1, 256, KIND>(a, F, s);
-    case 4: return launch_one<4, 1, 256, KIND>(a, F, s);
-    case 8: return launch_one<8, 1, 256, KIND>(a, F, s);
-    case 16: return launch_one<16, 1, 256, KIND>(a, F, s);
-    case 32: return launch_one<16, 2, 128, KIND>(a, F, s);
-    case 64: return launch_one<16, 4, 64, KIND>(a, F, s);
-    case 128: return launch_one<16, 8, 32, KIND>(a, F, s);
-    case 256: return launch_one<16, 16, 16, KIND>(a, F, s);
-    case 512: return launch_one<32, 16, 8, KIND>(a, F, s);
+    case 1: return launch_one<1, 1, 256, KIND>(a, F, ncu, s);
+    case 2: return launch_one<2, 1, 256, KIND>(a, F, ncu, s);
+    case 4: return launch_one<4, 1, 256, KIND>(a, F, ncu, s);
+    case 8: return launch_one<8, 1, 256, KIND>(a, F, ncu, s);
+    case 16: return launch_one<16, 1, 256, KIND>(a, F, ncu, s);
+    case 32: return launch_one<16, 2, 128, KIND>(a, F, ncu, s);
+    case 64: return launch_one<16, 4, 64, KIND>(a, F, ncu, s);
+    case 128: return launch_one<16, 8, 32, KIND>(a, F, ncu, s);
+    case 256: return launch_one<16, 16, 16, KIND>(a, F, ncu, s);
+    case 512: return launch_one<32, 16, 8, KIND>(a, F, ncu, s);
     default: return (int)hipErrorInvalidValue;
     }
 }
