@@ -390,24 +390,22 @@ void launch_leaf(const CrPhase &ph, const chy_grid *g, const CrArgs &a, const Fi
         hipLaunchKernelGGL((k_cr_leaf<R, G, W, true>), grid, dim3(64 * W), 0, s, a, F, run);
 }
 
-// One launch per phase.  Wavefronts per node: two rounds of 64/G roots each, at
-// most 4: a level of 16-23 (23-29, 21) roots takes 250/265 (144/154, 71) us up
-// and down per 32 fields at 256x128x256 with 4 or 2, and alone 14 (12, 10) us
-// with 4 but 20 (19, 16) with 2.
+// One launch per phase, a node on 4 wavefronts (2 where 8 lanes take a system):
+// 256x128x256's levels of 16-23, 23-29 and 21 roots take 250/265, 144/154 and 71
+// us up and down per 32 fields with 4 or 2, and alone 14, 12 and 10 us with 4
+// but 20, 19 and 16 with 2; two rounds of roots on fewer wavefronts took
+// 64x128x64 and 128x32x64 from 83.5 and 56.8 to 87.8 and 58.8 us alone, and no
+// less per field of a batch.  (8 wavefronts: the top node 8 us alone, 105 per 32
+// fields.  The count does not depend on the number of fields, as it orders
+// the sums.)
 template <int R, int G>
 int launch_phases(const chy_grid *g, const CrArgs &a, const Fields &F, hipStream_t s)
 {
-    constexpr int SPW = 64 / G;
     for (const CrPhase &ph : g->cr.phases) {
         if (ph.kind == CR_LEAF_UP || ph.kind == CR_LEAF_DOWN) {
             launch_leaf<R, G>(ph, g, a, F, s);
         } else {
-            switch (std::min(4, ph.np / (2 * SPW))) {
-            case 0:
-            case 1: launch_node<R, G, 1>(ph, a, F, s); break;
-            case 2: launch_node<R, G, 2>(ph, a, F, s); break;
-            default: launch_node<R, G, 4>(ph, a, F, s); break;
-            }
+            launch_node<R, G, G == 8 ? 2 : 4>(ph, a, F, s);
         }
     }
     return (int)hipGetLastError();
