@@ -1203,7 +1203,11 @@ int chy_source_grav(chy_ctx *ctx, const chy_source_desc *d, const double *r_d, c
     if (d->jstart < 2 || d->jstart > d->jmax + 1) return CHY_EINVAL;
     if (!(d->dr > 0.0) || !(d->dz > 0.0) || !(d->dtheta > 0.0)) return CHY_EINVAL;
     DeviceScope ds(ctx->device);
-    return dev_rc(launch_source_grav(d, r_d, rho_d, omega_d, phi_d, p_d, s_d, t_d, a_d, ctx->stream),
+    int ncu = 0;
+    const int rc = dev_rc((int)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, ctx->device),
+                          "hipDeviceGetAttribute");
+    if (rc) return rc;
+    return dev_rc(launch_source_grav(d, r_d, rho_d, omega_d, phi_d, p_d, s_d, t_d, a_d, ncu, ctx->stream),
                   "SOURCE launch");
 }
 

@@ -361,7 +361,7 @@ int launch_find_force(const chy_force_desc *d, const double *rhf, const double *
                       const double *rho, double x, double y, double *part, double *out, hipStream_t st);
 // The momentum sources of radhydro/source.f:41-79 (arguments checked by the caller).
 int launch_source_grav(const chy_source_desc *d, const double *r, const double *rho, const double *omega,
-                       const double *phi, const double *p, double *s, double *t, double *a, hipStream_t st);
+                       const double *phi, const double *p, double *s, double *t, double *a, int ncu, hipStream_t st);
 
 void set_device_error(hipError_t e, const char *where);
 

@@ -43,10 +43,10 @@ constexpr int kRawWord3 = 0x00020000;
 constexpr unsigned kDropOffset = 0x80000000u;
 typedef unsigned int ux2 __attribute__((ext_vector_type(2)));
 
-constexpr int SRC_KC = 16;  // K rows per thread
+constexpr int SRC_KC = 16;  // K rows per thread, at most
 constexpr int SRC_LB = 8;   // L planes per block
 
-__global__ __launch_bounds__(64 * SRC_LB) void k_source_grav(SourceArgs a, int nbx, int nby, int nblocks)
+__global__ __launch_bounds__(64 * SRC_LB) void k_source_grav(SourceArgs a, int nbx, int nby, int nblocks, int kc)
 {
 #pragma clang fp contract(off)
     // Blocks are handed to the 8 XCDs in turn (block b to XCD b % 8); tile
@@ -58,9 +58,9 @@ __global__ __launch_bounds__(64 * SRC_LB) void k_source_grav(SourceArgs a, int n
     const int bx = tile % nbx, by = (tile / nbx) % nby, bz = tile / (nbx * nby);
     const int J = a.jstart + bx * 64 + (int)threadIdx.x;  // Fortran indices
     const int L = 1 + by * SRC_LB + (int)threadIdx.y;
-    const int K0 = 2 + bz * SRC_KC;
+    const int K0 = 2 + bz * kc;
     if (J > a.jmax1 || L > a.lmax) return;
-    const int K1 = min(K0 + SRC_KC - 1, a.kmax + 1);
+    const int K1 = min(K0 + kc - 1, a.kmax + 1);
     const int LM = L == 1 ? a.lmax : L - 1;
     const int LP = L == a.lmax ? 1 : L + 1;
     const size_t hp = (size_t)a.j2 * a.k2, pp = (size_t)a.pj2 * a.pk2;
@@ -145,7 +145,7 @@ __global__ __launch_bounds__(64 * SRC_LB) void k_source_grav(SourceArgs a, int n
 }  // namespace
 
 int launch_source_grav(const chy_source_desc *d, const double *r, const double *rho, const double *omega,
-                       const double *phi, const double *p, double *s, double *t, double *a, hipStream_t st)
+                       const double *phi, const double *p, double *s, double *t, double *a, int ncu, hipStream_t st)
 {
     SourceArgs x{};
     x.r = r; x.rho = rho; x.omega = omega; x.phi = phi; x.p = p;
@@ -155,9 +155,14 @@ int launch_source_grav(const chy_source_desc *d, const double *r, const double *
     x.jstart = d->jstart; x.jmax1 = d->jmax + 1; x.kmax = d->kmax; x.lmax = d->lmax;
     x.delt = d->delt; x.dr = d->dr; x.dz = d->dz; x.dtheta = d->dtheta;
     const int nj = x.jmax1 - x.jstart + 1;
-    const int nbx = (nj + 63) / 64, nby = (d->lmax + SRC_LB - 1) / SRC_LB, nbz = (d->kmax + SRC_KC - 1) / SRC_KC;
-    const int nblocks = nbx * nby * nbz;
-    hipLaunchKernelGGL(k_source_grav, dim3(nblocks), dim3(64, SRC_LB), 0, st, x, nbx, nby, nblocks);
+    const int nbx = (nj + 63) / 64, nby = (d->lmax + SRC_LB - 1) / SRC_LB;
+    // fewer rows per thread where the grid would leave CUs idle: a thread's rows
+    // are a chain of loads (16 each: 15-18 us up to 128x64x128; now 4.4 us at
+    // 24x16x32, 5.0 at 64x32x64, 16 at 128x64x128, whose arrays take as long)
+    int kc = SRC_KC;
+    while (kc > 1 && (long)nbx * nby * ((d->kmax + kc - 1) / kc) < 2 * ncu) kc /= 2;
+    const int nblocks = nbx * nby * ((d->kmax + kc - 1) / kc);
+    hipLaunchKernelGGL(k_source_grav, dim3(nblocks), dim3(64, SRC_LB), 0, st, x, nbx, nby, nblocks, kc);
     return (int)hipGetLastError();
 }
 
