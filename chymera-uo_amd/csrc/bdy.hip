@@ -62,12 +62,13 @@ __device__ __forceinline__ void bind(BdyArgs &a, const Fields &F, int f)
 // chunk[0][2t+s][c]: sum over chunk c's rings of TERM_t * moment_s (inside
 // form), chunk[1][2t+s][c]: the same with TERM_t r^-(2l+1) (outside form);
 // s=0 cosine (SUMASS for m=0), s=1 sine.
-// blockIdx.x is the field and blockIdx.y the chunk, so the fields' blocks of
-// one chunk run together and share the chunk's rows of the grid's tables
-// (TERM, r) in L2 instead of each field streaming the whole tables again.
-__global__ __launch_bounds__(256) void k_bdy_chunks(BdyArgs a, const Fields F)
+// blockIdx.y is the chunk and blockIdx.x a run of per_block fields, so the
+// fields' blocks of one chunk run together and share the chunk's rows of the
+// grid's tables (TERM, r) in L2, and the fields of a block in registers: with
+// a block per field the tables were three quarters of what went through the L2
+// (32 fields at 256x128x256 178 us, 136 with two fields per block, 110 with eight).
+__global__ __launch_bounds__(256) void k_bdy_chunks(BdyArgs a, const Fields F, int per_block)
 {
-    bind(a, F, blockIdx.x);
     constexpr int IT = (kChunkRings + CHUNK_GROUPS - 1) / CHUNK_GROUPS;  // rings per thread
     __shared__ double smom[kChunkRings][kMoments + 1];
     __shared__ double part[CHUNK_GROUPS][kMaxTerms][4];
@@ -88,7 +89,7 @@ __global__ __launch_bounds__(256) void k_bdy_chunks(BdyArgs a, const Fields F)
     }
     // ... and the moments of the block's rings (ring order in memory, radius
     // order in LDS): positions, then ring indices, then moments, each step's
-    // loads all issued before any is used
+    // loads all issued before any is used, the next field's while this one is summed
     constexpr int GPER = (kChunkRings * kMoments + 255) / 256;
     const int ne = (p1 - p0) * kMoments;
     int gr[GPER];
@@ -98,46 +99,55 @@ __global__ __launch_bounds__(256) void k_bdy_chunks(BdyArgs a, const Fields F)
         gr[i] = a.ring_of_pos[p0 + (v < ne ? v / kMoments : 0)];
     }
     double gm[GPER];
+    auto fetch = [&](int f) {
+        const double *mom = F.mom[f];
 #pragma unroll
-    for (int i = 0; i < GPER; ++i) {
-        const int v = tid + 256 * i;
-        gm[i] = a.mom[(size_t)gr[i] * kMoments + (v < ne ? v % kMoments : 0)];
-    }
-#pragma unroll
-    for (int i = 0; i < GPER; ++i) {
-        const int v = tid + 256 * i;
-        if (v < ne) smom[v / kMoments][v % kMoments] = gm[i];
-    }
-    __syncthreads();
-    if (worker) {
-        const int m = kTermM[t];
-        double ic = 0.0, is = 0.0, oc = 0.0, os = 0.0;
-#pragma unroll
-        for (int it = 0; it < IT; ++it) {
-            const int r = grp + CHUNK_GROUPS * it;
-            // rings beyond REDGE are skipped (boundary.f:379)
-            const bool use = t < a.nt && p0 + r < p1 && !(a.redge > 0.0 && rs[it] > a.redge);
-            const int rr = use ? r : 0;
-            const double mc = smom[rr][m];                       // SUMASS (m=0) or CM(m)
-            const double ms = m == 0 ? 0.0 : smom[rr][10 + m];   // SM(m)
-            ic = use ? fma(ti[it], mc, ic) : ic;
-            is = use ? fma(ti[it], ms, is) : is;
-            oc = use ? fma(to[it], mc, oc) : oc;
-            os = use ? fma(to[it], ms, os) : os;
+        for (int i = 0; i < GPER; ++i) {
+            const int v = tid + 256 * i;
+            gm[i] = mom[(size_t)gr[i] * kMoments + (v < ne ? v % kMoments : 0)];
         }
-        part[grp][t][0] = ic;
-        part[grp][t][1] = is;
-        part[grp][t][2] = oc;
-        part[grp][t][3] = os;
-    }
-    __syncthreads();
-    if (tid < kMaxTerms * 4) {
-        const int tt = tid / 4, v = tid % 4;
-        double sum = 0.0;
+    };
+    const int f0 = (int)blockIdx.x * per_block, f1 = min(f0 + per_block, F.nf);
+    fetch(f0);
+#pragma unroll 1
+    for (int f = f0; f < f1; ++f) {
 #pragma unroll
-        for (int g2 = 0; g2 < CHUNK_GROUPS; ++g2) sum += part[g2][tt][v];
-        const int comp = v >> 1, cs = v & 1;
-        a.chunk[((size_t)comp * NCOL + 2 * tt + cs) * a.nchunk + c] = sum;
+        for (int i = 0; i < GPER; ++i) {
+            const int v = tid + 256 * i;
+            if (v < ne) smom[v / kMoments][v % kMoments] = gm[i];
+        }
+        __syncthreads();
+        if (f + 1 < f1) fetch(f + 1);
+        if (worker) {
+            const int m = kTermM[t];
+            double ic = 0.0, is = 0.0, oc = 0.0, os = 0.0;
+#pragma unroll
+            for (int it = 0; it < IT; ++it) {
+                const int r = grp + CHUNK_GROUPS * it;
+                // rings beyond REDGE are skipped (boundary.f:379)
+                const bool use = t < a.nt && p0 + r < p1 && !(a.redge > 0.0 && rs[it] > a.redge);
+                const int rr = use ? r : 0;
+                const double mc = smom[rr][m];                       // SUMASS (m=0) or CM(m)
+                const double ms = m == 0 ? 0.0 : smom[rr][10 + m];   // SM(m)
+                ic = use ? fma(ti[it], mc, ic) : ic;
+                is = use ? fma(ti[it], ms, is) : is;
+                oc = use ? fma(to[it], mc, oc) : oc;
+                os = use ? fma(to[it], ms, os) : os;
+            }
+            part[grp][t][0] = ic;
+            part[grp][t][1] = is;
+            part[grp][t][2] = oc;
+            part[grp][t][3] = os;
+        }
+        __syncthreads();
+        if (tid < kMaxTerms * 4) {
+            const int tt = tid / 4, v = tid % 4;
+            double sum = 0.0;
+#pragma unroll
+            for (int g2 = 0; g2 < CHUNK_GROUPS; ++g2) sum += part[g2][tt][v];
+            const int comp = v >> 1, cs = v & 1;
+            F.chunk[f][((size_t)comp * NCOL + 2 * tt + cs) * a.nchunk + c] = sum;
+        }
     }
 }
 
@@ -446,7 +456,12 @@ int launch_bdygen_from_moments_f(const chy_grid *g, const Fields &F, int maxtrm,
     a.redge = redge; a.grav = g->grav; a.pi = g->pi;
     a.cnmax = g->cnmax; a.cmmax = g->cmmax;
     const int nf = F.nf;
-    hipLaunchKernelGGL(k_bdy_chunks, dim3(nf, g->nchunk), dim3(256), 0, s, a, F);
+    int per_block = 1;  // as many as leave four blocks per CU
+    while (per_block < 8 && 2 * per_block <= nf &&
+           (long)((nf + 2 * per_block - 1) / (2 * per_block)) * g->nchunk >= 4 * g->ncu)
+        per_block *= 2;
+    hipLaunchKernelGGL(k_bdy_chunks, dim3((nf + per_block - 1) / per_block, g->nchunk), dim3(256), 0, s, a, F,
+                       per_block);
     hipLaunchKernelGGL(k_bdy_scan, dim3(2 * NCOL, nf), dim3(256), 0, s, a, F);
     if (spectral) {
         hipLaunchKernelGGL(k_bdy_spec, dim3(g->jkmax, nf), dim3(256), 0, s, a, F, g->d.twh, coef_mode, 1);
