@@ -74,17 +74,17 @@ struct Plane {
     }
 };
 
-// The sums of a node's block (one or two, two parts each): every lane holds
-// its root group's share; the W * 64/G shares of one part at a time meet in LDS
-// and are added in order, out(sum, part, j, value) for j < M.  (Adding the
-// groups of a wavefront by lane exchanges first cost 300 instructions per
-// wavefront, two thirds of a solve.)
+// The sums of a node (one or two, two parts each) by its team of W wavefronts
+// (tid: thread of the team): every lane holds its root group's share; the
+// W * 64/G shares of one part at a time meet in LDS and are added in order,
+// out(sum, part, j, value) for j < M.  (Adding the groups of a wavefront by lane
+// exchanges first cost 300 instructions per wavefront, two thirds of a solve.)
 template <int R, int G, int W, int NSUM, typename Out>
-__device__ __forceinline__ void block_sums(const double (&s)[NSUM][2][R], double *lds, int M, Out out)
+__device__ __forceinline__ void team_sums(const double (&s)[NSUM][2][R], double *lds, int tid, int M, Out out)
 {
     typedef Vec<R, G> V;
     constexpr int SLOTS = W * 64 / G;
-    const int slot = threadIdx.x / G, gl = threadIdx.x % G;
+    const int slot = tid / G, gl = tid % G;
 #pragma unroll
     for (int n = 0; n < NSUM; ++n) {
 #pragma unroll
@@ -93,7 +93,7 @@ __device__ __forceinline__ void block_sums(const double (&s)[NSUM][2][R], double
 #pragma unroll
             for (int r = 0; r < R; ++r) lds[slot * V::SIZE + r * V::PITCH + gl] = s[n][h][r];
             __syncthreads();
-            for (int j = threadIdx.x; j < R * G; j += 64 * W) {
+            for (int j = tid; j < R * G; j += 64 * W) {
                 const double *p = lds + V::at(j);
                 double v = p[0];
 #pragma unroll
@@ -265,34 +265,46 @@ __global__ __launch_bounds__(64 * W, 2) void k_cr_leaf(CrArgs a, const Fields F,
 }
 
 // A node of the tree: row i = (2 n + 1) h (1-based) with its block of 2h - 1
-// rows; the roots are dealt to the block's W wavefronts in turn.  Its
+// rows; the roots are dealt to the team's W wavefronts in turn.  Its
 // right-hand side is the spectrum's row plus the messages from its right (the
 // second buffer's row) and from its left (the row before).  With two or three
 // rounds of solves a block's loads, barriers and sums take as long as its
 // solves; LDS holds one vector per root in flight (24 KB, six blocks per CU)
 // and the sums' parts pass through it one after another (both at once, 41 KB
 // and three blocks: 272 instead of 250 us for the lowest level up).
-template <int R, int G, int W, bool DOWN>
-__global__ __launch_bounds__(64 * W, R == 8 ? 3 : 4) void k_cr_node(CrArgs a, const Fields F, CrPhase ph)
+template <int R, int G>
+struct Node {
+    // wavefronts: 256x128x256's levels of 16-23, 23-29 and 21 roots take 250/265,
+    // 144/154 and 71 us up and down per 32 fields with 4 or 2, and alone 14, 12
+    // and 10 us with 4 but 20, 19 and 16 with 2; two rounds of roots on fewer
+    // wavefronts took 64x128x64 and 128x32x64 from 83.5 and 56.8 to 87.8 and 58.8
+    // us alone, and no less per field of a batch.  (8 wavefronts: the top node 8
+    // us alone, 105 per 32 fields.  The count does not depend on the number of
+    // fields, as it orders the sums.)
+    static constexpr int W = G == 8 ? 2 : 4;
+    static constexpr int VECTORS(bool down) { return W * 64 / G > (down ? 6 : 2) ? W * 64 / G : down ? 6 : 2; }
+};
+
+// (n past the level's nodes: nothing is stored)
+template <int R, int G, bool DOWN>
+__device__ __forceinline__ void node_run(const CrArgs &a, const Plane<R, G> &q, const CrPhase &ph, double *lds,
+                                         const double *tri, int tid, int n)
 {
     typedef Vec<R, G> V;
-    constexpr int SPW = 64 / G, JP = R * G, NIN = DOWN ? 3 : 1, NSUM = DOWN ? 1 : 2;
-    constexpr int NV = 2 * NIN > W * SPW ? 2 * NIN : W * SPW;
-    __shared__ double lds[NV * V::SIZE], tri[3 * V::SIZE];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int W = Node<R, G>::W, SPW = 64 / G, JP = R * G, NIN = DOWN ? 3 : 1, NSUM = DOWN ? 1 : 2;
+    const int lane = tid & 63, wave = tid >> 6;
     const int gl = lane % G, sub = lane / G;
-    const int m = (int)blockIdx.x / ph.nnode, n = (int)blockIdx.x % ph.nnode;
+    const bool real = n < ph.nnode;
     const int h = ph.h, M = a.M;
+    n = min(n, ph.nnode - 1);
     const int i = (2 * n + 1) * h - 1;          // this row, 0-based
     const bool left = n > 0, right = n + 1 < ph.nnode;
-    const Plane<R, G> q(a, F, m);
-
     const double *rec = a.node + ((size_t)ph.rec0 + (size_t)n * (1 + ph.np)) * kNodeRec;
-    const int np = (int)rec[0];
+    const int np = real ? (int)rec[0] : 0;
     rec += (1 + sub) * kNodeRec;
 
     // the node's right-hand side and (down) the solved rows beside it
-    for (int e = threadIdx.x; e < NIN * 2 * JP; e += 64 * W) {
+    for (int e = tid; e < NIN * 2 * JP; e += 64 * W) {
         const int j = e % JP, c = (e / JP) % 2, w = e / (2 * JP);
         double v = 0.0;
         if (j < M && (c == 0 || q.two)) {
@@ -302,7 +314,6 @@ __global__ __launch_bounds__(64 * W, R == 8 ? 3 : 4) void k_cr_node(CrArgs a, co
         }
         lds[(w * 2 + c) * V::SIZE + V::at(j)] = v;
     }
-    rtri_load<R, G>(tri, a.am, a.cm, a.bm + (size_t)m * a.JP, M, 64 * W);
     const Neigh at = neighbours<G>(lane);
     __syncthreads();
 
@@ -346,8 +357,8 @@ __global__ __launch_bounds__(64 * W, R == 8 ? 3 : 4) void k_cr_node(CrArgs a, co
         }
         rt = rt_next;
     }
-    block_sums<R, G, W, NSUM>(s, lds, M, [&](int t, int c, int j, double v) {
-        if (c == 1 && !q.two) return;
+    team_sums<R, G, W, NSUM>(s, lds, tid, M, [&](int t, int c, int j, double v) {
+        if (!real || (c == 1 && !q.two)) return;
         if constexpr (DOWN) {
             (c ? q.ss : q.sc)[(size_t)i * a.J + j] = v;
         } else if (t == 0) {
@@ -358,14 +369,39 @@ __global__ __launch_bounds__(64 * W, R == 8 ? 3 : 4) void k_cr_node(CrArgs a, co
     });
 }
 
-template <int R, int G, int W>
-void launch_node(const CrPhase &ph, const CrArgs &a, const Fields &F, hipStream_t s)
+template <int R, int G, bool DOWN>
+__global__ __launch_bounds__((64 * Node<R, G>::W), R == 8 ? 3 : 4) void k_cr_node(CrArgs a, const Fields F, CrPhase ph)
 {
-    const dim3 grid((unsigned)((a.N + 1) * ph.nnode), F.nf);
-    if (ph.kind == CR_NODE_DOWN)
-        hipLaunchKernelGGL((k_cr_node<R, G, W, true>), grid, dim3(64 * W), 0, s, a, F, ph);
-    else
-        hipLaunchKernelGGL((k_cr_node<R, G, W, false>), grid, dim3(64 * W), 0, s, a, F, ph);
+    __shared__ double lds[Node<R, G>::VECTORS(DOWN) * Vec<R, G>::SIZE], tri[3 * Vec<R, G>::SIZE];
+    const int m = (int)blockIdx.x / ph.nnode;
+    const Plane<R, G> q(a, F, m);
+    rtri_load<R, G>(tri, a.am, a.cm, a.bm + (size_t)m * a.JP, a.M, 64 * Node<R, G>::W);
+    node_run<R, G, DOWN>(a, q, ph, lds, tri, threadIdx.x, (int)blockIdx.x % ph.nnode);
+}
+
+// The two highest levels, up, down and down again, by one block per order (two
+// teams, one of which the top node leaves idle): one launch instead of three for
+// launches too small to fill the chip.  What one phase leaves for the next lies
+// in global memory, written and read by the same block across a barrier.  The
+// teams are those of k_cr_node: the same results bit for bit.  One field at
+// 256x128x256 29.4 us, 33.8 in three launches (the solve 237 -> 232); with orders
+// past one per CU it is no faster (two fields 54.8 and 45.3, 32 fields 499 and
+// 370).  (The same for the whole tree, leaves and all: 153 us, 129 in its seven
+// launches; a CU's 8 wavefronts do not hide the solves' latency.)
+template <int R, int G>
+__global__ __launch_bounds__((128 * Node<R, G>::W)) void k_cr_top(CrArgs a, const Fields F, CrPhase second, CrPhase top)
+{
+    typedef Node<R, G> D;
+    constexpr int SIZE = D::VECTORS(true) * Vec<R, G>::SIZE;
+    __shared__ double lds[2 * SIZE], tri[3 * Vec<R, G>::SIZE];
+    const int team = threadIdx.x / (64 * D::W), tid = threadIdx.x % (64 * D::W);
+    const Plane<R, G> q(a, F, (int)blockIdx.x);
+    rtri_load<R, G>(tri, a.am, a.cm, a.bm + (size_t)blockIdx.x * a.JP, a.M, 128 * D::W);
+    node_run<R, G, false>(a, q, second, lds + team * SIZE, tri, tid, team);
+    __syncthreads();
+    node_run<R, G, true>(a, q, top, lds + team * SIZE, tri, tid, team);
+    __syncthreads();
+    node_run<R, G, true>(a, q, second, lds + team * SIZE, tri, tid, team);
 }
 
 template <int R, int G>
@@ -390,22 +426,25 @@ void launch_leaf(const CrPhase &ph, const chy_grid *g, const CrArgs &a, const Fi
         hipLaunchKernelGGL((k_cr_leaf<R, G, W, true>), grid, dim3(64 * W), 0, s, a, F, run);
 }
 
-// One launch per phase, a node on 4 wavefronts (2 where 8 lanes take a system):
-// 256x128x256's levels of 16-23, 23-29 and 21 roots take 250/265, 144/154 and 71
-// us up and down per 32 fields with 4 or 2, and alone 14, 12 and 10 us with 4
-// but 20, 19 and 16 with 2; two rounds of roots on fewer wavefronts took
-// 64x128x64 and 128x32x64 from 83.5 and 56.8 to 87.8 and 58.8 us alone, and no
-// less per field of a batch.  (8 wavefronts: the top node 8 us alone, 105 per 32
-// fields.  The count does not depend on the number of fields, as it orders
-// the sums.)
+// One launch per phase, or one for the three highest.
 template <int R, int G>
 int launch_phases(const chy_grid *g, const CrArgs &a, const Fields &F, hipStream_t s)
 {
-    for (const CrPhase &ph : g->cr.phases) {
-        if (ph.kind == CR_LEAF_UP || ph.kind == CR_LEAF_DOWN) {
-            launch_leaf<R, G>(ph, g, a, F, s);
+    const std::vector<CrPhase> &ph = g->cr.phases;
+    // first: the last level up, before the top and the way down from it
+    const size_t levels = (ph.size() - 1) / 2, first = levels - 1;
+    const bool fuse = levels >= 2 && (long)(g->N + 1) * F.nf <= g->ncu;
+    for (size_t i = 0; i < ph.size(); ++i) {
+        const dim3 grid((unsigned)((a.N + 1) * ph[i].nnode), F.nf), block(64 * Node<R, G>::W);
+        if (ph[i].kind == CR_LEAF_UP || ph[i].kind == CR_LEAF_DOWN) {
+            launch_leaf<R, G>(ph[i], g, a, F, s);
+        } else if (fuse && i == first) {
+            hipLaunchKernelGGL((k_cr_top<R, G>), dim3(g->N + 1, F.nf), dim3(2 * block.x), 0, s, a, F, ph[i], ph[i + 1]);
+            i += 2;
+        } else if (ph[i].kind == CR_NODE_DOWN) {
+            hipLaunchKernelGGL((k_cr_node<R, G, true>), grid, block, 0, s, a, F, ph[i]);
         } else {
-            launch_node<R, G, G == 8 ? 2 : 4>(ph, a, F, s);
+            hipLaunchKernelGGL((k_cr_node<R, G, false>), grid, block, 0, s, a, F, ph[i]);
         }
     }
     return (int)hipGetLastError();
