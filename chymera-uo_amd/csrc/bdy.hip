@@ -19,8 +19,7 @@
 //                  chunk boundaries include every boundary point's split, so
 //                  MASSIN/MASSOUT of a point are one entry each
 //   k_bdy_eval     TRMTOT and PHI at the boundary points for all L
-//                  (boundary.f:659-830)
-//   k_bdy_ghosts   ISYM=2 ghosts (boundary.f:876-893)
+//                  (boundary.f:659-830) and the ISYM=2 ghosts (:876-893)
 // Every reduction has a fixed order that depends on the grid only, so the
 // result does not depend on what else runs on the device.
 #include "chypot_impl.h"
@@ -246,6 +245,7 @@ __global__ __launch_bounds__(256) void k_bdy_eval(BdyArgs a, const Fields F)
     __syncthreads();
     const size_t plane = (size_t)a.JS * a.KS;
     const size_t pbase = (size_t)(a.jpos[jk] - 1) + (size_t)a.JS * (a.kpos[jk] - 1);
+    const bool below = a.jpos[jk] == a.J + 1 && a.kpos[jk] == 2, across = a.jpos[jk] == 2 && a.kpos[jk] == a.K + 1;
     for (int l = tid; l < a.L; l += blockDim.x) {
         double cr[10], sr[10];
 #pragma unroll
@@ -261,7 +261,12 @@ __global__ __launch_bounds__(256) void k_bdy_eval(BdyArgs a, const Fields F)
             if (kTermM[t] == 0) sum += t1[t];
             else sum += 2.0 * (cr[kTermM[t] - 1] * t1[t] + sr[kTermM[t] - 1] * t2[t]);
         }
-        a.phi[pbase + plane * l] = -a.grav * sum;
+        const double v = -a.grav * sum;
+        a.phi[pbase + plane * l] = v;
+        // the ISYM=2 ghosts (boundary.f:876-893): PHI(JMAX+1,1,L) = PHI(JMAX+1,2,L)
+        // and PHI(1,KMAX+1,L) = PHI(2,KMAX+1,L+-LMAX/2)
+        if (below) a.phi[pbase - a.JS + plane * l] = v;
+        if (across) a.phi[pbase - 1 + plane * (l < a.L / 2 ? l + a.L / 2 : l - a.L / 2)] = v;
     }
 }
 
@@ -424,21 +429,6 @@ __global__ __launch_bounds__(256) void k_bdy_spec(BdyArgs a, const Fields F, con
     }
 }
 
-__global__ __launch_bounds__(256) void k_bdy_ghosts(BdyArgs a, const Fields F)
-{
-    bind(a, F, blockIdx.y);
-    const int l = blockIdx.x * blockDim.x + threadIdx.x;
-    if (l >= a.L) return;
-    const size_t plane = (size_t)a.JS * a.KS;
-    const int n = a.L / 2;
-    // PHI(JMAX+1,1,LL) = PHI(JMAX+1,2,LL)
-    a.phi[(size_t)a.J + plane * l] = a.phi[(size_t)a.J + (size_t)a.JS + plane * l];
-    // PHI(1,KMAX+1,LL) = PHI(2,KMAX+1,LL+-LMAX/2)
-    const int lp = l < n ? l + n : l - n;
-    const size_t rowk = (size_t)a.JS * a.K;
-    a.phi[rowk + plane * l] = a.phi[rowk + 1 + plane * lp];
-}
-
 }  // namespace
 
 bool bdygen_spectral_ok(const chy_grid *g) { return g->L / 2 > kMaxTrm; }
@@ -471,7 +461,6 @@ int launch_bdygen_from_moments_f(const chy_grid *g, const Fields &F, int maxtrm,
         hipLaunchKernelGGL(k_bdy_spec, dim3(g->jkmax, nf), dim3(256), 0, s, a, F, g->d.twh, coef_mode, 1);
     } else {
         hipLaunchKernelGGL(k_bdy_eval, dim3(g->jkmax, nf), dim3(256), 0, s, a, F);
-        hipLaunchKernelGGL(k_bdy_ghosts, dim3((g->L + 255) / 256, nf), dim3(256), 0, s, a, F);
     }
     return (int)hipGetLastError();
 }
