@@ -24,6 +24,8 @@
 // LDS (layout [element][lane], lane fastest: conflict-free), then N2-point
 // DFTs in registers, then the real-split post-pass.  All twiddles are tables of
 // exact angles.
+#include <algorithm>
+
 #include "chypot_impl.h"
 
 namespace chy {
@@ -95,25 +97,53 @@ struct RadixPlan {
     int radix[kMaxPasses];
 };
 
-// the power-of-two part of N in passes of 16 (and one of 2, 4 or 8), then
-// each odd prime factor; false if N has a prime factor above 23
+// N's odd prime factors, each 3 or 5 with a factor 1, 2 or 4 of its power of
+// two, the rest of that in passes of up to 16: the fewest passes, then the
+// smallest largest radix (a pass of radix P keeps N/P of a lane's threads at
+// work, and every pass is a trip through LDS).  False if N has a prime factor
+// above 23.
 bool radix_plan(int N, RadixPlan &rp)
 {
-    rp.n = 0;
     if (N < 1) return false;
-    int n = N, p2 = 1;
+    int n = N, bits = 0, odd[kMaxPasses], m = 0, small = 0;
     while (n % 2 == 0) {
-        p2 *= 2;
+        ++bits;
         n /= 2;
     }
-    for (; p2 >= 16; p2 /= 16) rp.radix[rp.n++] = 16;
-    if (p2 > 1) rp.radix[rp.n++] = p2;
     for (int p : {3, 5, 7, 11, 13, 17, 19, 23})
         for (; n % p == 0; n /= p) {
-            if (rp.n == kMaxPasses) return false;
-            rp.radix[rp.n++] = p;
+            if (m == kMaxPasses) return false;
+            odd[m++] = p;
+            if (p <= 5) ++small;
         }
-    return n == 1;
+    if (n != 1) return false;
+    int best = 1 << 30;
+    rp.n = 0;
+    const int nc = 1 << (2 * std::min(small, 4));  // two bits of choice for each of the first four 3s and 5s
+    for (int c = 0; c < nc; ++c) {
+        RadixPlan t;
+        int left = bits, widest = 1;
+        t.n = 0;
+        for (int i = 0; i < m; ++i) {
+            const int take = i < 4 && odd[i] <= 5 ? (c >> (2 * i)) & 3 : 0;
+            left -= take == 3 ? 99 : take;
+            t.radix[t.n++] = odd[i] << (take & 3);
+        }
+        if (left < 0) continue;
+        const int passes = (left + 3) / 4;
+        if (t.n + passes > kMaxPasses) continue;
+        for (int i = 0; i < passes; ++i) {
+            const int take = (left + passes - i - 1) / (passes - i);
+            t.radix[t.n++] = 1 << take;
+            left -= take;
+        }
+        for (int i = 0; i < t.n; ++i) widest = std::max(widest, t.radix[i]);
+        if (t.n * 64 + widest < best) {
+            best = t.n * 64 + widest;
+            rp = t;
+        }
+    }
+    return best < 1 << 30;
 }
 
 struct FftArgs {
@@ -547,6 +577,71 @@ __device__ __forceinline__ void dft_odd_store(double2 (&v)[P], const double2 *tw
     }
 }
 
+// v[q] <- sum_r v[r] exp(SIGN 2 pi i r q / P), P = 3 or 5
+template <int P, int SIGN>
+__device__ __forceinline__ void dft_small(double2 (&v)[P])
+{
+    constexpr int H = P / 2;
+    constexpr double C3[1] = {-0.5}, S3[1] = {0.86602540378443864676};
+    constexpr double C5[2] = {0.30901699437494742410, -0.80901699437494742410};
+    constexpr double S5[2] = {0.95105651629515357212, 0.58778525229247312917};
+    double2 y[P];
+    y[0] = v[0];
+#pragma unroll
+    for (int r = 1; r <= H; ++r) {
+        const double2 a = v[r], b = v[P - r];
+        v[r] = cadd(a, b);
+        v[P - r] = csub(a, b);
+        y[0] = cadd(y[0], v[r]);
+    }
+#pragma unroll
+    for (int q = 1; q <= H; ++q) {
+        double cx = v[0].x, cy = v[0].y, sx = 0.0, sy = 0.0;
+#pragma unroll
+        for (int r = 1; r <= H; ++r) {
+            const int t = (r * q) % P, e = t <= H ? t : P - t;  // the angle 2 pi t / P
+            const double c = P == 3 ? C3[e - 1] : C5[e - 1];
+            const double n = (t <= H ? 1.0 : -1.0) * (P == 3 ? S3[e - 1] : S5[e - 1]) * SIGN;
+            cx += v[r].x * c;
+            cy += v[r].y * c;
+            sx += v[P - r].x * n;
+            sy += v[P - r].y * n;
+        }
+        y[q] = make_double2(cx - sy, cy + sx);
+        y[P - q] = make_double2(cx + sy, cy - sx);
+    }
+#pragma unroll
+    for (int q = 0; q < P; ++q) v[q] = y[q];
+}
+
+// v[q] <- sum_r v[r] exp(SIGN 2 pi i r q / P), P = A B with A = 2 or 4 and B = 3 or 5:
+// A-point transforms, twiddles, B-point transforms; tw holds exp(2 pi i e/L)
+template <int A, int B, int SIGN>
+__device__ __forceinline__ void dft_product(double2 (&v)[A * B], const double2 *tw, const double2 *tw64, int L)
+{
+    const int st = L / (A * B);
+    double2 x[A][B];
+#pragma unroll
+    for (int n = 0; n < B; ++n) {
+        double2 u[A];
+#pragma unroll
+        for (int r = 0; r < A; ++r) u[r] = v[B * r + n];
+        dft_reg<A, SIGN>(u, tw64);
+#pragma unroll
+        for (int k = 0; k < A; ++k) {
+            double2 w = tw[n * k * st];
+            if (SIGN < 0) w.y = -w.y;
+            x[k][n] = n * k == 0 ? u[k] : cmul(u[k], w);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < A; ++k) {
+        dft_small<B, SIGN>(x[k]);
+#pragma unroll
+        for (int q = 0; q < B; ++q) v[k + A * q] = x[k][q];
+    }
+}
+
 // one Stockham pass of radix P from src to dst (threads sub = 0..NS-1 of
 // each lane share the N/P butterflies)
 template <int P, int SIGN>
@@ -570,8 +665,12 @@ __device__ __forceinline__ void stockham_pass(const double2 *src, double2 *dst, 
             }
         }
         const int d = (b - kk) * P + kk;
-        if constexpr ((P & (P - 1)) == 0) {
-            dft_reg<P, SIGN>(v, tw64);
+        if constexpr ((P & (P - 1)) == 0 || P == 6 || P == 10 || P == 12 || P == 20) {
+            if constexpr (P == 6) dft_product<2, 3, SIGN>(v, tw, tw64, L);
+            else if constexpr (P == 10) dft_product<2, 5, SIGN>(v, tw, tw64, L);
+            else if constexpr (P == 12) dft_product<4, 3, SIGN>(v, tw, tw64, L);
+            else if constexpr (P == 20) dft_product<4, 5, SIGN>(v, tw, tw64, L);
+            else dft_reg<P, SIGN>(v, tw64);
 #pragma unroll
             for (int r = 0; r < P; ++r) dst[(d + r * Ns) * NL + lane] = v[r];
         } else {
@@ -593,13 +692,17 @@ __device__ __forceinline__ double2 *stockham(const RadixPlan &rp, double2 *src, 
         case 2: stockham_pass<2, SIGN>(src, dst, N, Ns, NL, NS, lane, sub, tw, tw64, L); break;
         case 3: stockham_pass<3, SIGN>(src, dst, N, Ns, NL, NS, lane, sub, tw, tw64, L); break;
         case 4: stockham_pass<4, SIGN>(src, dst, N, Ns, NL, NS, lane, sub, tw, tw64, L); break;
+        case 6: stockham_pass<6, SIGN>(src, dst, N, Ns, NL, NS, lane, sub, tw, tw64, L); break;
         case 5: stockham_pass<5, SIGN>(src, dst, N, Ns, NL, NS, lane, sub, tw, tw64, L); break;
         case 7: stockham_pass<7, SIGN>(src, dst, N, Ns, NL, NS, lane, sub, tw, tw64, L); break;
+        case 10: stockham_pass<10, SIGN>(src, dst, N, Ns, NL, NS, lane, sub, tw, tw64, L); break;
         case 8: stockham_pass<8, SIGN>(src, dst, N, Ns, NL, NS, lane, sub, tw, tw64, L); break;
+        case 12: stockham_pass<12, SIGN>(src, dst, N, Ns, NL, NS, lane, sub, tw, tw64, L); break;
         case 11: stockham_pass<11, SIGN>(src, dst, N, Ns, NL, NS, lane, sub, tw, tw64, L); break;
         case 13: stockham_pass<13, SIGN>(src, dst, N, Ns, NL, NS, lane, sub, tw, tw64, L); break;
         case 16: stockham_pass<16, SIGN>(src, dst, N, Ns, NL, NS, lane, sub, tw, tw64, L); break;
         case 17: stockham_pass<17, SIGN>(src, dst, N, Ns, NL, NS, lane, sub, tw, tw64, L); break;
+        case 20: stockham_pass<20, SIGN>(src, dst, N, Ns, NL, NS, lane, sub, tw, tw64, L); break;
         case 19: stockham_pass<19, SIGN>(src, dst, N, Ns, NL, NS, lane, sub, tw, tw64, L); break;
         default: stockham_pass<23, SIGN>(src, dst, N, Ns, NL, NS, lane, sub, tw, tw64, L); break;
         }
@@ -618,7 +721,8 @@ __device__ __forceinline__ double2 *stockham(const RadixPlan &rp, double2 *src, 
 // chain load, passes, store of a block, so a thread's (at most 8) loads are all
 // in flight at once and the index arithmetic has no division: 1000x32x96 (N = 48)
 // forward 24.3 -> 20.2 us, inverse 24.5 -> 19.9, 200x64x192 forward 23 -> 20,
-// inverse 26 -> 20 (a power of two's kernel would take 17).  In place, with
+// inverse 26 -> 20; with passes of 6, 10, 12 and 20 (200x64x192: 12 and 8 instead
+// of 2, 16 and 3) 15.1 -> 13.5, 18.8 -> 17.4 and 19.4 -> 18.1.  In place, with
 // one buffer and every butterfly in registers, 266 registers leave one
 // wavefront per SIMD: 36 and 30 us.
 template <int NL, int NS, int NMAX>
