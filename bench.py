@@ -135,7 +135,7 @@ def stage_work(g, path, steps):
 # stage -> name prefixes of the kernels its timed launches run
 STAGE_KERNELS = {"fft_fwd": ("k_fft_forward<",), "fft_inv": ("k_fft_inverse<",),
                  "zfwd": ("k_zgemm_reg<true,",), "zinv": ("k_zgemm_reg<false,",),
-                 "rsolve": ("k_rsolve<",), "cr": ("k_cr_leaf<", "k_cr_node<"), "resid": ("k_spec_residual",),
+                 "rsolve": ("k_rsolve<",), "cr": ("k_cr_leaf<", "k_cr_node<", "k_cr_top<"), "resid": ("k_spec_residual",),
                  "planes": ("k_refine_plane<",),
                  "bdygen": ("k_bdy_",), "ghost": ("k_zaxphi<",)}
 

@@ -417,7 +417,7 @@ static int rhs_spectrum_f(chy_grid *g, const Fields &F, hipStream_t s, int maxtr
 // the mode systems in one pass: it moves a third of the bytes of two
 // binary32 solves and the residual between them, and binary32 r solves run no
 // faster than binary64 ones on this VALU (mode work of 32 fields at
-// 256x128x256: 3.3 against 4.8 ms; of one, 200 against 230 us).  Otherwise by
+// 256x128x256: 2.4 against 4.8 ms; of one, 126 against 230 us).  Otherwise by
 // iterative refinement of the mode systems in the azimuthal
 // spectrum, where the 7-point operator is block diagonal by mode:
 //   B = the right-hand side spectrum (binary64, as the plain solve forms it);

@@ -18,9 +18,9 @@
 //   down  X(i)       = sum_p (T - r_p)^-1 (a_p Y(i) + cL_p X(i-h) + cR_p X(i+h))
 // and no intermediate vectors, chains or extra launches remain.  A node's sums
 // run over 15 to 35 roots that give the same functions of T as the block's
-// 31 to 511 (crplan.cpp): 511 r solves per mode in 7 launches at KMAX = 128 (867
-// with every root of the nodes' blocks, 5.66 ms per 32 fields at 256x128x256
-// against 5.06; level by level it is 2215 in 19, 13.7 ms).  The weights
+// 31 to 511 (crplan.cpp): 505 r solves per mode in 7 launches at KMAX = 128 (867
+// with every root of the nodes' blocks, a solve of 32 fields at 256x128x256
+// 5.66 ms against 5.06; level by level it is 2215 in 19, 13.6 ms).  The weights
 // alternate in sign; the terms stay as small as the block's own Green's
 // function, so the sums round as one more elimination order does (1-2e-14 from
 // BLKTRI's result at KMAX up to 512 on grids alike in r and z, 3-5e-14 with the
@@ -29,9 +29,9 @@
 // One block of a launch is one tree node (or leaf) of one order m: the cosine
 // and sine parts share T_m, so every solve has two right-hand sides; solves
 // run on groups of G lanes (rtri.h), 64/G roots per wavefront at a time.  The
-// leaves' changes of basis run on the FP64 matrix cores through LDS.  The spectrum spec[q][k][j] (J contiguous) is the mode
-// right-hand side on entry (with POT3's boundary terms applied) and the mode
-// solution on exit.  What the blocks add to a separating row goes to the grid's
+// leaves' changes of basis run on the FP64 matrix cores through LDS.  The
+// spectrum spec[q][k][j] (J contiguous) is the mode right-hand side on entry
+// (with POT3's boundary terms applied) and the mode solution on exit.  What the blocks add to a separating row goes to the grid's
 // second workspace buffer (yh), from its right side into its own row there and
 // from its left side into the row before (unused inside a leaf), so every row
 // has one writer per launch and the order of every sum is fixed.
@@ -115,12 +115,11 @@ __device__ __forceinline__ void team_sums(const double (&s)[NSUM][2][R], double 
 // the result D[l/16 + 4v][l%16].
 //
 // A block takes `run` leaves (one or two) of one order one after the other.  It
-// is bound by HBM (up: the spectrum read once, down: read and written: 0.63 and
-// 0.99 ms per 32 fields at 256x128x256, 0.44 and 0.87 at the rate of a copy),
+// is bound by HBM (up: the spectrum read once, down: read and written: 0.60 and
+// 0.95 ms per 32 fields at 256x128x256, 0.44 and 0.87 at the rate of a copy),
 // while its solves keep the VALU busy for about half as long, so the next
-// leaf's rows are
-// loaded into registers (a matrix operand each) before the current one is
-// solved.  Loads and stores of a wavefront complete in order: nothing the
+// leaf's rows are loaded into registers (a matrix operand each) before the
+// current one is solved.  Loads and stores of a wavefront complete in order: nothing the
 // solves need is loaded after those rows (the roots and weights wait in LDS),
 // and the next leaf's U is loaded before the current one's results are
 // stored.  LDS holds the 16 x 2 vectors: 76 KB at JMAX <= 256 (two blocks of 4
