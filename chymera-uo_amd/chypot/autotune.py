@@ -9,8 +9,9 @@ the fastest:
                     largest batch size asked for;
   * refine_fused    the largest number of fields per launch for which the
                     refined solve runs all mode work of a plane in one kernel
-                    (the binary32 plane in LDS) instead of one kernel per
-                    stage: both forms are timed at every batch size asked
+                    (the binary32 plane in LDS) instead of its default route
+                    (the binary64 tree, or one kernel per stage on grids
+                    without it; "per_stage" in the table): both forms are timed at every batch size asked
                     for, and the threshold is the largest size up to which
                     the one-kernel form was the faster at every size.
 
@@ -98,7 +99,7 @@ def tune_grid(ctx: Context, g, batch_sizes=(1, 32), refine_steps: int = 2, reps:
             entry["cr_lanes"] = min(lane_ms, key=lane_ms.get)
             for pg in grids:
                 pg.cr_lanes = entry["cr_lanes"]
-        # one kernel per plane or one per stage, per batch size (refined solve)
+        # one kernel per plane or the default route, per batch size (refined solve)
         if g.kmax <= 128 and refine_steps in (1, 2):
             tf, ts = {}, {}
             for b in sorted(batch_sizes):
