@@ -517,20 +517,75 @@ __device__ __forceinline__ void store_rows(TS *p, const AT (&d)[R])
     }
 }
 
+// Rows of R >= 8 values per lane through LDS.  Read straight from memory, a
+// load of 16 bytes per lane at a stride of 8 R bytes touches a cache line per
+// lane (64 for one instruction, each line visited R/2 times), and 40 of them,
+// with 16 stores, kept the address unit busy for a third of a solve; here a
+// wavefront reads whole lines and the lanes take their rows from LDS, at a pitch
+// of R + 2 values (conflict-free 16-byte reads): 1000x32x96 (R = 16) 22.9 ->
+// 15.6 us, 8 fields 122 -> 89, 400x256x32 (R = 8) 23.6 -> 18.9.  With 4 rows
+// neighbouring lanes share their lines: 256x128x256 31.6 -> 34.5, so not there.
+typedef double d2v __attribute__((ext_vector_type(2)));
+
+template <int R>
+struct Staged {
+    static constexpr bool ON = R >= 8;
+    static constexpr int PITCH = R + 2, SIZE = ON ? 64 * PITCH : 1;  // doubles per wavefront
+};
+
+// the wavefront's R * 64 values at p, 16 bytes per lane and load
+template <int R>
+__device__ __forceinline__ void load_lines(const double *p, int lane, d2v (&v)[R / 2])
+{
+#pragma unroll
+    for (int i = 0; i < R / 2; ++i) v[i] = reinterpret_cast<const d2v *>(p)[64 * i + lane];
+}
+
+// element e of the wavefront's values in the stage: row e % R of lane e / R
+template <int R>
+__device__ __forceinline__ d2v *stage_at(double *stage, int e)
+{
+    return reinterpret_cast<d2v *>(stage + e / R * Staged<R>::PITCH + e % R);
+}
+
+template <int R>
+__device__ __forceinline__ void lines_to_rows(double *stage, int lane, const d2v (&v)[R / 2], double (&d)[R])
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the stage's last readers are done
+#pragma unroll
+    for (int i = 0; i < R / 2; ++i) *stage_at<R>(stage, 128 * i + 2 * lane) = v[i];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int i = 0; i < R / 2; ++i) {
+        const d2v t = *stage_at<R>(stage, lane * R + 2 * i);
+        d[2 * i] = t.x;
+        d[2 * i + 1] = t.y;
+    }
+}
+
+template <int R>
+__device__ __forceinline__ void rows_to_lines(double *stage, int lane, const double (&d)[R], double *p)
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int i = 0; i < R / 2; ++i) *stage_at<R>(stage, lane * R + 2 * i) = d2v{d[2 * i], d[2 * i + 1]};
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int i = 0; i < R / 2; ++i)
+        reinterpret_cast<d2v *>(p)[64 * i + lane] = *stage_at<R>(stage, 128 * i + 2 * lane);
+}
+
 // One wavefront solves (T_m + lambda_p) x = y for two right-hand sides d0, d1
 // (the cosine and sine parts of order m) in arithmetic AT.  Lane i owns rows
-// [iR, iR+R); rows >= M are identity rows.  Inputs and outputs are the
-// lane's R rows in registers.
+// [iR, iR+R); rows >= M are identity rows.  Inputs (the operator's AM, BM_m
+// and CM among them) and outputs are the lane's R rows in registers.
 template <int R, typename AT>
-__device__ __forceinline__ void rsolve_rows(const ModeArgs &a, int m, int p, int lane, const AT (&d0)[R],
-                                            const AT (&d1)[R], AT (&x0)[R], AT (&x1)[R])
+__device__ __forceinline__ void rsolve_rows(const ModeArgs &a, int p, int lane, const AT (&ca)[R], AT (&cb)[R],
+                                            const AT (&cc)[R], const AT (&d0)[R], const AT (&d1)[R], AT (&x0)[R],
+                                            AT (&x1)[R])
 {
     const AT lam = (AT)a.lam[p];
     const int f = lane * R;
-    AT ca[R], cb[R], cc[R];
-    load_rows<R>(a.am + f, ca);
-    load_rows<R>(a.cm + f, cc);
-    load_rows<R>(a.bm + (size_t)m * a.JP + f, cb);
 #pragma unroll
     for (int r = 0; r < R; ++r) cb[r] = f + r < a.M ? cb[r] + lam : (AT)1;  // padding rows: x = 0
 
@@ -623,19 +678,44 @@ __global__ __launch_bounds__(256) void k_rsolve(ModeArgs a, const Fields F, int 
     const bool two = (m >= 1 && m <= a.N - 1);
     TS *y0 = static_cast<TS *>(a.yh) + ((size_t)m * a.PP + p) * a.JP;
     TS *y1 = static_cast<TS *>(a.yh) + ((size_t)(a.N + m) * a.PP + p) * a.JP;
-    const int f = lane * R;
+    const double *bm = a.bm + (size_t)m * a.JP;
     // rows j >= M of yh are zero (written so by the z forward transform)
-    AT d0[R], d1[R], x0[R], x1[R];
-    load_rows<R>(y0 + f, d0);
-    if (two) {
-        load_rows<R>(y1 + f, d1);
-    } else {
+    AT ca[R], cb[R], cc[R], d0[R], d1[R], x0[R], x1[R];
+    if constexpr (Staged<R>::ON && sizeof(TS) == 8 && sizeof(AT) == 8) {
+        __shared__ double lds[4][Staged<R>::SIZE];
+        double *stage = lds[wave];
+        d2v v0[R / 2], v1[R / 2], va[R / 2], vb[R / 2], vc[R / 2];  // every load issued before the first use
+        load_lines<R>(y0, lane, v0);
+        load_lines<R>(two ? y1 : y0, lane, v1);
+        load_lines<R>(a.am, lane, va);
+        load_lines<R>(bm, lane, vb);
+        load_lines<R>(a.cm, lane, vc);
+        lines_to_rows<R>(stage, lane, v0, d0);
+        lines_to_rows<R>(stage, lane, v1, d1);
+        lines_to_rows<R>(stage, lane, va, ca);
+        lines_to_rows<R>(stage, lane, vb, cb);
+        lines_to_rows<R>(stage, lane, vc, cc);
 #pragma unroll
-        for (int r = 0; r < R; ++r) d1[r] = (AT)0;
+        for (int r = 0; r < R; ++r) d1[r] = two ? d1[r] : 0.0;
+        rsolve_rows<R, AT>(a, p, lane, ca, cb, cc, d0, d1, x0, x1);
+        rows_to_lines<R>(stage, lane, x0, y0);
+        if (two) rows_to_lines<R>(stage, lane, x1, y1);
+    } else {
+        const int f = lane * R;
+        load_rows<R>(y0 + f, d0);
+        if (two) {
+            load_rows<R>(y1 + f, d1);
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; ++r) d1[r] = (AT)0;
+        }
+        load_rows<R>(a.am + f, ca);
+        load_rows<R>(a.cm + f, cc);
+        load_rows<R>(bm + f, cb);
+        rsolve_rows<R, AT>(a, p, lane, ca, cb, cc, d0, d1, x0, x1);
+        store_rows<R>(y0 + f, x0);
+        if (two) store_rows<R>(y1 + f, x1);
     }
-    rsolve_rows<R, AT>(a, m, p, lane, d0, d1, x0, x1);
-    store_rows<R>(y0 + f, x0);
-    if (two) store_rows<R>(y1 + f, x1);
 }
 
 // r solves of grids whose systems do not fit a wavefront's registers
