@@ -876,18 +876,42 @@ int dispatch(int N, int ncu, const FftArgs &a, const Fields &F, hipStream_t s)
         if (N <= 256) return launch_mr<8, KIND>(a, F, ncu, rp, s);
         return launch_mr<4, KIND>(a, F, ncu, rp, s);
     }
-    // Fewer lanes per block (a quarter, a half at N = 128, where pieces of 8
-    // lanes per plane cost more than they give) where the usual blocks fill
-    // less than half the CUs: the same arithmetic on each lane.  64x32x64
-    // (16 blocks): forward 13.4 -> 10.9 us, inverse 12.6 -> 11.2; no gain from
-    // 128 blocks on, nor at N = 256.
-    const int usual = N >= 16 && N <= 128 ? 4096 / N : 1;  // lanes per block below
-    if ((long)((a.nlanes + usual - 1) / usual) * F.nf < ncu / 2) {
+    // N = N1*N2 with N1 and N2 near each other: N2 threads per lane, so that a
+    // thread's chain of loads, butterflies and outputs is short (64x32x64
+    // forward 10.5 -> 8.1 us, inverse 11.4 -> 8.4 with 8*4 instead of 16*2;
+    // 64x128x32 12.4 -> 7.7 and 10.3 -> 6.9 with 4*4 instead of 16*1).  For
+    // N = 64 and fields of more than kSplitLanes lanes large batches are bound by
+    // their access pattern, where 16*4 with 64 lanes per block is the better
+    // one (256x128x128, 16 fields: forward 267 us, with 8*8 280; inverse 243 and
+    // 257; both of 256x64x128, 32 fields, 504 and 542).  The split is chosen by the
+    // field alone: it orders the sums, and a batch has the bits of single solves.
+    // The count of lanes per block does not, and goes by the blocks of the whole
+    // launch: a quarter or half of the usual one where those fill less than
+    // half the CUs, half up to two blocks per CU (256x128x64 forward 15.7 ->
+    // 15.0 us, but in a batch of 16 155 -> 179; 128x64x128, N = 64, 13.0 and 12.3 ->
+    // 12.8 and 10.5, its batch of 8 35.6 and 36.5 -> 32.9 and 32.2), the usual above.
+    constexpr int kSplitLanes = 12288;
+    const bool wide = a.nlanes > kSplitLanes;
+    const int usual = N == 16 || N == 32 ? 128 : N == 64 ? 64 : N == 128 ? 32 : 1;  // lanes per block below
+    const long blocks = (long)((a.nlanes + usual - 1) / usual) * F.nf;
+    if (blocks < ncu / 2) {
         switch (N) {
-        case 16: return launch_one<16, 1, 64, KIND>(a, F, ncu, s);
-        case 32: return launch_one<16, 2, 32, KIND>(a, F, ncu, s);
-        case 64: return launch_one<16, 4, 16, KIND>(a, F, ncu, s);
+        case 16: return launch_one<4, 4, 32, KIND>(a, F, ncu, s);
+        case 32: return launch_one<8, 4, 32, KIND>(a, F, ncu, s);
+        case 64:
+            if (!wide) return launch_one<8, 8, 16, KIND>(a, F, ncu, s);
+            break;
         case 128: return launch_one<16, 8, 16, KIND>(a, F, ncu, s);
+        default: break;
+        }
+    }
+    if (blocks < (N == 64 ? 8 : 2) * ncu) {
+        switch (N) {
+        case 16: return launch_one<4, 4, 64, KIND>(a, F, ncu, s);
+        case 32: return launch_one<8, 4, 64, KIND>(a, F, ncu, s);
+        case 64:
+            if (!wide) return launch_one<8, 8, 32, KIND>(a, F, ncu, s);
+            break;
         default: break;
         }
     }
@@ -896,9 +920,9 @@ int dispatch(int N, int ncu, const FftArgs &a, const Fields &F, hipStream_t s)
     case 2: return launch_one<2, 1, 256, KIND>(a, F, ncu, s);
     case 4: return launch_one<4, 1, 256, KIND>(a, F, ncu, s);
     case 8: return launch_one<8, 1, 256, KIND>(a, F, ncu, s);
-    case 16: return launch_one<16, 1, 256, KIND>(a, F, ncu, s);
-    case 32: return launch_one<16, 2, 128, KIND>(a, F, ncu, s);
-    case 64: return launch_one<16, 4, 64, KIND>(a, F, ncu, s);
+    case 16: return launch_one<4, 4, 128, KIND>(a, F, ncu, s);
+    case 32: return launch_one<8, 4, 128, KIND>(a, F, ncu, s);
+    case 64: return wide ? launch_one<16, 4, 64, KIND>(a, F, ncu, s) : launch_one<8, 8, 64, KIND>(a, F, ncu, s);
     case 128: return launch_one<16, 8, 32, KIND>(a, F, ncu, s);
     case 256: return launch_one<16, 16, 16, KIND>(a, F, ncu, s);
     case 512: return launch_one<32, 16, 8, KIND>(a, F, ncu, s);

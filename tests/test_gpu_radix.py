@@ -37,3 +37,38 @@ def test_azimuths(l):
     got = chypot.to_host(phi_d)
     pg.close()
     assert rel_max(got[1:g.jmax, 1:g.kmax], want[1:g.jmax, 1:g.kmax]) < 1e-12
+
+
+@pytest.mark.parametrize("jkl", [(18, 8, 32), (18, 8, 64), (18, 8, 128), (66, 32, 32), (130, 64, 64), (95, 128, 128),
+                                 (97, 128, 128)])
+def test_powers_of_two(jkl):
+    """LMAX 32, 64 and 128: the splits of LMAX/2, on both sides of the number of
+    lanes that decides it at 128, and each count of lanes per block: one field,
+    and a batch whose blocks fill the chip, bit for bit alike."""
+    import pyoracle as po
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    g = fields.unit_grid(*jkl)
+    print(f"[gpu] powers of two {g.name}", flush=True)
+    rho = fields.density_spiral_torus(g, seed=7)
+    po.use_cyclic_reduction(True)
+    try:
+        want = po.solve(g, rho)["phi"]
+    finally:
+        po.use_cyclic_reduction(False)
+    ctx = chypot.Context(0)
+    jobs = []
+    for i in range(24):
+        rho_d = chypot.to_device(rho if i in (0, 23) else fields.density_spiral_torus(g, seed=8))
+        jobs.append(dict(grid=chypot.PreparedGrid(ctx, g), rho=rho_d, phi=torch.zeros_like(rho_d)))
+    jobs[0]["grid"].solve(jobs[0]["rho"], jobs[0]["phi"])
+    ctx.sync()
+    alone = jobs[0]["phi"].clone()
+    ctx.solve_batch(jobs)
+    ctx.sync()
+    got = chypot.to_host(alone)
+    assert rel_max(got[1:g.jmax, 1:g.kmax], want[1:g.jmax, 1:g.kmax]) < 1e-12
+    assert torch.equal(jobs[0]["phi"], alone)
+    assert torch.equal(jobs[23]["phi"], alone)
+    for j in jobs:
+        j["grid"].close()
