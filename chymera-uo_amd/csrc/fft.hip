@@ -871,10 +871,22 @@ int dispatch(int N, int ncu, const FftArgs &a, const Fields &F, hipStream_t s)
     if (N & (N - 1)) {
         RadixPlan rp;
         if (N > 512 || !radix_plan(N, rp)) return (int)hipErrorInvalidValue;
-        if (N <= 64) return launch_mr<32, KIND>(a, F, ncu, rp, s);
-        if (N <= 128) return launch_mr<16, KIND>(a, F, ncu, rp, s);
-        if (N <= 256) return launch_mr<8, KIND>(a, F, ncu, rp, s);
-        return launch_mr<4, KIND>(a, F, ncu, rp, s);
+        // as many lanes per block as the buffers hold; half or a quarter of them,
+        // so twice or four times the threads per lane, where the blocks still
+        // fit one per CU: 64x32x96 (64 blocks of 32 lanes) forward 11.3 -> 9.7
+        // us, inverse 11.5 -> 9.6, 64x32x192 (128 of 16) 11.3 -> 10.6 and 11.8 ->
+        // 10.8; with more blocks the smaller pieces per plane cost more
+        // (128x64x96, 256 of 32: 14.0 and 12.3, halved 14.0 and 12.1, quartered
+        // 17.8 and 15.7; 200x64x192 20.3 and 20.6, halved 24.6 and 24.1), and
+        // so do pieces of 4 lanes (64x32x384 13.9 and 13.5 -> 14.5 and 14.2)
+        int nl = N <= 64 ? 32 : N <= 128 ? 16 : N <= 256 ? 8 : 4;
+        while (nl > 8 && 2 * ((long)((a.nlanes + nl - 1) / nl) * F.nf) <= ncu) nl /= 2;
+        switch (nl) {
+        case 32: return launch_mr<32, KIND>(a, F, ncu, rp, s);
+        case 16: return launch_mr<16, KIND>(a, F, ncu, rp, s);
+        case 8: return launch_mr<8, KIND>(a, F, ncu, rp, s);
+        default: return launch_mr<4, KIND>(a, F, ncu, rp, s);
+        }
     }
     // N = N1*N2 with N1 and N2 near each other: N2 threads per lane, so that a
     // thread's chain of loads, butterflies and outputs is short (64x32x64
