@@ -1069,6 +1069,7 @@ int chy_solve(chy_grid *g, int maxtrm, int isym, double redge, int npoint, const
     if (!rho_d || !phi_d) return CHY_EINVAL;
     int rc = check_pot3_args(g, npoint, coef_mode, coef_d);
     if (rc) return rc;
+    if (!bdygen_args_ok(maxtrm, isym, redge)) return CHY_EINVAL;
     DeviceScope ds(g->ctx->device);
     rc = run_solve(g, g->ctx->stream, maxtrm, isym, redge, npoint, rho_d, phi_d, coef_d, coef_mode,
                    diag ? diag->klocat : 0);
