@@ -358,9 +358,17 @@ static int run_pot3(chy_grid *g, int npoint, const double *rho, double *phi, dou
     return run_pot3_tail(g, s, npoint, phi, klocat_in, true);
 }
 
-// True where refined solves on g may run the binary32 mode solves: the
-// one-kernel-per-plane form is on, or the binary64 tree does not take the grid.
-static bool refine_may_use32(const chy_grid *g) { return g->refine_fused > 0 || !cr_supported(g); }
+// True where a refined solve of `steps` steps without statistics takes the
+// binary64 tree: for one or two steps, which leave more error than the tree
+// does (against 80-bit solutions at JMAX 24..512, KMAX 8..256: two steps
+// 3e-14..4e-11, the tree 8e-15..1e-11 and nowhere more than the two steps).
+// Three steps and more reach the exact solution of the mode systems (2e-15 to
+// 2e-12), which the tree does not: its result, as the plain solve's, carries
+// the errors of BLKTRI's roots.
+static bool refine_by_tree(const chy_grid *g, int steps) { return steps <= 2 && cr_supported(g); }
+
+// True where such a solve may run the binary32 mode solves
+static bool refine_may_use32(const chy_grid *g, int steps) { return g->refine_fused > 0 || !refine_by_tree(g, steps); }
 
 // Buffers of the refined solve's binary32 mode solves, allocated on first use.
 static int ensure_refine(chy_grid *g, bool use32)
@@ -412,14 +420,13 @@ static int rhs_spectrum_f(chy_grid *g, const Fields &F, hipStream_t s, int maxtr
 }
 
 // Refined solve of every field of F (grids[f] owns field f's workspace; g's
-// tables).  Where the binary64 tree takes the grid (cr.hip) and neither the
-// per-step statistics nor the one-kernel form is asked for, the tree solves
-// the mode systems in one pass: it moves a third of the bytes of two
-// binary32 solves and the residual between them, and binary32 r solves run no
-// faster than binary64 ones on this VALU (mode work of 32 fields at
-// 256x128x256: 2.4 against 4.8 ms; of one, 126 against 230 us).  Otherwise by
-// iterative refinement of the mode systems in the azimuthal
-// spectrum, where the 7-point operator is block diagonal by mode:
+// tables).  One or two steps take the binary64 tree (cr.hip, refine_by_tree) if
+// neither the per-step statistics nor the one-kernel form is asked for: it
+// moves a third of the bytes of two binary32 solves and the residual between
+// them, and binary32 r solves run no faster than binary64 ones on this VALU
+// (mode work of 32 fields at 256x128x256: 2.4 against 4.8 ms; of one, 126
+// against 230 us).  Otherwise by iterative refinement of the mode systems in
+// the azimuthal spectrum, where the 7-point operator is block diagonal by mode:
 //   B = the right-hand side spectrum (binary64, as the plain solve forms it);
 //   X = 0; for each step: R = B - A X (binary64, per mode, rounded to
 //   binary32), D = A^-1 R by the binary32 mode solves (binary64 r solves for
@@ -462,7 +469,7 @@ static int run_refined_fields(chy_grid *g, const std::vector<chy_grid *> &grids,
         if (!rc) rc = dev_rc(launch_refine_planes_f(g, Fp, steps, g->refine_m64, s), "refined mode planes launch");
         if (p) p->end(s);
         steps = 0;  // the mode work is done
-    } else if (!with_stats && cr_supported(g)) {
+    } else if (!with_stats && refine_by_tree(g, steps)) {
         if (p) p->begin(CHY_STAGE_CR, s);
         if (!rc) rc = dev_rc(launch_cr_solve_f(g, F, s), "mode solve launch");
         if (p) p->end(s);
@@ -501,7 +508,7 @@ static int run_refined(chy_grid *g, hipStream_t s, int maxtrm, int isym, double 
                        const double *rho, double *phi, double *coef, int coef_mode, int steps, int klocat_in,
                        bool with_stats)
 {
-    int rc = ensure_refine(g, with_stats || refine_may_use32(g));
+    int rc = ensure_refine(g, with_stats || refine_may_use32(g, steps));
     if (rc) return rc;
     const Fields F = one_field(g, rho, phi, coef, klocat_in);
     return run_refined_fields(g, std::vector<chy_grid *>{g}, F, s, maxtrm, isym, redge, npoint, coef_mode, steps,
@@ -874,7 +881,7 @@ static int solve_batch(chy_ctx *ctx, const chy_solve_item *items, int n, int ste
     int rc = ensure_workers(ctx);
     if (rc) return rc;
     bool use32 = false;
-    for (int i = 0; i < n; ++i) use32 = use32 || refine_may_use32(items[i].grid);
+    for (int i = 0; i < n; ++i) use32 = use32 || refine_may_use32(items[i].grid, steps);
     for (int i = 0; i < n && steps > 0 && rc == CHY_OK; ++i) rc = ensure_refine(items[i].grid, use32);
     if (rc) return rc;
     if (any_diag && ctx->diag_cap < n) {

@@ -226,10 +226,10 @@ int chy_pot3_host(chy_grid *g, int npoint, const double *rho_h, double *phi_h, d
  * accuracy: within 1e-10 of chy_solve's for 2 or more steps.  BDYGEN, COEF,
  * both transforms, POT3's ghost cells and ZAXPHI in binary64 as chy_solve
  * computes them; the mode systems in one of two ways:
- *   - JMAX-1 <= 512, rel_corr NULL and no one-kernel form in force
- *     (CHY_TUNE_REFINE_FUSED): by CHY_MODES_CR's binary64 solves, which are
- *     the faster way there and give chy_solve's own results whatever `steps`
- *     is;
+ *   - 1 or 2 steps, JMAX-1 <= 512, rel_corr NULL and no one-kernel form in
+ *     force (CHY_TUNE_REFINE_FUSED): by CHY_MODES_CR's binary64 solves, which
+ *     are the faster way there and nearer to the exact solution of the mode
+ *     systems than two steps are;
  *   - otherwise by iterative refinement in the azimuthal spectrum: `steps`
  *     (1..8) mode solves in binary32 (z transforms on the FP32 matrix cores,
  *     r solves in binary32 except the orders m <= CHY_TUNE_REFINE_M64, which
@@ -237,7 +237,8 @@ int chy_pot3_host(chy_grid *g, int npoint, const double *rho_h, double *phi_h, d
  *     one of the binary64 residual of the mode systems (pot/pot3.f:203-231) at
  *     the binary64 solution so far, rounded to binary32, its solution added
  *     in binary64.  One step puts PHI within ~1e-6 of chy_solve's, two within
- *     ~1e-11 at 256x128x256.
+ *     ~1e-11 at 256x128x256; three and more reach the exact solution of the
+ *     mode systems, as CHY_MODES_EIGEN does (2.4e-12 from CHY_MODES_CR's there).
  * KMAX <= 256 (CHY_EUNSUPPORTED otherwise).  rel_corr (host, may be NULL)
  * receives, per step, the largest correction relative to the largest
  * |solution| after it (1 for the first step).  Waits when diag or rel_corr is

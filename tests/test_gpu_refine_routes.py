@@ -1,0 +1,67 @@
+"""Which mode solves a refined solve takes (csrc/api.cpp refine_by_tree): the
+binary64 tree where its result is no further from the exact solution of the
+mode systems than the refinement's, else the refinement, whose arithmetic does
+not depend on whether the per-step corrections are asked for."""
+import pytest
+
+import chypot
+from chypot import fields
+from helpers import rel_max
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    return chypot.Context(0)
+
+
+def _refined(ctx, pg, rho, steps, report):
+    phi = torch.zeros_like(rho)
+    pg.solve_refined(rho, phi, steps=steps, npoint=4, report=report)
+    ctx.sync()
+    return phi
+
+
+@pytest.mark.parametrize("steps", [3, 4, 8])
+@pytest.mark.parametrize("jkl", [(16, 4, 4), (64, 32, 24), (130, 64, 40), (257, 16, 32), (300, 8, 24), (40, 256, 16)])
+def test_three_steps_and_more_refine(ctx, jkl, steps):
+    """Three steps and more run the refinement, alone and in a batch, bit for bit what they are with
+    the corrections reported."""
+    g = fields.unit_grid(*jkl)
+    print(f"[gpu] refine {g.name} steps {steps}", flush=True)
+    pgs = [chypot.PreparedGrid(ctx, g) for _ in range(2)]
+    rhos = [chypot.to_device(fields.density_spiral_torus(g, seed=30 + i)) for i in range(2)]
+    jobs = [dict(grid=pg, rho=r, phi=torch.zeros_like(r), npoint=4) for pg, r in zip(pgs, rhos)]
+    ctx.solve_batch(jobs, refine_steps=steps)
+    ctx.sync()
+    for pg, rho, job in zip(pgs, rhos, jobs):
+        reported = _refined(ctx, pg, rho, steps, True)
+        assert torch.equal(_refined(ctx, pg, rho, steps, False), reported)
+        assert torch.equal(job["phi"], reported)
+    for pg in pgs:
+        pg.close()
+
+
+def test_three_steps_reach_the_exact_solution(ctx):
+    """The refinement's limit is the exact solution of the mode systems, here the oracle's in 80 bits: an
+    order of magnitude nearer than BLKTRI's roots leave the tree (2.3e-12)."""
+    import pyoracle as po
+    g = fields.unit_grid(64, 128, 24)
+    rho = fields.density_spiral_torus(g, seed=6)
+    po.use_extended(True)
+    try:
+        want = po.solve(g, rho, npoint=4)["phi"]
+    finally:
+        po.use_extended(False)
+    pg = chypot.PreparedGrid(ctx, g)
+    rho_d = chypot.to_device(rho)
+    for steps in (3, 4):
+        err = rel_max(chypot.to_host(_refined(ctx, pg, rho_d, steps, False)), want)
+        print(f"[gpu] refine {g.name}: {steps} steps, {err:.1e} from the exact solution", flush=True)
+        assert err < 2e-13
+    pg.close()
