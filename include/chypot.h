@@ -226,10 +226,10 @@ int chy_pot3_host(chy_grid *g, int npoint, const double *rho_h, double *phi_h, d
  * accuracy: within 1e-10 of chy_solve's for 2 or more steps.  BDYGEN, COEF,
  * both transforms, POT3's ghost cells and ZAXPHI in binary64 as chy_solve
  * computes them; the mode systems in one of two ways:
- *   - 1 or 2 steps, JMAX-1 <= 512, rel_corr NULL and no one-kernel form in
- *     force (CHY_TUNE_REFINE_FUSED): by CHY_MODES_CR's binary64 solves, which
- *     are the faster way there and nearer to the exact solution of the mode
- *     systems than two steps are;
+ *   - 1 or 2 steps on a grid with CHY_MODES_CR, rel_corr NULL and no
+ *     one-kernel form in force (CHY_TUNE_REFINE_FUSED): by that solver's
+ *     binary64 solves, which are the faster way there and nearer to the exact
+ *     solution of the mode systems than two steps are;
  *   - otherwise by iterative refinement in the azimuthal spectrum: `steps`
  *     (1..8) mode solves in binary32 (z transforms on the FP32 matrix cores,
  *     r solves in binary32 except the orders m <= CHY_TUNE_REFINE_M64, which

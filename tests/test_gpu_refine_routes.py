@@ -2,6 +2,7 @@
 binary64 tree where its result is no further from the exact solution of the
 mode systems than the refinement's, else the refinement, whose arithmetic does
 not depend on whether the per-step corrections are asked for."""
+import numpy as np
 import pytest
 
 import chypot
@@ -64,4 +65,47 @@ def test_three_steps_reach_the_exact_solution(ctx):
         err = rel_max(chypot.to_host(_refined(ctx, pg, rho_d, steps, False)), want)
         print(f"[gpu] refine {g.name}: {steps} steps, {err:.1e} from the exact solution", flush=True)
         assert err < 2e-13
+    pg.close()
+
+
+def graded_column(g, growth):
+    """z and zhf of a column of the unit grid's height whose cells grow by a factor per row."""
+    z = np.concatenate([[0.0], np.cumsum(growth ** np.arange(g.kmax + 1))])
+    z = (z - z[1]) / (z[-1] - z[1]) * g.z()[-1]
+    top = z[-1] + 0.5 * (z[-1] - z[-2])
+    return z, np.append(0.5 * (z[:-1] + z[1:]), top)
+
+
+@pytest.mark.parametrize("jkl", [(64, 32, 24), (257, 16, 32), (16, 8, 4)])
+@pytest.mark.parametrize("steps", [1, 2])
+def test_eigenbasis_grids_refine(ctx, jkl, steps):
+    """A grid whose solver is the z eigenbasis refines in it, bit for bit what it does with the
+    corrections reported."""
+    g = fields.unit_grid(*jkl)
+    pg = chypot.PreparedGrid(ctx, g)
+    pg.mode_solver = chypot.MODES_EIGEN
+    rho = chypot.to_device(fields.density_spiral_torus(g, seed=31))
+    print(f"[gpu] refine, eigenbasis {g.name} steps {steps}", flush=True)
+    reported = _refined(ctx, pg, rho, steps, True)
+    assert torch.equal(_refined(ctx, pg, rho, steps, False), reported)
+    job = dict(grid=pg, rho=rho, phi=torch.zeros_like(rho), npoint=4)
+    ctx.solve_batch([job], refine_steps=steps)
+    ctx.sync()
+    assert torch.equal(job["phi"], reported)
+    pg.close()
+
+
+def test_eigenbasis_grids_keep_the_stated_accuracy(ctx):
+    """Two steps stay within 1e-10 of the grid's own chy_solve, also on a graded column, whose BLKTRI
+    roots are 1.3e-9 from the eigenbasis' result."""
+    g = fields.unit_grid(64, 128, 24)
+    z, zhf = graded_column(g, 1.03)
+    pg = chypot.PreparedGrid(ctx, g, z=z, zhf=zhf)
+    pg.mode_solver = chypot.MODES_EIGEN
+    rho = chypot.to_device(fields.density_spiral_torus(g, seed=6))
+    plain = torch.zeros_like(rho)
+    pg.solve(rho, plain, npoint=4)
+    err = float((_refined(ctx, pg, rho, 2, False) - plain).abs().max()) / float(plain.abs().max())
+    print(f"[gpu] refine, eigenbasis, graded {g.name}: {err:.1e} from chy_solve", flush=True)
+    assert err < 1e-10
     pg.close()
