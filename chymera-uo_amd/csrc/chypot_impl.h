@@ -41,11 +41,11 @@ const Term *terms_table(int *count);  // the kMaxTerms terms, l-major, m ascendi
 
 // Cyclic reduction of the per-mode systems (pot/blktri.f:60-260) as a tree
 // over the z rows 1..n, n = 2^k - 1 (cr.hip).  Leaves: `rows` rows between
-// separators at multiples of rows + 1 (16, or half the column where that is
-// less).  Nodes: rows odd * h, h = rows + 1, 2 (rows + 1), .., (n+1)/2, each
-// with the roots of its block of 2h - 1 rows.  Phases in execution order: the leaves' messages, each level's
-// messages from the lowest up, each level's solutions from the top down, the
-// leaves' solutions.
+// separators at multiples of rows + 1 (16, 4 where the z spacing varies, or half
+// the column where that is less).  Nodes: rows odd * h, h = rows + 1,
+// 2 (rows + 1), .., (n+1)/2, each with the roots of its block of 2h - 1 rows.
+// Phases in execution order: the leaves' messages, each level's messages from
+// the lowest up, each level's solutions from the top down, the leaves' solutions.
 enum { CR_LEAF_UP = 0, CR_NODE_UP = 1, CR_NODE_DOWN = 2, CR_LEAF_DOWN = 3 };
 struct CrPhase {
     int kind, h, nnode, rec0, np;  // nodes: their level's h, their number, the level's first record, root records per node
@@ -67,6 +67,7 @@ constexpr int kNodeRec = 8, kNodePad = 8;
 struct CrPlan {
     int kx = 0;
     int rows = 0, nleaf = 0;
+    bool even = false;             // the rows are spaced evenly (to 1%)
     long nsolve = 0;               // r solves per mode
     std::vector<CrPhase> phases;   // in execution order
     std::vector<double> leaf, node;

@@ -5,9 +5,10 @@
 // A mode's unknowns are X(j, i): j = 1..M along r (JMAX-1 rows), i = 1..N
 // along z (KMAX-1 = 2^k - 1 rows).  BLKTRI eliminates the rows level by level,
 // applying products of r-tridiagonal solves (T_m - rt)^-1.  The same
-// elimination is a tree here (crplan.cpp): leaves of 15 z rows, then one node
-// per row i = odd * h, h = 16, 32, .., whose block of 2h - 1 rows has its
-// roots in BLKTRI's table.  Up the tree every block sends what its right-hand
+// elimination is a tree here (crplan.cpp): leaves of 15 z rows (3 where their
+// spacing varies), then one node per row i = odd * h, h = 16, 32, .. (4, 8, ..),
+// whose block of 2h - 1 rows has its roots in BLKTRI's table.  Up the tree every
+// block sends what its right-hand
 // side adds to the two rows beside it; down the tree every block is solved
 // from its own right-hand side and the solved rows beside it.  BLKTRI's
 // product of a block (all its roots below the line, the roots of its halves

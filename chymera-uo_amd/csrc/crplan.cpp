@@ -31,6 +31,14 @@
 // leaves have at most 15 rows (cr.hip), and fewer than half of the column:
 // solved as one leaf, a whole column on a grid much finer in r than in z
 // (512x16) lands 9e-13 away, with one node above the leaves 1.5e-13.
+// That is for evenly spaced rows.  Where the spacing varies, the roots of small
+// blocks miss the exact ones by more and leaves of 15 rows put the result 7e-13
+// (cells growing by 3% a row, KMAX 32 and 128), 1e-12 (10%, 64) and 7e-11 (30%,
+// 32) from BLKTRI's, leaves of 3 rows nowhere more than 5e-14 (64 rows along r;
+// growths of -30% to 60% a row, random heights, KMAX 16..256): so 3 rows
+// there (one solve at 256x128x256, cells growing by 1%: 404 us, with 15 rows
+// 234, level by level 766).  Spacings that vary by up to 1%, from rounding to noise, stay within
+// 5e-13 with 15 rows (KMAX 16..256).
 #include <algorithm>
 #include <array>
 #include <cmath>
@@ -456,7 +464,15 @@ int build_cr_plan(CrPlan &plan, int n, const double *an, const double *bn, const
     // lev[lv][b * (2^(lv+1)-1) + i]: roots of block b of level lv (rows
     // 1 + b 2^lv .. b 2^lv + 2^(lv+1) - 1), negated eigenvalues of the z
     // sub-tridiagonal, by increasing magnitude
-    const int lv0 = std::min(kx - 1, 4);  // the lowest nodes' level: leaves of 2^lv0 - 1 rows
+    // the lowest nodes' level: leaves of 2^lv0 - 1 rows, up to 15 on columns spaced
+    // evenly (to 1%: couplings within 4%), up to 3 on others (see above)
+    double least = cn[0], greatest = cn[0];
+    for (int i = 1; i < n; ++i) {
+        least = std::min({least, an[i], i + 1 < n ? cn[i] : an[i]});
+        greatest = std::max({greatest, an[i], i + 1 < n ? cn[i] : an[i]});
+    }
+    plan.even = greatest <= 1.04 * least;
+    const int lv0 = std::min(kx - 1, plan.even ? 4 : 2);
     const double machep = cr_machep();
     std::vector<std::vector<double>> lev(kx);
     lev[0].resize(n);
