@@ -359,15 +359,19 @@ static int run_pot3(chy_grid *g, int npoint, const double *rho, double *phi, dou
 }
 
 // True where a refined solve of `steps` steps without statistics takes the
-// binary64 tree: for one or two steps, which leave more error than the tree
-// does (against 80-bit solutions at JMAX 24..512, KMAX 8..256: two steps
-// 3e-14..4e-11, the tree 8e-15..1e-11 and nowhere more than the two steps).
-// Three steps and more reach the exact solution of the mode systems (2e-15 to
-// 2e-12), which the tree does not: its result, as the plain solve's, carries
-// the errors of BLKTRI's roots.  And only where the grid's own solver is the
-// tree: the z eigenbasis has the exact roots, and on a column whose spacing
-// grows by 3% a row BLKTRI's are 1.3e-9 away (64x128x24; two steps 1.3e-11).
-static bool refine_by_tree(const chy_grid *g, int steps) { return steps <= 2 && g->mode_solver == CHY_MODES_CR; }
+// binary64 tree: for one or two steps on evenly spaced columns, which leave more
+// error than the tree does (against 80-bit solutions at JMAX 24..512, KMAX
+// 8..256: two steps 3e-14..4e-11, the tree 8e-15..1e-11 and nowhere more than
+// the two steps).  Three steps and more reach the exact solution of the mode
+// systems (2e-15 to 2e-12), which the tree does not: its result, as the plain
+// solve's, carries the errors of BLKTRI's roots.  Where the spacing varies
+// these exceed what two steps leave (64x128x24, cells growing by 1% a row
+// 4.6e-11 and 4.8e-12, by 3% 1.3e-9 and 1.3e-11).  And only where the grid's own
+// solver is the tree: the z eigenbasis has the exact roots.
+static bool refine_by_tree(const chy_grid *g, int steps)
+{
+    return steps <= 2 && g->mode_solver == CHY_MODES_CR && g->cr.even;
+}
 
 // True where such a solve may run the binary32 mode solves
 static bool refine_may_use32(const chy_grid *g, int steps) { return g->refine_fused > 0 || !refine_by_tree(g, steps); }

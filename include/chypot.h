@@ -223,13 +223,17 @@ int chy_pot3_host(chy_grid *g, int npoint, const double *rho_h, double *phi_h, d
 
 /* ---- refined solve (no reference counterpart) ----
  * The same results as chy_solve (PHI, COEF, diagnostics) to a stated
- * accuracy: within 1e-10 of chy_solve's for 2 or more steps.  BDYGEN, COEF,
- * both transforms, POT3's ghost cells and ZAXPHI in binary64 as chy_solve
- * computes them; the mode systems in one of two ways:
- *   - 1 or 2 steps on a grid with CHY_MODES_CR, rel_corr NULL and no
- *     one-kernel form in force (CHY_TUNE_REFINE_FUSED): by that solver's
- *     binary64 solves, which are the faster way there and nearer to the exact
- *     solution of the mode systems than two steps are;
+ * accuracy: for 2 or more steps within 1e-10 of chy_solve's on evenly spaced
+ * columns and of chy_solve's with CHY_MODES_EIGEN on every one.  (Where the z
+ * spacing varies BLKTRI's roots, and so CHY_MODES_CR, may be further than that
+ * from the exact solution of the mode systems: 1.3e-9 at 64x128x24 with cells
+ * growing by 3% a row.)  BDYGEN, COEF, both transforms, POT3's ghost cells and
+ * ZAXPHI in binary64 as chy_solve computes them; the mode systems in one of
+ * two ways:
+ *   - 1 or 2 steps on an evenly spaced column (to 1%) with CHY_MODES_CR,
+ *     rel_corr NULL and no one-kernel form in force (CHY_TUNE_REFINE_FUSED): by
+ *     that solver's binary64 solves, which are the faster way there and no
+ *     further from the exact solution than two steps are;
  *   - otherwise by iterative refinement in the azimuthal spectrum: `steps`
  *     (1..8) mode solves in binary32 (z transforms on the FP32 matrix cores,
  *     r solves in binary32 except the orders m <= CHY_TUNE_REFINE_M64, which

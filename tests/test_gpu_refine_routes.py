@@ -2,12 +2,12 @@
 binary64 tree where its result is no further from the exact solution of the
 mode systems than the refinement's, else the refinement, whose arithmetic does
 not depend on whether the per-step corrections are asked for."""
-import numpy as np
 import pytest
 
 import chypot
 from chypot import fields
 from helpers import rel_max
+from test_gpu_cr_columns import Column, heights
 
 pytestmark = pytest.mark.gpu
 
@@ -68,14 +68,6 @@ def test_three_steps_reach_the_exact_solution(ctx):
     pg.close()
 
 
-def graded_column(g, growth):
-    """z and zhf of a column of the unit grid's height whose cells grow by a factor per row."""
-    z = np.concatenate([[0.0], np.cumsum(growth ** np.arange(g.kmax + 1))])
-    z = (z - z[1]) / (z[-1] - z[1]) * g.z()[-1]
-    top = z[-1] + 0.5 * (z[-1] - z[-2])
-    return z, np.append(0.5 * (z[:-1] + z[1:]), top)
-
-
 @pytest.mark.parametrize("jkl", [(64, 32, 24), (257, 16, 32), (16, 8, 4)])
 @pytest.mark.parametrize("steps", [1, 2])
 def test_eigenbasis_grids_refine(ctx, jkl, steps):
@@ -99,8 +91,7 @@ def test_eigenbasis_grids_keep_the_stated_accuracy(ctx):
     """Two steps stay within 1e-10 of the grid's own chy_solve, also on a graded column, whose BLKTRI
     roots are 1.3e-9 from the eigenbasis' result."""
     g = fields.unit_grid(64, 128, 24)
-    z, zhf = graded_column(g, 1.03)
-    pg = chypot.PreparedGrid(ctx, g, z=z, zhf=zhf)
+    pg = chypot.PreparedGrid(ctx, Column(g, heights("1.03", g.kmax + 1)))
     pg.mode_solver = chypot.MODES_EIGEN
     rho = chypot.to_device(fields.density_spiral_torus(g, seed=6))
     plain = torch.zeros_like(rho)
@@ -109,3 +100,32 @@ def test_eigenbasis_grids_keep_the_stated_accuracy(ctx):
     print(f"[gpu] refine, eigenbasis, graded {g.name}: {err:.1e} from chy_solve", flush=True)
     assert err < 1e-10
     pg.close()
+
+
+@pytest.mark.parametrize("jkl,growth", [((64, 32, 24), 1.3), ((64, 64, 8), 1.06), ((64, 128, 24), 1.03)])
+def test_uneven_columns_refine(ctx, jkl, growth):
+    """Two steps on a column whose spacing varies refine, alone and in a batch, bit for bit what they do
+    with the corrections reported: within 1e-10 of the exact solution (the oracle's in 80 bits), from
+    which BLKTRI's roots are 3e-10 to 1.9e-9 away."""
+    import pyoracle as po
+    g = fields.unit_grid(*jkl)
+    c = Column(g, heights(str(growth), g.kmax + 1))
+    rho = fields.density_spiral_torus(g, seed=6)
+    po.use_extended(True)
+    try:
+        want = po.solve(c, rho, npoint=4)["phi"]
+    finally:
+        po.use_extended(False)
+    pgs = [chypot.PreparedGrid(ctx, c) for _ in range(2)]
+    rho_d = chypot.to_device(rho)
+    phi = _refined(ctx, pgs[0], rho_d, 2, False)
+    assert torch.equal(phi, _refined(ctx, pgs[0], rho_d, 2, True))
+    jobs = [dict(grid=pg, rho=rho_d, phi=torch.zeros_like(rho_d), npoint=4) for pg in pgs]
+    ctx.solve_batch(jobs, refine_steps=2)
+    ctx.sync()
+    assert all(torch.equal(job["phi"], phi) for job in jobs)
+    err = rel_max(chypot.to_host(phi), want)
+    print(f"[gpu] refine, uneven {g.name} {growth}: {err:.1e} from the exact solution", flush=True)
+    assert err < 1e-10
+    for pg in pgs:
+        pg.close()
