@@ -658,11 +658,15 @@ int chy_ctx_workers(chy_ctx *ctx, int n)
 
 // chy_solve_batch (steps = 0) and chy_solve_batch_refined (steps > 0)
 
-// items that may run together, one launch per kernel
-static bool batchable(const chy_solve_item &a, const chy_solve_item &b)
+// items that may run together, one launch per kernel: the group runs with its
+// first item's settings, so those that shape the arithmetic must be alike (of
+// refined solves also the refinement's)
+static bool batchable(const chy_solve_item &a, const chy_solve_item &b, int steps)
 {
     return same_tables(a.grid, b.grid) && bdygen_spectral_ok(a.grid) && a.maxtrm == b.maxtrm && a.isym == b.isym &&
-           a.redge == b.redge && std::min(a.npoint, 10) == std::min(b.npoint, 10) && a.coef_mode == b.coef_mode;
+           a.redge == b.redge && std::min(a.npoint, 10) == std::min(b.npoint, 10) && a.coef_mode == b.coef_mode &&
+           a.grid->cr_lanes == b.grid->cr_lanes &&
+           (steps == 0 || (a.grid->refine_m64 == b.grid->refine_m64 && a.grid->refine_fused == b.grid->refine_fused));
 }
 
 // One group of a batch (items grp of identically described grids, one launch
@@ -700,11 +704,11 @@ static int run_group(chy_ctx *ctx, const chy_solve_item *items, const std::vecto
 
 // True when the batch is one group: every item on a grid object of its own,
 // all of them together in one launch per kernel.
-static bool one_group(const chy_solve_item *items, int n)
+static bool one_group(const chy_solve_item *items, int n, int steps)
 {
     if (n > kMaxBatch) return false;
     for (int i = 1; i < n; ++i) {
-        if (!batchable(items[0], items[i])) return false;
+        if (!batchable(items[0], items[i], steps)) return false;
         for (int j = 0; j < i; ++j)
             if (items[j].grid == items[i].grid) return false;
     }
@@ -746,7 +750,7 @@ static int issue_batch(chy_ctx *ctx, const chy_solve_item *items, int n, int ste
             if (round[i] != r) continue;
             size_t k = first;
             while (k < tasks.size() && !(tasks[k].grp.size() < (size_t)kMaxBatch &&
-                                         batchable(items[tasks[k].grp[0]], items[i])))
+                                         batchable(items[tasks[k].grp[0]], items[i], steps)))
                 ++k;
             if (k == tasks.size()) tasks.push_back(Task{{}, 3e6, 0});  // launches: as long as 3e6 cells
             tasks[k].grp.push_back(i);
@@ -903,7 +907,7 @@ static int solve_batch(chy_ctx *ctx, const chy_solve_item *items, int n, int ste
     // one group: plain launches on the context's own stream.  Several: one graph
     // launch unless stage timing is on, graphs are off or the caller is
     // capturing the context's stream
-    if (one_group(items, n)) {
+    if (one_group(items, n, steps)) {
         std::vector<int> all(n);
         std::iota(all.begin(), all.end(), 0);
         rc = run_group(ctx, items, all, ctx->stream, steps);

@@ -137,8 +137,11 @@ int chy_grid_mode_solver(const chy_grid *g);
  *                        mode work of a mode plane in one kernel with the
  *                        binary32 plane in LDS, where it fits (KMAX <= 129,
  *                        JMAX <= 257) instead of the mode solves that
- *                        chy_solve_refined otherwise uses
- * Results do not depend on the shapes beyond rounding.  Changing a value
+ *                        chy_solve_refined otherwise uses.  Above 0 a refined
+ *                        field's result may depend on how many run with it:
+ *                        the two forms agree to the steps' accuracy (1e-6 for
+ *                        one, 1e-10 for two)
+ * Otherwise results do not depend on the shapes beyond rounding.  Changing a value
  * drops the captured batches that use the grid.  CHY_EINVAL for a value the grid
  * cannot take. */
 enum { CHY_TUNE_CR_LANES = 0, CHY_TUNE_REFINE_M64 = 1, CHY_TUNE_REFINE_FUSED = 2 };
@@ -186,9 +189,9 @@ int chy_ctx_graphs(chy_ctx *ctx, int enable);
  * the call is ordered after earlier work on that stream and later work waits
  * for the whole batch.  Items on one grid object run in order (they share
  * its workspace).  Items on different grid objects prepared from identical
- * descriptions, with the same maxtrm, isym, redge, npoint and coef_mode, run
- * together, up to 32 per launch of each kernel; other items overlap on the
- * worker streams.  Each item's results are bitwise those of chy_solve on the
+ * descriptions, with the same tunables, maxtrm, isym, redge, npoint and
+ * coef_mode, run together, up to 32 per launch of each kernel; other items
+ * overlap on the worker streams.  Each item's results are bitwise those of chy_solve on the
  * same arguments.  If any item has a diag pointer the call waits and fills
  * every such diag.  Every item is checked before anything is launched.
  * A batch whose items all run together goes to the context's stream itself.
@@ -253,7 +256,7 @@ int chy_solve_refined(chy_grid *g, int maxtrm, int isym, double redge, int npoin
 /* chy_solve_batch with every item solved as chy_solve_refined with `steps`
  * correction steps (items grouped and launched together as in
  * chy_solve_batch; each item's results are bitwise those of its own
- * chy_solve_refined). */
+ * chy_solve_refined, unless CHY_TUNE_REFINE_FUSED says otherwise). */
 int chy_solve_batch_refined(chy_ctx *ctx, const chy_solve_item *items, int n, int steps);
 
 /* ---- ZAXPHI alone (pot/pot3.f:311-399) ----
