@@ -890,9 +890,9 @@ static int solve_batch(chy_ctx *ctx, const chy_solve_item *items, int n, int ste
     DeviceScope ds(ctx->device);
     int rc = ensure_workers(ctx);
     if (rc) return rc;
-    bool use32 = false;
-    for (int i = 0; i < n; ++i) use32 = use32 || refine_may_use32(items[i].grid, steps);
-    for (int i = 0; i < n && steps > 0 && rc == CHY_OK; ++i) rc = ensure_refine(items[i].grid, use32);
+    // (the grids of a group are alike in what the route goes by)
+    for (int i = 0; i < n && steps > 0 && rc == CHY_OK; ++i)
+        rc = ensure_refine(items[i].grid, refine_may_use32(items[i].grid, steps));
     if (rc) return rc;
     if (any_diag && ctx->diag_cap < n) {
         drop_graphs(ctx, nullptr);  // they copy into the old staging

@@ -57,3 +57,23 @@ def test_unlike_tunings_keep_their_own(ctx, jkl, steps, tunings, graphs):
     ctx.graphs(True)
     for j in jobs:
         j["grid"].close()
+
+
+@pytest.mark.parametrize("other", [((600, 8, 24), {}), ((64, 32, 64), dict(refine_fused=4)), ((32, 16, 64), dict(mode_solver=chypot.MODES_EIGEN))])
+def test_refined_batches_allocate_for_their_own_route(ctx, other):
+    """Grids whose own refined solves take the binary64 tree get no binary32 buffers for a neighbour
+    in the batch that refines in binary32 (which gets them)."""
+    jobs = _jobs(ctx, (64, 32, 64), [{}, {}]) + _jobs(ctx, other[0], [other[1]])
+    before = [j["grid"].device_bytes for j in jobs]
+    print(f"[gpu] buffers of a mixed refined batch, {other}", flush=True)
+    ctx.solve_batch(jobs, refine_steps=2)
+    ctx.sync()
+    after = [j["grid"].device_bytes for j in jobs]
+    assert after[:2] == before[:2]
+    assert after[2] > before[2]
+    for j in jobs:
+        alone = torch.zeros_like(j["rho"])
+        j["grid"].solve_refined(j["rho"], alone, steps=2)
+        ctx.sync()
+        assert torch.equal(j["phi"], alone)
+        j["grid"].close()
