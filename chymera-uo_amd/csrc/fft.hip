@@ -280,10 +280,11 @@ __device__ __forceinline__ void forward_outputs(const FftArgs &a, const double2 
         }
     }
     if (!want_coef) return;
-    // COEF(J,K,m,1) amplitude, COEF(J,K,m,2) phase (pot3.f:105-132), two
-    // orders at a time without branches (the chain of the square root, the
-    // divisions and the arc tangent takes 0.6 us)
-    const double A0 = 2.0 * xm(0).x, x1 = fabs(A0), two_x1 = 2.0 / x1, deg = 180.0 / a.pi;
+    // COEF(J,K,m,1) amplitude, COEF(J,K,m,2) phase (pot3.f:105-132, its operations
+    // in its order: a factor 2/|A0| overflows for the smallest |A0|), two orders
+    // at a time without branches (the chain of the square root, the divisions
+    // and the arc tangent takes 0.6 us)
+    const double A0 = 2.0 * xm(0).x, x1 = fabs(A0);
     const size_t cstep = plane * (size_t)NS, chalf = plane * (size_t)N;
     constexpr int U = kCoefOrders;
     for (int m0 = sub + part * U * NS; m0 <= N; m0 += parts * U * NS) {
@@ -297,7 +298,7 @@ __device__ __forceinline__ void forward_outputs(const FftArgs &a, const double2 
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            amp[u] = two_x1 * sqrt(A[u] * A[u] + B[u] * B[u]);
+            amp[u] = 2.0 * sqrt(A[u] * A[u] + B[u] * B[u]) / x1;
             const double t = atan(B[u] / A[u]);
             ph[u] = A[u] > 0.0 ? t : A[u] < 0.0 ? t + a.pi : B[u] > 0.0 ? 0.5 * a.pi : B[u] < 0.0 ? -0.5 * a.pi : 4.0 * a.pi;
         }
@@ -307,7 +308,7 @@ __device__ __forceinline__ void forward_outputs(const FftArgs &a, const double2 
             if (m < 1 || m > N) continue;
             double *c = c1 + (size_t)u * cstep;
             if (x1 != 0.0) c[0] = m < N ? amp[u] : fabs(A[u]) / x1;
-            c[chalf] = m < N ? ph[u] * deg : A0;
+            c[chalf] = m < N ? ph[u] * 180.0 / a.pi : A0;
         }
     }
 }
