@@ -61,13 +61,16 @@ __device__ __forceinline__ void block_sum(double &fx, double &fy, double (&red)[
 }
 
 // q^(-3/2) to binary64 accuracy: the hardware's estimate of q^(-1/2) (28
-// bits) and one third-order step r (1 + e/2 + 3/8 e^2), e = 1 - q r^2.
+// bits) and one third-order step r (1 + e/2 + 3/8 e^2), e = 1 - q r^2.  Where q
+// is infinite or zero (distances past 1e154 or below 1e-162, and a softening
+// as small) e is not a number and the estimate, 0 or infinity, is the value.
 __device__ __forceinline__ double inv_sqrt_cubed(double q)
 {
     const double r = __builtin_amdgcn_rsq(q);
     const double e = __builtin_fma(-q * r, r, 1.0);
     const double s = __builtin_fma(r * e, __builtin_fma(e, 0.375, 0.5), r);
-    return s * s * s;
+    const double v = e == e ? s : r;
+    return v * v * v;
 }
 
 // Bound by the read of RHO: about 20 binary64 operations per cell (a square
