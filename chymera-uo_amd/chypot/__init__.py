@@ -207,8 +207,8 @@ class Context:
     def solve_batch(self, jobs, diag=False, refine_steps=0):
         """Solve independent fields in one call.  jobs: iterable of dicts with
         keys grid (PreparedGrid), rho, phi and optionally coef, coef_mode,
-        maxtrm, isym, redge, npoint.  refine_steps > 0: every field by the
-        refined solve with that many correction steps.  Returns a list of Diag
+        maxtrm, isym, redge, npoint.  refine_steps > 0: every field by
+        solve_refined with that many steps.  Returns a list of Diag
         (diag=True, waits) or None (asynchronous on this context's stream)."""
         jobs = list(jobs)
         items = (SolveItem * len(jobs))()
@@ -406,8 +406,11 @@ class PreparedGrid:
 
     def solve_refined(self, rho, phi, steps=2, maxtrm=10, isym=None, redge=0.0, npoint=8, coef=None,
                       coef_mode=COEF_NONE, diag=None, report=False):
-        """BDYGEN + POT3 by refinement with binary32 correction solves.
-        Returns (Diag or None, per-step relative corrections or None)."""
+        """The refined solve: the results of solve() to 1e-10 (two steps or more) by
+        whichever mode solves chy_solve_refined takes for the grid, the steps and
+        report: the plain solve's own binary64 ones, or binary32 solves with
+        binary64 residuals.  Returns (Diag or None, per-step relative corrections or
+        None)."""
         d = diag if isinstance(diag, Diag) else (Diag() if diag else None)
         rel = (C.c_double * steps)() if report else None
         _check(lib().chy_solve_refined(self.handle, maxtrm, self.isym if isym is None else isym, redge, npoint,

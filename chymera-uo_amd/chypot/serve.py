@@ -27,7 +27,8 @@ the server prepares.
 
 Solves are deterministic and independent, so a request's potential does not
 depend on what it was batched with (tests/test_gpu_serve.py checks this bit
-for bit).
+for bit; with a tune_table that turns the refined solve's one-kernel form on,
+which the measured one does not, to that solve's accuracy).
 """
 from __future__ import annotations
 

@@ -294,7 +294,7 @@ static int run_pot3_tail(chy_grid *g, hipStream_t s, int npoint, double *phi, in
 // lanes' spectrum directly (a Fourier series of order <= MAXTRM).  For
 // LMAX/2 <= 10 the boundary values go through PHI and a transform instead.
 static int run_solve(chy_grid *g, hipStream_t s, int maxtrm, int isym, double redge, int npoint,
-                           const double *rho, double *phi, double *coef, int coef_mode, int klocat_in)
+                     const double *rho, double *phi, double *coef, int coef_mode, int klocat_in)
 {
     Profiler *p = g->ctx->prof.on ? &g->ctx->prof : nullptr;
     const bool spectral = bdygen_spectral_ok(g);

@@ -8,9 +8,9 @@
 // elimination is a tree here (crplan.cpp): leaves of 15 z rows (3 where their
 // spacing varies), then one node per row i = odd * h, h = 16, 32, .. (4, 8, ..),
 // whose block of 2h - 1 rows has its roots in BLKTRI's table.  Up the tree every
-// block sends what its right-hand
-// side adds to the two rows beside it; down the tree every block is solved
-// from its own right-hand side and the solved rows beside it.  BLKTRI's
+// block sends what its right-hand side adds to the two rows beside it; down the
+// tree every block is solved from its own right-hand side and the solved rows
+// beside it.  BLKTRI's
 // product of a block (all its roots below the line, the roots of its halves
 // above) and the chain that follows it (the roots of one half below the line)
 // cancel root by root, so each message and each solution is one sum of
@@ -21,7 +21,7 @@
 // run over 15 to 35 roots that give the same functions of T as the block's
 // 31 to 511 (crplan.cpp): 505 r solves per mode in 7 launches at KMAX = 128 (867
 // with every root of the nodes' blocks, a solve of 32 fields at 256x128x256
-// 5.66 ms against 5.06; level by level it is 2215 in 19, 13.6 ms).  The weights
+// 5.66 ms against 4.97; level by level it is 2215 in 19, 13.6 ms).  The weights
 // alternate in sign; the terms stay as small as the block's own Green's
 // function, so the sums round as one more elimination order does (1-2e-14 from
 // BLKTRI's result at KMAX up to 512 on grids alike in r and z, 3-5e-14 with the
@@ -32,10 +32,11 @@
 // run on groups of G lanes (rtri.h), 64/G roots per wavefront at a time.  The
 // leaves' changes of basis run on the FP64 matrix cores through LDS.  The
 // spectrum spec[q][k][j] (J contiguous) is the mode right-hand side on entry
-// (with POT3's boundary terms applied) and the mode solution on exit.  What the blocks add to a separating row goes to the grid's
-// second workspace buffer (yh), from its right side into its own row there and
-// from its left side into the row before (unused inside a leaf), so every row
-// has one writer per launch and the order of every sum is fixed.
+// (with POT3's boundary terms applied) and the mode solution on exit.  What the
+// blocks add to a separating row goes to the grid's second workspace buffer
+// (yh), from its right side into its own row there and from its left side into
+// the row before (unused inside a leaf), so every row has one writer per launch
+// and the order of every sum is fixed.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

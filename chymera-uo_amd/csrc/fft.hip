@@ -902,7 +902,10 @@ int dispatch(int N, int ncu, const FftArgs &a, const Fields &F, hipStream_t s)
     // launch: a quarter or half of the usual one where those fill less than
     // half the CUs, half up to two blocks per CU (256x128x64 forward 15.7 ->
     // 15.0 us, but in a batch of 16 155 -> 179; 128x64x128, N = 64, 13.0 and 12.3 ->
-    // 12.8 and 10.5, its batch of 8 35.6 and 36.5 -> 32.9 and 32.2), the usual above.
+    // 12.8 and 10.5), for N = 64 up to eight (128x64x128 in batches of 6, 8, 12 and
+    // 16, so 3 to 8 blocks per CU: forward 28.7, 34.0, 56.2, 72.2 -> 25.4, 32.7,
+    // 53.6, 70.0 us, inverse 26.4, 31.5, 44.8, 58.4 -> 25.8, 31.0, 43.3, 58.8), the
+    // usual above.
     constexpr int kSplitLanes = 12288;
     const bool wide = a.nlanes > kSplitLanes;
     const int usual = N == 16 || N == 32 ? 128 : N == 64 ? 64 : N == 128 ? 32 : 1;  // lanes per block below

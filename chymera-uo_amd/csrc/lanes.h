@@ -81,8 +81,9 @@ __device__ __forceinline__ double row_swap(double x)
     });
 }
 
-// x of lane i ^ S, S = 16 or 32: the halves of the pair of rows (or of the
-// wavefront) change places
+// v of both halves of a pair of rows (S = 16) or of the wavefront (S = 32) on
+// both: even is the first half's value, odd the second's, of the lane at the
+// same place in its half
 template <int S>
 __device__ __forceinline__ void half_pair(int v, int &even, int &odd)
 {

@@ -111,13 +111,14 @@ size_t chy_grid_device_bytes(const chy_grid *g);
  *                   (COMPB/TQLRAT, pot/blktri.f:264-423, the same arithmetic),
  *                   its products as sums of independent solves: the
  *                   reference's results to rounding (2.2e-13 relative at
- *                   256x128x256).
+ *                   256x128x256), and the faster one (32 fields there 4.85
+ *                   ms, 5.97 by CHY_MODES_EIGEN).
  *   CHY_MODES_EIGEN the m-independent z operator diagonalised once per grid
  *                   (80-bit arithmetic) and r-tridiagonal solves per z
  *                   eigenvalue, the transforms on FP64 matrix cores: closer to
  *                   the exact solution of the discrete system than BLKTRI
  *                   (whose root tables put it up to a few 1e-12 from it at
- *                   256x128x256), and faster.
+ *                   256x128x256, and further where the z spacing varies).
  * CHY_MODES_CR needs JMAX-1 <= 512 (CHY_EUNSUPPORTED otherwise; such grids
  * start with CHY_MODES_EIGEN).  Changing the solver drops the captured batches
  * that use the grid. */
